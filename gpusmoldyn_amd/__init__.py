@@ -302,8 +302,9 @@ class Engine:
 
     def set_knob(self, knob, value):
         """Launch shape (KNOB_PRODUCER_BLOCK, KNOB_PAIR_BLOCK) or sort layout
-        (KNOB_SEGMENTED_SORT: 1 sorts each replica on its local cells, 0 all
-        keys at once); results are identical for every setting."""
+        (KNOB_SEGMENTED_SORT: 1 counts keys per cell, or sorts each replica on
+        its local cells, 0 sorts all keys at once by digits); results are
+        identical for every setting."""
         _check(lib().smd_engine_set_knob(self._h, int(knob), int(value)), "smd_engine_set_knob")
 
     def get_knob(self, knob):
@@ -352,8 +353,8 @@ class Engine:
         return lib().smd_engine_radix_bits(self._h)
 
     def sort_plan(self):
-        """(digit passes of the step's key sort, True when it sorts each
-        replica on its local cells)."""
+        """(digit passes of the digit form of the step's key sort, True when it
+        sorts each replica on its local cells)."""
         p, g = ctypes.c_int(0), ctypes.c_int(0)
         _check(lib().smd_engine_sort_plan(self._h, ctypes.byref(p), ctypes.byref(g)), "smd_engine_sort_plan")
         return p.value, bool(g.value)

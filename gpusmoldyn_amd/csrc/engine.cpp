@@ -108,6 +108,8 @@ Engine::~Engine() {
   dfree(dMtPar);
   dfree(dGauss);
   dfree(dFirst);
+  dfree(dCellGroups);
+  dfree(dCellSlices);
   dfree(dRetire);
   dfree(dInjCount);
   dfree(dInjBase);
@@ -187,9 +189,9 @@ smd_status Engine::alloc_particle_buffers(uint32_t c) {
   HIPCHK(dalloc(&dBirthType, cap));
   HIPCHK(dalloc(&dSortedPT, cap));
   HIPCHK(dalloc(&dCand, cap));
-  HIPCHK(dalloc(&sb.keys, cap));
+  HIPCHK(dalloc(&sb.keys, (size_t)cap + 4));
   HIPCHK(dalloc(&sb.vals, cap));
-  HIPCHK(dalloc(&sb.keysAlt, cap));
+  HIPCHK(dalloc(&sb.keysAlt, (size_t)cap + 4));
   HIPCHK(dalloc(&sb.valsAlt, cap));
   HIPCHK(dalloc(&sb.counts, sort_counts_words(cap, radixBits)));
   nTilesCap = cap / kCompactTile + 2;
@@ -327,6 +329,10 @@ smd_status Engine::finalize(uint32_t capacity) {
   const uint32_t tot32 = (uint32_t)total;
   HIPCHK(hipMemcpy(dN, &tot32, sizeof(uint32_t), hipMemcpyHostToDevice));
   HIPCHK(dalloc(&dFirst, first_words(nb)));
+  {
+    smd_status st = plan_cell_sort();
+    if (st != SMD_OK) return st;
+  }
 
   // Gaussian table: the producer keeps its half t[1 .. kGaussDim / 2], from
   // which the antisymmetry rebuilds every entry (gauss_entry).
@@ -613,13 +619,133 @@ SegSortArgs Engine::seg_args() const {
   return g;
 }
 
-hipError_t Engine::sort_keys(uint32_t maxN, bool tilesLaid) {
-  if (seg_sorted()) {
-    SegSortArgs g = seg_args();
-    g.tilesLaid = tilesLaid ? 1 : 0;
-    return launch_sort_seg(sb, g, dN, maxN, true, stream);
+// Form and workgroups of the counting cell sort.  By replica, every slice of
+// a replica's cells reads all of the replica's keys; by bins, a digit pass
+// over the keys' high bits comes first and every slice of a bin reads the
+// bin's.  Measured (us per sort, by replica against by bins): 512 replicas of
+// 2k to 64k 130 / 270, 48 of 4k to 131k 32 / 70, one of 16k 8 / 17, one of
+// 100k 35 / 20; so bins take single systems from 48k particles and ensembles
+// with a replica above 131k.  Slot engines keep the digit sort (16 jobs of 1k
+// to 262k: 121 / 71, digits 65): most of their bins are empty, and an empty
+// workgroup still costs its start (4 us per 1000).
+smd_status Engine::plan_cell_sort() {
+  uint64_t most = 1, total = 0;
+  for (uint32_t r = 0; r < R; ++r) {
+    most = std::max<uint64_t>(most, type0[r].size());
+    total += type0[r].size();
   }
-  return launch_sort(sb, dN, maxN, keyBits, radixBits, true, stream);
+  uint32_t bits = 0;
+  while ((1ull << bits) < deadKey) ++bits;
+  // bins of up to 16 slices: more would read their keys over too often
+  cellBinBits = std::max<uint32_t>(11, bits > 8 ? bits - 8 : 0);
+  if (cellBinBits > kCellSliceBits + 4 || slotsMode) cellBinBits = 0;
+  if (slotsMode || most > 131072 || (R == 1 && most > 49152)) return SMD_OK;
+  std::vector<uint32_t> slices(R), order(R);
+  // a few systems get more slices than their lists need, to spread over the
+  // CUs, up to 2M keys read
+  cellMinSlices = R < 256 ? (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(256 / R, (2u << 20) / most)) : 1u;
+  for (uint32_t r = 0; r < R; ++r) {
+    order[r] = r;
+    const uint64_t n = type0[r].size(), c = tabs[r].numBuckets;
+    uint64_t k = std::max<uint64_t>((c + kCellSlice - 1) / kCellSlice, (n + kCellFill - 1) / kCellFill);
+    k = std::max<uint64_t>(k, std::min<uint64_t>(cellMinSlices, (c + 63) / 64));
+    if (k > 1024 || R >= (1u << (32 - kCellGroupShift))) return SMD_OK;
+    slices[r] = (uint32_t)k;
+  }
+  // Workgroups are dealt round robin over the 8 XCDs: a replica's slices go
+  // to one XCD, whose L2 then holds its keys and records (the largest
+  // replicas first); a few replicas are spread.
+  std::sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
+    return type0[a].size() != type0[b].size() ? type0[a].size() > type0[b].size() : a < b;
+  });
+  std::vector<uint32_t> lists[8];
+  for (uint32_t r : order) {
+    int x = 0;
+    for (int q = 1; q < 8; ++q)
+      if (lists[q].size() < lists[x].size()) x = q;
+    for (uint32_t k = 0; k < slices[r]; ++k) lists[R < 8 ? (x + k) % 8 : x].push_back(r << kCellGroupShift | k);
+  }
+  size_t longest = 0;
+  for (const auto& l : lists) longest = std::max(longest, l.size());
+  std::vector<uint32_t> tab(8 * longest, kCellNoGroup);
+  for (int x = 0; x < 8; ++x)
+    for (size_t k = 0; k < lists[x].size(); ++k) tab[8 * k + x] = lists[x][k];
+  HIPCHK(dalloc(&dCellGroups, tab.size()));
+  HIPCHK(dalloc(&dCellSlices, R));
+  HIPCHK(hipMemcpy(dCellGroups, tab.data(), tab.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(dCellSlices, slices.data(), R * sizeof(uint32_t), hipMemcpyHostToDevice));
+  cellGroups = (uint32_t)tab.size();
+  cellGroupsN = R == 1 ? 49152 : 2 * std::max<uint64_t>(total, 4096ull * R);
+  return SMD_OK;
+}
+
+Engine::SortForm Engine::sort_form(uint32_t maxN) const {
+  if (!segSort || sb.algo != 1 || radixBits != 8 || maxN == 0) return SortForm::kDigits;
+  // a system that has grown well past what the slices were laid out for
+  // takes the bins
+  if (cellGroups && (knownN <= cellGroupsN || !cellBinBits)) return SortForm::kCellsByReplica;
+  return cellBinBits ? SortForm::kCellsByBin : SortForm::kDigits;
+}
+
+hipError_t Engine::sort_keys(uint32_t maxN, bool tilesLaid, StageTimer* timer, bool debug) {
+  const SortForm form = sort_form(maxN);
+  hipError_t e;
+  if (form == SortForm::kDigits) {
+    if (seg_sorted()) {
+      SegSortArgs g = seg_args();
+      g.tilesLaid = tilesLaid ? 1 : 0;
+      e = launch_sort_seg(sb, g, dN, maxN, true, stream);
+    } else {
+      e = launch_sort(sb, dN, maxN, keyBits, radixBits, true, stream);
+    }
+    if (timer) (void)hipEventRecord(timer->ev[2], stream);
+    if (e != hipSuccess) return e;
+    return launch_first(sb.keys, dN, maxN, nb, dFirst, dLive, dTables, slotsMode ? slotBits : 0u, R, stream);
+  }
+  CellSortArgs a;
+  a.tables = dTables;
+  a.src = sb.gatherSrc;
+  a.dN = dN;
+  a.maxN = maxN;
+  a.R = (int)R;
+  a.segOff = dRepOff;
+  a.segCount = dRepCount;
+  a.segDead = dRepDeaths;
+  a.bucketOff = dBucketStart;
+  a.groups = dCellGroups;
+  a.groupSlices = dCellSlices;
+  a.minSlices = cellMinSlices;
+  a.binBits = cellBinBits;
+  a.slicesPerBin = 0;
+  a.binTotals = nullptr;
+  a.deadKey = deadKey;
+  a.dLive = dLive;
+  a.first = dFirst;
+  a.dst = sb.gatherDst;
+  a.packIndex = sb.packIndex;
+  a.status = sb.status;
+  uint32_t wg = cellGroups;
+  const bool part = form == SortForm::kCellsByBin;
+  if (part) {
+    e = launch_sort_bins(sb, dN, maxN, (int)cellBinBits, &a.binTotals, stream);
+    if (e != hipSuccess) return e;
+    // twice the slices that the cells need: bins of clustered systems hold
+    // more particles than the average
+    a.slicesPerBin = std::max(2u, 2u * ((1u << cellBinBits) / kCellSlice));
+    wg = ((deadKey + (1u << cellBinBits) - 1u) >> cellBinBits) * a.slicesPerBin;
+  }
+  a.keys = sb.keys;
+  a.vals = sb.vals;
+  a.keysOut = sb.keysAlt;
+  a.valsOut = sb.valsAlt;
+  e = launch_cell_sort(a, part, wg, stream);
+  if (e == hipSuccess && debug)
+    e = launch_cell_sort_removed(sb.keys, part ? sb.vals : nullptr, dN, maxN, deadKey, dLive, sb.keysAlt, sb.valsAlt,
+                                 stream);
+  std::swap(sb.keys, sb.keysAlt);
+  std::swap(sb.vals, sb.valsAlt);
+  if (timer) (void)hipEventRecord(timer->ev[2], stream);
+  return e;
 }
 
 smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
@@ -649,7 +775,7 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
   pa.retire = dRetire;
   // the segmented sort's tile table by one more workgroup of the producer's
   // launch (it reads only the per-replica counts the step starts with)
-  const bool tilesLaid = anyBim && seg_sorted();
+  const bool tilesLaid = anyBim && seg_sorted() && sort_form(maxN) == SortForm::kDigits;
   if (tilesLaid) {
     pa.segTilesOn = 1;
     pa.segTiles = seg_tiles_args(seg_args(), dN, maxN, sb.status);
@@ -676,9 +802,7 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
     // the sort's last pass puts each particle's index into its sorted record
     // when the gather is fused into it and every index fits
     sb.packIndex = (sb.algo == 1 && cap <= kMaxPackedIndex) ? 1 : 0;
-    HIPCHK(sort_keys(maxN, tilesLaid));
-    mark(2);
-    HIPCHK(launch_first(sb.keys, dN, maxN, nb, dFirst, dLive, dTables, slotsMode ? slotBits : 0u, R, stream));
+    HIPCHK(sort_keys(maxN, tilesLaid, timer, false));
     mark(3);
     CandArgs ca;
     ca.tables = dTables;
@@ -1176,8 +1300,7 @@ smd_status Engine::debug_stage(int stage, float* pos4, int* types, uint32_t* key
     sb.gatherDeadKey = deadKey;
     sb.sizeHint = (uint32_t)std::min<uint64_t>(knownN, 0xFFFFFFFFu);
     sb.packIndex = 0;  // the sorted values are returned
-    HIPCHK(sort_keys(maxN));
-    HIPCHK(launch_first(sb.keys, dN, maxN, nb, dFirst, dLive, dTables, slotsMode ? slotBits : 0u, R, stream));
+    HIPCHK(sort_keys(maxN, false, nullptr, true));
   }
   if (stage >= 3) {
     CandArgs ca;

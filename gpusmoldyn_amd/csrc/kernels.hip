@@ -302,7 +302,15 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nTiles) {
   return x * q + min(x, r) + j;
 }
 
-template <int BITS, int ITEMS>
+// Digit of a key.  TOP: the key's remaining high bits, where keys past the
+// last digit (the removed particles' key can be one bit longer than any live
+// one) count as the last digit.
+template <int BITS, bool TOP>
+__device__ __forceinline__ uint32_t sort_digit(uint32_t key, int shift) {
+  return TOP ? min(key >> shift, (1u << BITS) - 1u) : (key >> shift) & ((1u << BITS) - 1u);
+}
+
+template <int BITS, int ITEMS, bool TOP>
 __global__ __launch_bounds__(256) void k_sort_up(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ dN,
                                                  uint32_t* __restrict__ counts, uint32_t stride, int shift) {
   constexpr int RADIX = 1 << BITS;
@@ -327,7 +335,7 @@ __global__ __launch_bounds__(256) void k_sort_up(const uint32_t* __restrict__ ke
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
     const bool valid = base + k * 256 + threadIdx.x < n;
-    const uint32_t d = (kk[k] >> shift) & (RADIX - 1);
+    const uint32_t d = sort_digit<BITS, TOP>(kk[k], shift);
     const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);
     const uint64_t vm = __ballot(valid);
     if (__all(d == d0 || !valid)) {
@@ -432,7 +440,7 @@ __global__ __launch_bounds__(256) void k_sort_rowscan_wave(uint32_t* __restrict_
   if (lane == 0) totals[d] = carry;
 }
 
-template <int BITS, int ITEMS, bool GATHER>
+template <int BITS, int ITEMS, bool GATHER, bool TOP>
 __global__ __launch_bounds__(256) void k_sort_down(const uint32_t* __restrict__ keysIn,
                                                    const uint32_t* __restrict__ valsIn,
                                                    uint32_t* __restrict__ keysOut, uint32_t* __restrict__ valsOut,
@@ -502,7 +510,7 @@ __global__ __launch_bounds__(256) void k_sort_down(const uint32_t* __restrict__ 
     const uint32_t e = base + it * 64 + lane;
     const bool valid = e < n;
     const uint32_t k = kk[it];
-    const uint32_t d = (k >> shift) & (RADIX - 1);
+    const uint32_t d = sort_digit<BITS, TOP>(k, shift);
     const uint64_t mm = wave_digit_peers<BITS>(d, valid);
     // every lane of the digit writes the same new count (a lane past the
     // end counts its valid peers only, which is the same number)
@@ -541,7 +549,7 @@ __global__ __launch_bounds__(256) void k_sort_down(const uint32_t* __restrict__ 
   for (int it = 0; it < ITEMS; ++it) {
     const uint32_t e = base + it * 64 + lane;
     if (e < n) {
-      const uint32_t d = (kk[it] >> shift) & (RADIX - 1);
+      const uint32_t d = sort_digit<BITS, TOP>(kk[it], shift);
       const uint32_t lp = s_tstart[d] + s_wcnt[w][d] + rk[it];
       s_key[lp] = kk[it];
       s_val[lp] = vv[it];
@@ -558,7 +566,7 @@ __global__ __launch_bounds__(256) void k_sort_down(const uint32_t* __restrict__ 
       const uint32_t idx = t + q * 256u;
       const bool ok = idx < tileN;
       const uint32_t k = ok ? s_key[idx] : 0xFFFFFFFFu;
-      const uint32_t d = (k >> shift) & (RADIX - 1);
+      const uint32_t d = sort_digit<BITS, TOP>(k, shift);
       dk[q] = k;
       dv[q] = ok ? s_val[idx] : 0u;
       dd[q] = ok ? s_base[d] + (idx - s_tstart[d]) : 0u;
@@ -583,7 +591,7 @@ __global__ __launch_bounds__(256) void k_sort_down(const uint32_t* __restrict__ 
   }
   for (uint32_t idx = t; idx < tileN; idx += 256) {
     const uint32_t k = s_key[idx];
-    const uint32_t d = (k >> shift) & (RADIX - 1);
+    const uint32_t d = sort_digit<BITS, TOP>(k, shift);
     const uint32_t dst = s_base[d] + (idx - s_tstart[d]);
     keysOut[dst] = k;
     valsOut[dst] = s_val[idx];
@@ -2332,10 +2340,10 @@ hipError_t launch_sort(SortBuffers& b, const uint32_t* dN, uint32_t maxN, uint32
 }
 
 // One digit pass of the count / scan / scatter sort.
-template <int BITS, int ITEMS>
+template <int BITS, int ITEMS, bool TOP = false>
 static hipError_t sort3k_pass(SortBuffers& b, const uint32_t* dN, uint32_t maxTiles, uint32_t stride,
                               uint32_t* totals, int shift, bool idv, bool gather, hipStream_t stream) {
-  hipLaunchKernelGGL((k_sort_up<BITS, ITEMS>), dim3(maxTiles), dim3(256), 0, stream, b.keys, dN, b.counts, stride,
+  hipLaunchKernelGGL((k_sort_up<BITS, ITEMS, TOP>), dim3(maxTiles), dim3(256), 0, stream, b.keys, dN, b.counts, stride,
                      shift);
   // measured: one wave per digit is faster up to ~100 tiles (16k keys: 1.5 us
   // per step), slower at 512 (1M keys: 1 us per digit pass)
@@ -2346,11 +2354,11 @@ static hipError_t sort3k_pass(SortBuffers& b, const uint32_t* dN, uint32_t maxTi
     hipLaunchKernelGGL((k_sort_rowscan<BITS, ITEMS>), dim3(1 << BITS), dim3(256), 0, stream, b.counts, totals, dN,
                        stride);
   if (gather)
-    hipLaunchKernelGGL((k_sort_down<BITS, ITEMS, true>), dim3(maxTiles), dim3(256), 0, stream, b.keys, b.vals,
+    hipLaunchKernelGGL((k_sort_down<BITS, ITEMS, true, TOP>), dim3(maxTiles), dim3(256), 0, stream, b.keys, b.vals,
                        b.keysAlt, b.valsAlt, b.counts, totals, dN, stride, shift, idv ? 1 : 0, b.gatherSrc,
                        b.gatherDst, b.gatherDeadKey, b.packIndex);
   else
-    hipLaunchKernelGGL((k_sort_down<BITS, ITEMS, false>), dim3(maxTiles), dim3(256), 0, stream, b.keys, b.vals,
+    hipLaunchKernelGGL((k_sort_down<BITS, ITEMS, false, TOP>), dim3(maxTiles), dim3(256), 0, stream, b.keys, b.vals,
                        b.keysAlt, b.valsAlt, b.counts, totals, dN, stride, shift, idv ? 1 : 0, nullptr, nullptr, 0u,
                        0);
   return hipGetLastError();
@@ -2402,6 +2410,21 @@ hipError_t launch_sort_3k(SortBuffers& b, const uint32_t* dN, uint32_t maxN, uin
     b.valsAlt = tv;
   }
   return hipGetLastError();
+}
+
+hipError_t launch_sort_bins(SortBuffers& b, const uint32_t* dN, uint32_t maxN, int shift, const uint32_t** totals,
+                            hipStream_t stream) {
+  const int items = sort3k_items(maxN, b.sizeHint);
+  const uint32_t maxTiles = cdiv(maxN, 256u * items);
+  if (maxTiles == 0) return hipErrorInvalidValue;
+  const uint32_t stride = maxTiles + 1;
+  uint32_t* tot = b.counts + 256 * (size_t)stride;
+  *totals = tot;
+  const hipError_t e = items == 8 ? sort3k_pass<8, 8, true>(b, dN, maxTiles, stride, tot, shift, true, false, stream)
+                                  : sort3k_pass<8, 16, true>(b, dN, maxTiles, stride, tot, shift, true, false, stream);
+  std::swap(b.keys, b.keysAlt);
+  std::swap(b.vals, b.valsAlt);
+  return e;
 }
 
 size_t first_words(uint32_t nb) { return (size_t)nb + 1; }

@@ -117,6 +117,14 @@ class Engine {
   int segLow = 0, segHigh = 0;       // digit widths of the segmented sort, 0: not applicable
   uint32_t* dSegScratch = nullptr;   // its tile table and counters
   smd_status set_knob(int knob, int value);
+  // the counting cell sort's workgroups when segments are the replicas:
+  // replica << kCellGroupShift | slice, largest replicas first
+  uint32_t* dCellGroups = nullptr;
+  uint32_t* dCellSlices = nullptr;  // per replica: its slices
+  uint32_t cellGroups = 0;          // 0: not applicable
+  uint32_t cellMinSlices = 1;
+  uint64_t cellGroupsN = 0;         // particles (all replicas) up to which they serve
+  uint32_t cellBinBits = 0;         // cells per bin (log2) when segments are bins of the high key bits
 
   // hipGraph replay of two-step pairs, one executable graph per ping-pong
   // parity (an eager step between pairs flips the parity)
@@ -132,7 +140,15 @@ class Engine {
  private:
   smd_status enqueue_kernels(uint32_t maxN, StageTimer* timer);
   SegSortArgs seg_args() const;
-  hipError_t sort_keys(uint32_t maxN, bool tilesLaid = false);
+  // How the step sorts its keys: digit passes (global or segmented) and the
+  // cell table kernel, or the counting cell sort by replica or by bins of
+  // the high key bits, which writes the cell table itself.
+  enum class SortForm { kDigits, kCellsByReplica, kCellsByBin };
+  SortForm sort_form(uint32_t maxN) const;
+  smd_status plan_cell_sort();
+  // sorted keys, records and cell table of the step (debug: also the values
+  // and the removed particles)
+  hipError_t sort_keys(uint32_t maxN, bool tilesLaid, StageTimer* timer, bool debug);
   smd_status step_graph(int pairs);
   smd_status alloc_particle_buffers(uint32_t c);
   void free_particle_buffers();

@@ -92,6 +92,46 @@ struct SegSortArgs {
 // keys).
 void seg_sort_digits(uint32_t maxGridBits, int& lowBits, int& highBits);
 
+// The counting cell sort (k_cell_sort): slices of at most kCellSlice cells,
+// aiming at kCellFill particles, whose list holds kCellList.
+constexpr int kCellThreads = 512;
+constexpr int kCellSliceBits = 12;
+constexpr uint32_t kCellSlice = 1u << kCellSliceBits;
+constexpr uint32_t kCellList = 5376;
+constexpr uint32_t kCellFill = 4838;
+constexpr int kCellGroupShift = 12;  // workgroup table: replica << kCellGroupShift | slice
+constexpr uint32_t kCellNoGroup = 0xFFFFFFFFu;  // an entry without work
+
+struct CellSortArgs {
+  const ReplicaTables* tables;
+  const uint32_t* keys;        // in canonical order, or binned (then vals holds the indices)
+  const uint32_t* vals;
+  const float4* src;           // canonical records
+  const uint32_t* dN;
+  uint32_t maxN;
+  int R;
+  const uint32_t* segOff;      // per replica: first particle, particles, removed particles
+  const uint32_t* segCount;
+  const uint32_t* segDead;
+  const uint32_t* bucketOff;
+  // by replica: the slice of each workgroup, and the slices each replica has
+  // workgroups for (at least ceil(cells / kCellSlice))
+  const uint32_t* groups;
+  const uint32_t* groupSlices;
+  uint32_t minSlices;          // slices per segment for small systems
+  // by bins of the keys' high bits: 2^binBits cells each
+  uint32_t binBits, slicesPerBin;
+  const uint32_t* binTotals;   // keys per bin
+  uint32_t deadKey;
+  uint32_t* dLive;
+  uint32_t* first;             // first_words(deadKey + 1) words
+  uint32_t* keysOut;
+  uint32_t* valsOut;           // written unless packIndex
+  float4* dst;                 // records in sorted order
+  int packIndex;
+  uint32_t* status;
+};
+
 struct CandArgs {
   const ReplicaTables* tables;
   const uint32_t* bucketStart;  // per replica bucketOff, [R] = deadKey
@@ -205,6 +245,19 @@ int sort_passes(uint32_t keyBits, int radixBits);
 size_t sort_counts_words(uint32_t maxN, int radixBits);
 hipError_t launch_sort(SortBuffers& b, const uint32_t* dN, uint32_t maxN, uint32_t keyBits, int radixBits,
                        bool identityVals, hipStream_t stream);
+// One stable 8-bit digit pass (count / scan / scatter) on the key bits from
+// `shift` (keys past the last digit go into the last bin), values = indices; totals gets the address of the 256 digit counts.
+// Swaps the buffers.
+hipError_t launch_sort_bins(SortBuffers& b, const uint32_t* dN, uint32_t maxN, int shift, const uint32_t** totals,
+                            hipStream_t stream);
+// Sorted keys (live ones), records and cell table in one kernel; part: by
+// bins of launch_sort_bins.
+hipError_t launch_cell_sort(const CellSortArgs& a, bool part, uint32_t workgroups, hipStream_t stream);
+// The removed keys and values behind the live ones, in index order (vals
+// nullptr: keys are in canonical order).
+hipError_t launch_cell_sort_removed(const uint32_t* keys, const uint32_t* vals, const uint32_t* dN, uint32_t maxN,
+                                    uint32_t deadKey, const uint32_t* dLive, uint32_t* keysOut, uint32_t* valsOut,
+                                    hipStream_t stream);
 // Segmented two-pass sort of an ensemble's keys (same output as launch_sort
 // with identityVals over all keys: live keys in order, removed ones after
 // them in index order).

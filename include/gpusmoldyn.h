@@ -188,9 +188,10 @@ smd_status smd_engine_set_graphs(smd_engine* e, int on);
 typedef enum smd_knob {
   SMD_KNOB_PRODUCER_BLOCK = 0,
   SMD_KNOB_PAIR_BLOCK = 1,
-  /* 1 (default): an engine of several replicas sorts each replica's keys on
-   * its local cells (two digit passes where the global keys need three);
-   * 0: one sort over all keys */
+  /* 1 (default): keys are sorted by counting them per cell where that applies
+   * (8-bit digits, not in slot engines), otherwise an engine of several
+   * replicas sorts each replica's keys on its local cells (two digit passes
+   * where the global keys need three); 0: one digit sort over all keys */
   SMD_KNOB_SEGMENTED_SORT = 2
 } smd_knob;
 smd_status smd_engine_set_knob(smd_engine* e, int knob, int value);
@@ -237,9 +238,11 @@ smd_status smd_engine_debug_first(smd_engine* e, uint32_t* first, uint32_t cap, 
 /* Number of buckets (keys deadKey = total buckets) and key bits. */
 smd_status smd_engine_layout(smd_engine* e, uint32_t* total_buckets, uint32_t* key_bits, uint32_t* total_streams,
                              uint32_t* capacity);
-/* How the step sorts its keys: *passes digit passes, *segmented = 1 when each
- * replica is sorted on its local cells (SMD_KNOB_SEGMENTED_SORT applies),
- * 0 for one sort over the global keys.  No counterpart in the reference. */
+/* The plan of the digit form of the step's key sort: *passes digit passes,
+ * *segmented = 1 when each replica is sorted on its local cells
+ * (SMD_KNOB_SEGMENTED_SORT applies), 0 for one sort over the global keys.
+ * Where the step counts keys per cell instead, the order is the same.  No
+ * counterpart in the reference. */
 smd_status smd_engine_sort_plan(const smd_engine* e, int* passes, int* segmented);
 /* Per-kernel timing of the last timed step (HIP events, microseconds):
  * names is a '\n' separated list written into buf. */
