@@ -336,7 +336,7 @@ __global__ __launch_bounds__(T, 8) void k_cell_sort(CellSortArgs a, const Replic
     }
     a.keysOut[dst] = key0 + (ent >> kIndexBits);
     if (a.packIndex) {
-      rec.w = __int_as_float(pack_index_type(idx, __float_as_int(rec.w)));
+      rec.w = __int_as_float(pack_index_type(idx, __float_as_int(rec.w) & kTypeMask));
     } else {
       a.valsOut[dst] = idx;
     }

@@ -39,45 +39,33 @@ static void dfree(T*& p) {
 
 static inline uint32_t round64(uint32_t x) { return (x + 63u) & ~63u; }
 
-// Caller layout (pos4 = x, y, z, w; int types) to and from the canonical
-// device layout (pt = x, y, z, type bits; w apart).
-static void pack_particles(const float* pos4, const int* types, size_t n, std::vector<float4>& pt,
-                           std::vector<float>& w) {
-  pt.resize(n);
-  w.resize(n);
+// Whether every fourth component's bits leave room for a type.
+static bool components_pack(const float* pos4, size_t n) {
   for (size_t i = 0; i < n; ++i) {
-    float tb;
-    std::memcpy(&tb, &types[i], sizeof(float));
-    pt[i] = make_float4(pos4[4 * i], pos4[4 * i + 1], pos4[4 * i + 2], tb);
-    w[i] = pos4[4 * i + 3];
+    uint32_t b;
+    std::memcpy(&b, &pos4[4 * i + 3], sizeof(b));
+    if (b & (uint32_t)kTypeMask) return false;
   }
+  return true;
 }
 
+// Caller layout (pos4 = x, y, z, w; int types) to the canonical device layout
+// (w in the records, or in dw when that is given).
 static hipError_t upload_particles(const float* pos4, const int* types, size_t n, float4* dpt, float* dw) {
-  std::vector<float4> pt;
-  std::vector<float> w;
-  pack_particles(pos4, types, n, pt, w);
-  hipError_t e = hipMemcpy(dpt, pt.data(), n * sizeof(float4), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(dw, w.data(), n * sizeof(float), hipMemcpyHostToDevice);
-  return e;
-}
-
-static hipError_t download_particles(const float4* dpt, const float* dw, size_t n, float* pos4, int* types) {
   std::vector<float4> pt(n);
-  std::vector<float> w(pos4 ? n : 0);
-  hipError_t e = hipMemcpy(pt.data(), dpt, n * sizeof(float4), hipMemcpyDeviceToHost);
-  if (e == hipSuccess && pos4) e = hipMemcpy(w.data(), dw, n * sizeof(float), hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return e;
+  std::vector<float> w(dw ? n : 0);
   for (size_t i = 0; i < n; ++i) {
-    if (pos4) {
-      pos4[4 * i] = pt[i].x;
-      pos4[4 * i + 1] = pt[i].y;
-      pos4[4 * i + 2] = pt[i].z;
-      pos4[4 * i + 3] = w[i];
-    }
-    if (types) std::memcpy(&types[i], &pt[i].w, sizeof(int));
+    uint32_t b = 0;
+    if (dw) w[i] = pos4[4 * i + 3];
+    else std::memcpy(&b, &pos4[4 * i + 3], sizeof(b));
+    b |= (uint32_t)types[i];
+    float wb;
+    std::memcpy(&wb, &b, sizeof(wb));
+    pt[i] = make_float4(pos4[4 * i], pos4[4 * i + 1], pos4[4 * i + 2], wb);
   }
-  return hipSuccess;
+  hipError_t e = hipMemcpy(dpt, pt.data(), n * sizeof(float4), hipMemcpyHostToDevice);
+  if (e == hipSuccess && dw) e = hipMemcpy(dw, w.data(), n * sizeof(float), hipMemcpyHostToDevice);
+  return e;
 }
 
 Engine::Engine(int dev, int rbits) : device(dev), radixBits(rbits == 4 || rbits == 8 || rbits == 11 ? rbits : 0) {}
@@ -97,9 +85,11 @@ Engine::~Engine() {
   dfree(dRepCount);
   dfree(dNewOff);
   dfree(dNewCount);
-  dfree(dAliveBase);
+  dfree(dAlive);
+  dfree(dHoleOff);
+  dfree(dHoleN);
+  dfree(dExtraOff);
   dfree(dBirthBase);
-  dfree(dRepAlive);
   dfree(dRepDeaths);
   dfree(dRepBirths);
   dfree(dCounters);
@@ -125,6 +115,7 @@ Engine::~Engine() {
   dfree(dInjType);
   dfree(dInjRep);
   if (countRing) (void)hipHostFree(countRing);
+  if (hostStatus) (void)hipHostFree(hostStatus);
   dfree(dStepCount);
   if (stream) (void)hipStreamDestroy(stream);
 }
@@ -146,9 +137,11 @@ void Engine::free_particle_buffers() {
   dfree(sb.keysAlt);
   dfree(sb.valsAlt);
   dfree(sb.counts);
-  dfree(dTileAlive);
+  dfree(dDeadBits);
+  dfree(dTileDead[0]);
+  dfree(dTileDead[1]);
+  dfree(dHoles);
   dfree(dTileBirth);
-  dfree(dTileAlivePre);
   dfree(dTileBirthPre);
   dfree(dBlockSum);
   dfree(dSegScratch);
@@ -181,30 +174,74 @@ int Engine::add_replica(const smd_sim_spec& spec, const float* pos4, const int* 
 
 smd_status Engine::alloc_particle_buffers(uint32_t c) {
   cap = c;
-  for (int k = 0; k < 2; ++k) {
-    HIPCHK(dalloc(&dPT[k], cap));
-    HIPCHK(dalloc(&dW[k], cap));
+  extraCap = (anySplit || anyZero || slotsMode) ? cap : 0;
+  for (int k = 0; k < 2; ++k) HIPCHK(dalloc(&dPT[k], (size_t)cap + extraCap));
+  if (wApart) {
+    smd_status st = alloc_apart();
+    if (st != SMD_OK) return st;
   }
   HIPCHK(dalloc(&dAddedPos, cap));
   HIPCHK(dalloc(&dBirthType, cap));
   HIPCHK(dalloc(&dSortedPT, cap));
   HIPCHK(dalloc(&dCand, cap));
+  // the cell sort reads keys as whole vectors of four
   HIPCHK(dalloc(&sb.keys, (size_t)cap + 4));
   HIPCHK(dalloc(&sb.vals, cap));
   HIPCHK(dalloc(&sb.keysAlt, (size_t)cap + 4));
   HIPCHK(dalloc(&sb.valsAlt, cap));
   HIPCHK(dalloc(&sb.counts, sort_counts_words(cap, radixBits)));
   nTilesCap = cap / kCompactTile + 2;
-  HIPCHK(dalloc(&dTileAlive, nTilesCap));
+  const size_t words = (size_t)nTilesCap * (kCompactTile / 32);
+  HIPCHK(dalloc(&dDeadBits, words));
+  HIPCHK(dalloc(&dHoles, cap));
   HIPCHK(dalloc(&dTileBirth, nTilesCap));
-  HIPCHK(dalloc(&dTileAlivePre, nTilesCap));
   HIPCHK(dalloc(&dTileBirthPre, nTilesCap));
-  blockStride = finalize_blocks(cap);
-  HIPCHK(dalloc(&dBlockSum, 2 * (size_t)blockStride));
+  HIPCHK(dalloc(&dBlockSum, finalize_blocks(nTilesCap * kCompactTile)));
   if (segHigh) HIPCHK(dalloc(&dSegScratch, seg_sort_words(cap, (int)R, std::max(segLow, segHigh))));
-  HIPCHK(hipMemsetAsync(dTileAlive, 0, nTilesCap * sizeof(uint32_t), stream));
+  HIPCHK(hipMemsetAsync(dDeadBits, 0, words * sizeof(uint32_t), stream));
+  for (int k = 0; k < 2; ++k) {
+    HIPCHK(dalloc(&dTileDead[k], nTilesCap));
+    HIPCHK(hipMemsetAsync(dTileDead[k], 0, nTilesCap * sizeof(uint32_t), stream));
+  }
   HIPCHK(hipMemsetAsync(dTileBirth, 0, nTilesCap * sizeof(uint32_t), stream));
   HIPCHK(hipMemsetAsync(dBirthType, 0, (size_t)cap * sizeof(int), stream));
+  return SMD_OK;
+}
+
+smd_status Engine::alloc_apart() {
+  for (int k = 0; k < 2; ++k) HIPCHK(dalloc(&dW[k], (size_t)cap + extraCap));
+  return SMD_OK;
+}
+
+// New particles whose fourth components do not pack: from here on all
+// components live apart.
+smd_status Engine::take_apart(const float* pos4, size_t n) {
+  if (wApart || components_pack(pos4, n)) return SMD_OK;
+  drop_graph();
+  HIPCHK(hipStreamSynchronize(stream));
+  smd_status st = alloc_apart();
+  if (st != SMD_OK) return st;
+  wApart = true;
+  HIPCHK(launch_split_w(dPT[cur], dW[cur], cap + extraCap, stream));
+  HIPCHK(hipStreamSynchronize(stream));
+  return SMD_OK;
+}
+
+CanonMap Engine::canon_map() const {
+  CanonMap m;
+  m.srcOff = dNewOff;  // the layout of the last step: swapped with the next one's
+  m.alive = dAlive;
+  m.holeOff = dHoleOff;
+  m.holeN = dHoleN;
+  m.holes = dHoles;
+  m.extraOff = dExtraOff;
+  m.extraBase = cap;
+  return m;
+}
+
+// The map of particles that lie densely by dRepOff / dRepCount in dPT[cur].
+smd_status Engine::set_dense() {
+  HIPCHK(launch_identity_map((int)R, dRepOff, dRepCount, dNewOff, dAlive, dHoleN, stream));
   return SMD_OK;
 }
 
@@ -314,8 +351,11 @@ smd_status Engine::finalize(uint32_t capacity) {
   }
   off[R] = (uint32_t)o;
   for (uint32_t** p : {&dRepOff, &dNewOff}) HIPCHK(dalloc(p, R + 1));
-  for (uint32_t** p : {&dRepCount, &dNewCount, &dAliveBase, &dBirthBase, &dRepAlive, &dRepDeaths, &dRepBirths})
+  for (uint32_t** p : {&dRepCount, &dNewCount, &dAlive, &dHoleOff, &dHoleN, &dExtraOff, &dBirthBase, &dRepDeaths,
+                       &dRepBirths})
     HIPCHK(dalloc(p, R));
+  HIPCHK(hipMemset(dHoleOff, 0, R * sizeof(uint32_t)));
+  HIPCHK(hipMemset(dExtraOff, 0, R * sizeof(uint32_t)));
   HIPCHK(hipMemcpy(dRepOff, off.data(), (R + 1) * sizeof(uint32_t), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(dRepCount, cnt.data(), R * sizeof(uint32_t), hipMemcpyHostToDevice));
   HIPCHK(hipMemset(dRepDeaths, 0, R * sizeof(uint32_t)));
@@ -414,13 +454,17 @@ smd_status Engine::finalize(uint32_t capacity) {
   }
 
   // Particles.
+  for (uint32_t r = 0; r < R && !wApart; ++r) wApart = !components_pack(pos0[r].data(), cnt[r]);
   smd_status st = alloc_particle_buffers((uint32_t)c);
   if (st != SMD_OK) return st;
   for (uint32_t r = 0; r < R; ++r) {
     if (cnt[r] == 0) continue;
-    HIPCHK(upload_particles(pos0[r].data(), type0[r].data(), cnt[r], dPT[0] + off[r], dW[0] + off[r]));
+    HIPCHK(upload_particles(pos0[r].data(), type0[r].data(), cnt[r], dPT[0] + off[r],
+                            wApart ? dW[0] + off[r] : nullptr));
   }
   cur = 0;
+  st = set_dense();
+  if (st != SMD_OK) return st;
   Nub = total;
   knownN = total;
   stepsDone = 0;
@@ -428,6 +472,9 @@ smd_status Engine::finalize(uint32_t capacity) {
                        hipHostMallocMapped | hipHostMallocCoherent));
   std::memset(countRing, 0, kRing * sizeof(unsigned long long));
   HIPCHK(hipHostGetDevicePointer((void**)&dCountRing, countRing, 0));
+  HIPCHK(hipHostMalloc((void**)&hostStatus, sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
+  *hostStatus = 0;
+  HIPCHK(hipHostGetDevicePointer((void**)&dHostStatus, hostStatus, 0));
   HIPCHK(dalloc(&dStepCount, 1));
   HIPCHK(hipMemset(dStepCount, 0, sizeof(uint32_t)));
   lastSeen = 0;
@@ -467,23 +514,22 @@ smd_status Engine::grow(uint64_t need) {
   float4* keepPT = nullptr;
   float* keepW = nullptr;
   HIPCHK(dalloc(&keepPT, n));
-  HIPCHK(dalloc(&keepW, n));
-  if (n) {
-    HIPCHK(hipMemcpy(keepPT, dPT[cur], n * sizeof(float4), hipMemcpyDeviceToDevice));
-    HIPCHK(hipMemcpy(keepW, dW[cur], n * sizeof(float), hipMemcpyDeviceToDevice));
-  }
+  if (wApart) HIPCHK(dalloc(&keepW, n));
+  HIPCHK(launch_compact(export_args(-1), n, keepPT, keepW, stream));
+  HIPCHK(hipStreamSynchronize(stream));
   free_particle_buffers();
   smd_status st = alloc_particle_buffers((uint32_t)nc);
   if (st != SMD_OK) return st;
   cur = 0;
   if (n) {
-    HIPCHK(hipMemcpy(dPT[0], keepPT, n * sizeof(float4), hipMemcpyDeviceToDevice));
-    HIPCHK(hipMemcpy(dW[0], keepW, n * sizeof(float), hipMemcpyDeviceToDevice));
+    HIPCHK(hipMemcpyAsync(dPT[0], keepPT, n * sizeof(float4), hipMemcpyDeviceToDevice, stream));
+    if (wApart) HIPCHK(hipMemcpyAsync(dW[0], keepW, n * sizeof(float), hipMemcpyDeviceToDevice, stream));
   }
+  st = set_dense();
+  HIPCHK(hipStreamSynchronize(stream));
   dfree(keepPT);
   dfree(keepW);
-  HIPCHK(hipStreamSynchronize(stream));
-  return SMD_OK;
+  return st;
 }
 
 smd_status Engine::ensure_capacity() {
@@ -748,11 +794,7 @@ hipError_t Engine::sort_keys(uint32_t maxN, bool tilesLaid, StageTimer* timer, b
   return e;
 }
 
-smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
-  auto mark = [&](int stage) {
-    if (timer) (void)hipEventRecord(timer->ev[stage], stream);
-  };
-  mark(0);
+ProducerArgs Engine::producer_args() const {
   ProducerArgs pa;
   pa.tables = dTables;
   pa.streamReplica = dStreamReplica;
@@ -762,17 +804,29 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
   pa.mtPar = dMtPar;
   pa.Stot = Stot;
   pa.gauss = dGauss;
-  pa.pt = dPT[cur];
-  pa.w = dW[cur];
+  pa.ptIn = dPT[cur];
+  pa.map = canon_map();
+  pa.pt = dPT[cur ^ 1];
+  pa.wIn = dW[cur];
+  pa.w = dW[cur ^ 1];
   pa.addedPos = dAddedPos;
   pa.birthType = dBirthType;
   pa.key = sb.keys;
   pa.deadKey = deadKey;
   pa.repDeaths = dRepDeaths;
   pa.repBirths = dRepBirths;
-  pa.tileAlive = dTileAlive;
+  pa.deaths = DeathMarks{dDeadBits, dTileDead[cur]};
   pa.tileBirth = dTileBirth;
   pa.retire = dRetire;
+  return pa;
+}
+
+smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
+  auto mark = [&](int stage) {
+    if (timer) (void)hipEventRecord(timer->ev[stage], stream);
+  };
+  mark(0);
+  ProducerArgs pa = producer_args();
   // the segmented sort's tile table by one more workgroup of the producer's
   // launch (it reads only the per-replica counts the step starts with)
   const bool tilesLaid = anyBim && seg_sorted() && sort_form(maxN) == SortForm::kDigits;
@@ -795,7 +849,7 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
   }
   mark(1);
   if (anyBim) {
-    sb.gatherSrc = dPT[cur];
+    sb.gatherSrc = dPT[cur ^ 1];
     sb.gatherDst = dSortedPT;
     sb.gatherDeadKey = deadKey;
     sb.sizeHint = (uint32_t)std::min<uint64_t>(knownN, 0xFFFFFFFFu);
@@ -828,10 +882,10 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
     ra.sortedPT = dSortedPT;
     ra.vals = sb.vals;
     ra.packed = sb.packIndex;
-    ra.pt = dPT[cur];
-    ra.w = dW[cur];
+    ra.pt = dPT[cur ^ 1];
+    ra.w = dW[cur ^ 1];
     ra.repDeaths = dRepDeaths;
-    ra.tileAlive = dTileAlive;
+    ra.deaths = pa.deaths;
     HIPCHK(launch_resolve(ra, stream));
     mark(5);
   } else {
@@ -844,51 +898,53 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
   fa.repBirths = dRepBirths;
   fa.newOff = dNewOff;
   fa.newCount = dNewCount;
-  fa.aliveBase = dAliveBase;
+  fa.alive = dAlive;
+  fa.holeOff = dHoleOff;
+  fa.holeN = dHoleN;
+  fa.holes = dHoles;
+  fa.extraOff = dExtraOff;
   fa.birthBase = dBirthBase;
-  fa.repAlive = dRepAlive;
   fa.dNnext = dNnext;
   fa.dN = dN;
-  fa.tileAlive = dTileAlive;
-  fa.tileBirth = dTileBirth;
-  fa.tileAlivePre = dTileAlivePre;
+  fa.deaths = pa.deaths;
+  fa.tileDeadNext = dTileDead[cur ^ 1];
+  fa.tileBirth = anySplit ? dTileBirth : nullptr;
   fa.tileBirthPre = dTileBirthPre;
   fa.particleSteps = dParticleSteps;
   fa.stepCount = dStepCount;
   fa.countRing = dCountRing;
   fa.ringMask = kRing - 1;
+  fa.status = dStatus;
+  fa.hostStatus = dHostStatus;
   fa.injCount = dInjCount;
   fa.zCount = anyZero ? dZCount : nullptr;
   fa.zeroBase = dZeroBase;
   fa.injBase = dInjBase;
   fa.retire = dRetire;
   fa.blockSum = dBlockSum;
-  fa.blockStride = blockStride;
-  HIPCHK(launch_finalize(fa, maxN, stream));
+  fa.tilesCap = nTilesCap;
+  HIPCHK(launch_finalize(fa, stream));
   mark(6);
-  ScatterArgs sa;
-  sa.R = (int)R;
-  sa.dN = dN;
-  sa.repOff = dRepOff;
-  sa.newOff = dNewOff;
-  sa.aliveBase = dAliveBase;
-  sa.birthBase = dBirthBase;
-  sa.repAlive = dRepAlive;
-  sa.tileAlivePre = dTileAlivePre;
-  sa.tileBirthPre = dTileBirthPre;
-  sa.pt = dPT[cur];
-  sa.w = dW[cur];
-  sa.addedPos = dAddedPos;
-  sa.birthType = dBirthType;
-  sa.tileBirth = dTileBirth;
-  sa.ptOut = dPT[cur ^ 1];
-  sa.wOut = dW[cur ^ 1];
-  sa.blockSum = dBlockSum;
-  sa.blockStride = blockStride;
-  HIPCHK(launch_scatter(sa, maxN, stream));
+  float4* const extra = dPT[cur ^ 1] + cap;
+  float* const extraW = wApart ? dW[cur ^ 1] + cap : nullptr;
+  if (anySplit) {
+    BirthArgs ba;
+    ba.R = (int)R;
+    ba.dN = dN;
+    ba.repOff = dRepOff;
+    ba.birthBase = dBirthBase;
+    ba.extraOff = dExtraOff;
+    ba.tileBirthPre = dTileBirthPre;
+    ba.addedPos = dAddedPos;
+    ba.birthType = dBirthType;
+    ba.tileBirth = dTileBirth;
+    ba.blockSum = dBlockSum;
+    ba.extra = extra;
+    ba.extraW = extraW;
+    HIPCHK(launch_births(ba, maxN, stream));
+  }
   if (anyZero)
-    HIPCHK(launch_zero_place((int)R, dTables, dZPos, dZType, dZCount, dNewOff, dZeroBase, dPT[cur ^ 1],
-                             dW[cur ^ 1], stream));
+    HIPCHK(launch_zero_place((int)R, dTables, dZPos, dZType, dZCount, dZeroBase, extra, extraW, stream));
   if (injN) {
     InjectArgs ia;
     ia.injPos = dInjPos;
@@ -896,10 +952,9 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
     ia.injRep = dInjRep;
     ia.injSrcOff = dInjSrcOff;
     ia.nInj = injN;
-    ia.newOff = dNewOff;
     ia.injBase = dInjBase;
-    ia.ptOut = dPT[cur ^ 1];
-    ia.wOut = dW[cur ^ 1];
+    ia.extra = extra;
+    ia.extraW = extraW;
     HIPCHK(launch_inject(ia, stream));
     injN = 0;
   }
@@ -948,16 +1003,15 @@ smd_status Engine::step(int nsteps) {
 smd_status Engine::sync() {
   HIPCHK(hipSetDevice(device));
   HIPCHK(hipStreamSynchronize(stream));
-  refresh_bound(true);
+  refresh_bound(false);  // the stream has drained: the last step's count is there
   return check_status();
 }
 
 // Error bits the kernels set since finalize (they stay set: the state after
 // such a step is not trustworthy).
 smd_status Engine::check_status() {
-  if (!dStatus) return SMD_OK;
-  uint32_t v = 0;
-  HIPCHK(hipMemcpy(&v, dStatus, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  if (!hostStatus) return SMD_OK;
+  const uint32_t v = __atomic_load_n(hostStatus, __ATOMIC_ACQUIRE);
   if (v & kStatusZeroOverflow) {
     set_error("order-0 reactions created more particles in one step than the per-step limit");
     return SMD_ERR_CAPACITY;
@@ -1089,6 +1143,7 @@ smd_status Engine::admit(int slot, const smd_sim_spec& spec, const float* pos4, 
       return SMD_ERR_INVALID;
     }
   smd_status st = sync();
+  if (st == SMD_OK) st = take_apart(pos4, n);
   if (st != SMD_OK) return st;
   const uint32_t S = T.numStreams;
   T.bucketOff = tabs[slot].bucketOff;
@@ -1165,17 +1220,21 @@ smd_status Engine::set_particles(const float* pos4, const int* types, uint32_t n
       return SMD_ERR_INVALID;
     }
   smd_status st = sync();
+  if (st == SMD_OK) st = take_apart(pos4, n);
   if (st != SMD_OK) return st;
   if (step_bound(n) > cap) {
     knownN = 0;
     st = grow(4ull * n);
     if (st != SMD_OK) return st;
   }
-  if (n) HIPCHK(upload_particles(pos4, types, n, dPT[cur], dW[cur]));
+  if (n) HIPCHK(upload_particles(pos4, types, n, dPT[cur], wApart ? dW[cur] : nullptr));
   const uint32_t off[2] = {0u, n};
   HIPCHK(hipMemcpy(dRepOff, off, 2 * sizeof(uint32_t), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(dRepCount, &n, sizeof(uint32_t), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(dN, &n, sizeof(uint32_t), hipMemcpyHostToDevice));
+  st = set_dense();
+  if (st != SMD_OK) return st;
+  HIPCHK(hipStreamSynchronize(stream));
   Nub = n;
   knownN = n;
   lastSeen = stepsDone;  // counts published before this call are stale
@@ -1196,6 +1255,33 @@ smd_status Engine::counts(uint32_t* out) {
   return SMD_OK;
 }
 
+ExportArgs Engine::export_args(int r) const {
+  ExportArgs a;
+  a.pt = dPT[cur];
+  a.w = wApart ? dW[cur] : nullptr;
+  a.map = canon_map();
+  a.repOff = dRepOff;
+  a.repCount = dRepCount;
+  a.R = (int)R;
+  a.rep = r;
+  a.begin = 0;
+  a.cap = 0xFFFFFFFFu;
+  a.pos4 = nullptr;
+  a.types = nullptr;
+  a.header = nullptr;
+  return a;
+}
+
+smd_status Engine::view_buffers(uint32_t n) {
+  if (n <= viewCap && dViewPos) return SMD_OK;
+  dfree(dViewPos);
+  dfree(dViewType);
+  viewCap = std::max<uint32_t>(n, 1u);
+  HIPCHK(dalloc(&dViewPos, viewCap));
+  HIPCHK(dalloc(&dViewType, viewCap));
+  return SMD_OK;
+}
+
 smd_status Engine::get(int r, float* pos4, int* types, uint32_t capN, uint32_t* nOut) {
   if (r < 0 || (uint32_t)r >= R) {
     set_error("replica id out of range");
@@ -1203,12 +1289,21 @@ smd_status Engine::get(int r, float* pos4, int* types, uint32_t capN, uint32_t* 
   }
   smd_status st = sync();
   if (st != SMD_OK) return st;
-  uint32_t off = 0, n = 0;
-  HIPCHK(hipMemcpy(&off, dRepOff + r, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  uint32_t n = 0;
   HIPCHK(hipMemcpy(&n, dRepCount + r, sizeof(uint32_t), hipMemcpyDeviceToHost));
   if (nOut) *nOut = n;
   const uint32_t m = std::min(n, capN);
-  if (m && (pos4 || types)) HIPCHK(download_particles(dPT[cur] + off, dW[cur] + off, m, pos4, types));
+  if (!m || !(pos4 || types)) return SMD_OK;
+  st = view_buffers(m);
+  if (st != SMD_OK) return st;
+  ExportArgs a = export_args(r);
+  a.cap = m;
+  a.pos4 = pos4 ? dViewPos : nullptr;
+  a.types = types ? dViewType : nullptr;
+  HIPCHK(launch_export(a, m, stream));
+  HIPCHK(hipStreamSynchronize(stream));
+  if (pos4) HIPCHK(hipMemcpy(pos4, dViewPos, m * sizeof(float4), hipMemcpyDeviceToHost));
+  if (types) HIPCHK(hipMemcpy(types, dViewType, m * sizeof(int), hipMemcpyDeviceToHost));
   return SMD_OK;
 }
 
@@ -1221,14 +1316,12 @@ smd_status Engine::view(float4** pos4, int** types, uint32_t* nOut) {
   if (st != SMD_OK) return st;
   uint32_t n = 0;
   HIPCHK(hipMemcpy(&n, dN, sizeof(uint32_t), hipMemcpyDeviceToHost));
-  if (n > viewCap || !dViewPos) {
-    dfree(dViewPos);
-    dfree(dViewType);
-    viewCap = std::max<uint32_t>(n, 1u);
-    HIPCHK(dalloc(&dViewPos, viewCap));
-    HIPCHK(dalloc(&dViewType, viewCap));
-  }
-  HIPCHK(launch_unpack(dPT[cur], dW[cur], n, dViewPos, dViewType, stream));
+  st = view_buffers(n);
+  if (st != SMD_OK) return st;
+  ExportArgs a = export_args(-1);
+  a.pos4 = dViewPos;
+  a.types = dViewType;
+  HIPCHK(launch_export(a, n, stream));
   HIPCHK(hipStreamSynchronize(stream));
   *pos4 = dViewPos;
   *types = dViewType;
@@ -1272,30 +1365,12 @@ smd_status Engine::debug_stage(int stage, float* pos4, int* types, uint32_t* key
   HIPCHK(hipMemcpy(&n, dN, sizeof(uint32_t), hipMemcpyDeviceToHost));
   const uint32_t maxN = n;
   broken = true;
-  ProducerArgs pa;
-  pa.tables = dTables;
-  pa.streamReplica = dStreamReplica;
-  pa.repOff = dRepOff;
-  pa.repCount = dRepCount;
-  pa.mtState = dMtState;
-  pa.mtPar = dMtPar;
-  pa.Stot = Stot;
-  pa.gauss = dGauss;
-  pa.pt = dPT[cur];
-  pa.w = dW[cur];
-  pa.addedPos = dAddedPos;
-  pa.birthType = dBirthType;
-  pa.key = sb.keys;
-  pa.deadKey = deadKey;
-  pa.repDeaths = dRepDeaths;
-  pa.repBirths = dRepBirths;
-  pa.tileAlive = dTileAlive;
-  pa.tileBirth = dTileBirth;
+  ProducerArgs pa = producer_args();
   pa.retire = nullptr;
   HIPCHK(launch_producer(pa, producerBlock, stream));
   uint32_t live = 0;
   if (stage >= 2) {
-    sb.gatherSrc = dPT[cur];
+    sb.gatherSrc = dPT[cur ^ 1];
     sb.gatherDst = dSortedPT;
     sb.gatherDeadKey = deadKey;
     sb.sizeHint = (uint32_t)std::min<uint64_t>(knownN, 0xFFFFFFFFu);
@@ -1328,10 +1403,10 @@ smd_status Engine::debug_stage(int stage, float* pos4, int* types, uint32_t* key
     ra.sortedPT = dSortedPT;
     ra.vals = sb.vals;
     ra.packed = 0;
-    ra.pt = dPT[cur];
-    ra.w = dW[cur];
+    ra.pt = dPT[cur ^ 1];
+    ra.w = dW[cur ^ 1];
     ra.repDeaths = dRepDeaths;
-    ra.tileAlive = dTileAlive;
+    ra.deaths = pa.deaths;
     HIPCHK(launch_resolve(ra, stream));
   }
   HIPCHK(hipStreamSynchronize(stream));
@@ -1339,7 +1414,28 @@ smd_status Engine::debug_stage(int stage, float* pos4, int* types, uint32_t* key
   if (nTotal) *nTotal = n;
   if (nLive) *nLive = live;
   if (n) {
-    if (pos4 || types) HIPCHK(download_particles(dPT[cur], dW[cur], n, pos4, types));
+    if (pos4 || types) {
+      // the stage's records are dense in the other buffer
+      std::vector<float4> pt(n);
+      std::vector<float> w(wApart ? n : 0);
+      HIPCHK(hipMemcpy(pt.data(), dPT[cur ^ 1], n * sizeof(float4), hipMemcpyDeviceToHost));
+      if (wApart) HIPCHK(hipMemcpy(w.data(), dW[cur ^ 1], n * sizeof(float), hipMemcpyDeviceToHost));
+      for (uint32_t i = 0; i < n; ++i) {
+        uint32_t b;
+        std::memcpy(&b, &pt[i].w, sizeof(b));
+        // an absent product's type is -1
+        const int ty = (int)(b & (uint32_t)kTypeMask);
+        if (types) types[i] = ty == kTypeMask ? -1 : ty;
+        b &= ~(uint32_t)kTypeMask;
+        if (pos4) {
+          pos4[4 * i] = pt[i].x;
+          pos4[4 * i + 1] = pt[i].y;
+          pos4[4 * i + 2] = pt[i].z;
+          if (wApart) pos4[4 * i + 3] = w[i];
+          else std::memcpy(&pos4[4 * i + 3], &b, sizeof(b));
+        }
+      }
+    }
     if (stage == 1 && keysSorted) HIPCHK(hipMemcpy(keysSorted, sb.keys, n * sizeof(uint32_t), hipMemcpyDeviceToHost));
     if (stage >= 2 && keysSorted)
       HIPCHK(hipMemcpy(keysSorted, sb.keys, n * sizeof(uint32_t), hipMemcpyDeviceToHost));

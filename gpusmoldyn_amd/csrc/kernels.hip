@@ -7,8 +7,10 @@
 //   k_first       lower bound of every bucket in the sorted keys
 //   k_candidates  neighbour-cell search for each particle's nearest reactive partner
 //   k_resolve     mutual-nearest pairs react (bimReact)                (one thread per RNG stream)
-//   k_finalize    per-replica counts, offsets and compaction-tile prefixes (one workgroup)
-//   k_scatter     order-preserving compaction of survivors, births appended per replica
+//   k_finalize    per-replica counts and offsets, the sorted list of removed particles
+//   k_births      births behind their replica's survivors
+// Removed particles stay in place until the next step's producer, which reads
+// every record anyway, reads around them (CanonMap) and writes densely.
 // (k_gather copies the records after the single-sweep sort variant.)
 #include <hip/hip_runtime.h>
 
@@ -68,7 +70,11 @@ __global__ __launch_bounds__(kBS) void k_mt_fill(uint32_t* __restrict__ st, cons
 // the surface semantics of surfaces_kernel.cuh) + calcHash
 // (particles_kernel.cu:188-207), fused.  Thread g owns stream g and handles
 // the particles i = s, s + S, s + 2S, ... of its replica in increasing order,
-// so every stream's draws happen in a fixed order.
+// so every stream's draws happen in a fixed order.  It reads the records from
+// where the last step left them (CanonMap) and writes them densely: the pass
+// that used to move every record and fourth component once more per step (40
+// bytes per particle: 67 us of 474 for 9.36M particles, 33 of 315 for 4M) is
+// gone for a few registers here.
 // ---------------------------------------------------------------------------
 // Per-type and per-reaction entries the producer indexes per particle, staged
 // in LDS for each wave's replica (a few hundred bytes per wave).
@@ -87,10 +93,45 @@ struct ProducerLds {
 template <int BS>
 __device__ __forceinline__ void seg_tiles_body(const SegTilesArgs& a, uint32_t* wsum, uint32_t* sLong);
 
+// Survivors of a replica that come after hole k number at least (slot of the
+// hole) - srcOff - k before it; how many of its H holes lie before survivor il.
+__device__ __forceinline__ uint32_t holes_before(const uint32_t* __restrict__ holes, uint32_t H, uint32_t srcOff,
+                                                 uint32_t il) {
+  uint32_t lo = 0, hi = H;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (holes[mid] - srcOff - mid <= il) lo = mid + 1u;
+    else hi = mid;
+  }
+  return lo;
+}
+
+// Marks the slots base + (bits of mask) removed; one lane.
+__device__ __forceinline__ void mark_removed(const DeathMarks& d, uint32_t base, uint64_t mask) {
+  const uint32_t sh = base & 31u, w = base >> 5;
+  const uint32_t m0 = (uint32_t)(mask << sh);
+  const uint64_t m1 = mask >> (32u - sh);
+  if (m0) atomicOr(&d.bits[w], m0);
+  if ((uint32_t)m1) atomicOr(&d.bits[w + 1u], (uint32_t)m1);
+  if (m1 >> 32) atomicOr(&d.bits[w + 2u], (uint32_t)(m1 >> 32));
+}
+
+// Adds the set bits of mask (slots from base on) to the counts of their tiles.
+__device__ __forceinline__ void count_tiles(uint32_t* tiles, uint32_t base, uint64_t mask) {
+  const uint32_t t0 = base / kCompactTile;
+  const uint32_t split = (t0 + 1) * kCompactTile - base;  // first bit of the next tile
+  const uint64_t lo = split >= 64 ? ~0ull : ((1ull << split) - 1ull);
+  const uint32_t n0 = __popcll(mask & lo), n1 = __popcll(mask & ~lo);
+  if (n0) atomicAdd(&tiles[t0], n0);
+  if (n1) atomicAdd(&tiles[t0 + 1u], n1);
+}
+
 // The replica tables arrive as a separate read-only, non-aliased argument:
 // their wave-uniform fields then load through the scalar cache, whose waits
 // do not hold up the particle records in flight.
-template <int BS>
+// APART: the fourth components are not in the records but in arrays of their
+// own (a.wIn, a.w).
+template <int BS, bool APART>
 __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTables* __restrict__ tables) {
   __shared__ uint32_t lds_mt[kMtNN * BS];
   __shared__ float lds_gauss[kGaussDim / 2];  // half of the table (gauss_entry)
@@ -145,19 +186,50 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
     // the replica's box, grid and reaction flags in registers for the loop
     const BoxGeom G = box_geom(T);
     const int hasUni = T.hasUni, unbindOffsets = T.unbindOffsets, numSpheres = T.numSpheres;
-    // Records are requested one pair of particles ahead.
-    auto rec = [&](uint32_t it) __attribute__((always_inline)) {
-      const uint32_t iq = s + it * S;
-      return (laneOK && iq < n) ? a.pt[off + iq] : make_float4(0.f, 0.f, 0.f, 0.f);
+    // Records are requested one pair of particles ahead, from where the last
+    // step left them: behind the holes of the particles it removed.  Lane q
+    // holds, for the wave's iteration 64 * block + q, the holes before lane
+    // 0's particle and how many survivors precede the next hole; a wave whose
+    // particles lie between two holes (nearly all) reads one run of slots.
+    const uint32_t so = a.map.srcOff[rw], na = a.map.alive[rw], H = a.map.holeN[rw];
+    const uint32_t* const holes = a.map.holes + a.map.holeOff[rw];
+    const uint32_t gained = a.map.extraBase + a.map.extraOff[rw] - na;  // + il
+    uint32_t holesAt = 0, nextHole = 0xFFFFFFFFu, block = 0xFFFFFFFFu;
+    auto src_index = [&](uint32_t it) __attribute__((always_inline)) -> uint32_t {
+      const uint32_t il = s + it * S;
+      uint32_t skip = 0;
+      if (H) {
+        if ((it >> 6) != block) {
+          block = it >> 6;
+          holesAt = holes_before(holes, H, so, s0 + (64u * block + lane) * S);
+          nextHole = holesAt < H ? holes[holesAt] - so - holesAt : 0xFFFFFFFFu;
+        }
+        uint32_t k = __builtin_amdgcn_readlane(holesAt, it & 63u);
+        uint32_t next = __builtin_amdgcn_readlane(nextHole, it & 63u);
+        const uint32_t last = s0 + it * S + 63u;
+        skip = k;
+        while (next <= last) {
+          ++k;
+          if (next <= il) skip = k;
+          next = k < H ? holes[k] - so - k : 0xFFFFFFFFu;
+        }
+      }
+      return il < na ? so + il + skip : gained + il;
     };
-    float4 p0 = rec(0), p1 = rec(1);
+    // (by all lanes of the wave together; src stays with the record)
+    auto rec = [&](uint32_t it, uint32_t& src) __attribute__((always_inline)) {
+      src = src_index(it);
+      return (laneOK && s + it * S < n) ? a.ptIn[src] : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
+    uint32_t i0, i1;
+    float4 p0 = rec(0, i0), p1 = rec(1, i1);
     Mt m;
     if (laneOK && !kill) mt_load<BS>(m, &lds_mt[threadIdx.x], a.mtState, a.mtPar, a.Stot, g);
     // the stream parameters are complete before the loop, so no wait inside
     // it covers them (such a wait would also cover the records in flight)
     asm volatile("" ::"v"(m.a), "v"(m.mb), "v"(m.mc), "v"(m.mti1));
     // returns the particle's births << 32 | deaths
-    auto step_one = [&](const float4 pCur, const uint32_t it) __attribute__((always_inline)) -> uint64_t {
+    auto step_one = [&](const float4 pCur, const uint32_t it, const uint32_t src) __attribute__((always_inline)) -> uint64_t {
       uint64_t db = 0;
       const uint32_t il = s + it * S;
       const bool act = laneOK && il < n;
@@ -169,10 +241,11 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
         db += 1u;
       } else if (act) {
         const float4 p = pCur;
-        int t = __float_as_int(pCur.w);
+        const int word = __float_as_int(pCur.w);
+        int t = word & kTypeMask;
         uint32_t u0, u1, u2;
         mt_draw3<BS>(m, u0, u1, u2);
-        const float rt = L.rate[t > 0 ? t : 0];
+        const float rt = L.rate[t];
         float np[3];
         np[0] = fmaf(rt, gauss_entry(lds_gauss, u0 & (kGaussDim - 1)), p.x);
         np[1] = fmaf(rt, gauss_entry(lds_gauss, u1 & (kGaussDim - 1)), p.y);
@@ -181,9 +254,7 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
         int bt = 0;
         float bp[3] = {np[0], np[1], np[2]};
         float bw = 0.0f;
-        if (t <= 0) {
-          t = 0;
-        } else if (hasUni) {
+        if (t > 0 && hasUni) {
           const int cnt = L.uniCount[t];
           const int base = L.uniStart[t];
           for (int j = 0; j < cnt; ++j) {
@@ -210,7 +281,8 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
                     np[2] = np[2] + v1[2];
                     wZero = true;
                   } else {
-                    bw = a.w[i];  // the birth inherits the parent's fourth component
+                    // the birth inherits the parent's fourth component
+                    bw = APART ? a.wIn[src] : __int_as_float(word & ~kTypeMask);
                   }
                 }
               }
@@ -228,8 +300,8 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
             key = bucketOff + grid_hash(G, np[0], np[1], np[2]);
           }
         }
-        a.pt[i] = make_float4(np[0], np[1], np[2], __int_as_float(t));
-        if (wZero) a.w[i] = 0.0f;
+        a.pt[i] = make_float4(np[0], np[1], np[2], __int_as_float((wZero ? 0 : word & ~kTypeMask) | t));
+        if (APART) a.w[i] = wZero ? 0.0f : a.wIn[src];
         a.key[i] = key;
         // birth types are zero except where the scatter has a birth to take
         // (it clears them again), so only births are written
@@ -241,20 +313,16 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
         birth = bt > 0;
         db += (alive ? 0ull : 1ull) + (birth ? (1ull << 32) : 0ull);
       }
-      // Compaction tile counters: lanes hold consecutive particle indices.
-      const uint64_t am = __ballot(alive);
+      // removed particles and births, by slot: lanes hold consecutive slots
+      const uint64_t dm = __ballot(act && !alive);
       const uint64_t bm = __ballot(birth);
-      if (lane == 0) {
+      if ((dm | bm) != 0 && lane == 0) {
         const uint32_t base = off + s0 + it * S;
-        const uint32_t t0 = base / kCompactTile;
-        const uint32_t split = (t0 + 1) * kCompactTile - base;  // first lane in the next tile
-        const uint64_t loMask = split >= 64 ? ~0ull : ((1ull << split) - 1ull);
-        const uint32_t aLo = __popcll(am & loMask), aHi = __popcll(am & ~loMask);
-        const uint32_t bLo = __popcll(bm & loMask), bHi = __popcll(bm & ~loMask);
-        if (aLo) atomicAdd(&a.tileAlive[t0], aLo);
-        if (aHi) atomicAdd(&a.tileAlive[t0 + 1], aHi);
-        if (bLo) atomicAdd(&a.tileBirth[t0], bLo);
-        if (bHi) atomicAdd(&a.tileBirth[t0 + 1], bHi);
+        if (dm) {
+          mark_removed(a.deaths, base, dm);
+          count_tiles(a.deaths.tileDead, base, dm);
+        }
+        if (bm) count_tiles(a.tileBirth, base, bm);
       }
       return db;
     };
@@ -265,12 +333,13 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
       // requested before this pair's stores, so waiting for them later does
       // not wait for those stores
       const float4 c0 = p0, c1 = p1;
-      p0 = rec(it + 2);
-      p1 = rec(it + 3);
-      db += step_one(c0, it);
-      db += step_one(c1, it + 1);
+      const uint32_t j0 = i0, j1 = i1;
+      p0 = rec(it + 2, i0);
+      p1 = rec(it + 3, i1);
+      db += step_one(c0, it, j0);
+      db += step_one(c1, it + 1, j1);
     }
-    if (it < iters) db += step_one(p0, it);
+    if (it < iters) db += step_one(p0, it, i0);
     nDeaths += (uint32_t)db;
     nBirths += (uint32_t)(db >> 32);
     if (laneOK && !kill) mt_store<BS>(m, a.mtState, a.Stot, g);
@@ -580,7 +649,7 @@ __global__ __launch_bounds__(256) void k_sort_down(const uint32_t* __restrict__ 
           // the record carries its particle's index above the type bits
           if (dk[q] < gatherDeadKey)
             gatherDst[dd[q]] = make_float4(rec[q].x, rec[q].y, rec[q].z,
-                                           __int_as_float(pack_index_type(dv[q], __float_as_int(rec[q].w))));
+                                           __int_as_float(pack_index_type(dv[q], __float_as_int(rec[q].w) & kTypeMask)));
         } else {
           valsOut[dd[q]] = dv[q];
           if (dk[q] < gatherDeadKey) gatherDst[dd[q]] = rec[q];
@@ -1226,44 +1295,26 @@ __global__ __launch_bounds__(kBS) void k_resolve(ResolveArgs a, const ReplicaTab
         }
       }
       const int nt1 = T.prodX[rx], nt2 = T.prodY[rx];
-      a.pt[mol1] = make_float4(n1[0], n1[1], n1[2], __int_as_float(nt1));
-      a.pt[mol2] = make_float4(n2[0], n2[1], n2[2], __int_as_float(nt2));
-      a.w[mol1] = 0.0f;
-      a.w[mol2] = 0.0f;
+      a.pt[mol1] = make_float4(n1[0], n1[1], n1[2], __int_as_float(nt1 & kTypeMask));
+      a.pt[mol2] = make_float4(n2[0], n2[1], n2[2], __int_as_float(nt2 & kTypeMask));
+      if (a.w) {
+        a.w[mol1] = 0.0f;
+        a.w[mol2] = 0.0f;
+      }
       if (nt1 <= 0) {
         ++deaths;
-        atomicSub(&a.tileAlive[mol1 / kCompactTile], 1u);
+        mark_removed(a.deaths, mol1, 1ull);
+        count_tiles(a.deaths.tileDead, mol1, 1ull);
       }
       if (nt2 <= 0) {
         ++deaths;
-        atomicSub(&a.tileAlive[mol2 / kCompactTile], 1u);
+        mark_removed(a.deaths, mol2, 1ull);
+        count_tiles(a.deaths.tileDead, mol2, 1ull);
       }
     }
   }
   if (loaded) mt_store<kBS>(m, a.mtState, a.Stot, g);
   if (deaths) atomicAdd(&a.repDeaths[r], deaths);
-}
-
-// ---------------------------------------------------------------------------
-// Finalize (one workgroup of 1024): per-replica survivor/birth counts and new
-// offsets, and exclusive prefixes of the compaction tile counters (which are
-// reset for the next step).
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t block_exscan1024(uint32_t v, uint32_t* wsum, uint32_t* total) {
-  const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-  uint32_t x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(x, o, 64);
-    if (lane >= (uint32_t)o) x += y;
-  }
-  if (lane == 63) wsum[w] = x;
-  __syncthreads();
-  uint32_t pre = 0;
-  for (uint32_t k = 0; k < w; ++k) pre += wsum[k];
-  if (threadIdx.x == 1023) *total = pre + x;
-  __syncthreads();
-  return pre + x - v;
 }
 
 // Exclusive scans of K values per thread over the 1024-thread workgroup in
@@ -1304,235 +1355,246 @@ __device__ __forceinline__ void block_exscan1024_k(const uint32_t (&v)[K], uint3
   __syncthreads();
 }
 
-// Compaction tiles per finalize workgroup (1024 threads x 4 consecutive tiles).
-constexpr uint32_t kFinTPT = 1;
-constexpr uint32_t kFinBlockTiles = 1024 * kFinTPT;
+// ---------------------------------------------------------------------------
+// Finalize: per-step bookkeeping after the pair step.  The removed particles
+// stay where they are; the next step reads around them (CanonMap).  Workgroup
+// g turns the death bits of tiles [g * 1024, (g + 1) * 1024) into their part
+// of the sorted hole list (its place: the deaths of all earlier tiles), clears
+// them, and scans the tiles' births.  Workgroup 0 also lays out every
+// replica's particles for the next step and publishes the step's counts.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kFinBlockTiles = 1024;
 
-// Per-step bookkeeping after the pair step.  Workgroup g scans the compaction
-// tiles [g * 1024, (g + 1) * 1024): exclusive prefixes of both counters inside
-// the block, the counters reset, the block's totals published for the
-// scatter (which adds the totals of the earlier blocks).  Workgroup 0 also
-// lays out every replica's new segment and publishes the step's counts.
 __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
-  __shared__ uint32_t wsum[3][16];
+  __shared__ uint32_t wsum[4][16];
+  __shared__ uint32_t s_base[16];
   const uint32_t t0 = blockIdx.x * kFinBlockTiles;
-  const uint32_t e0 = t0 + threadIdx.x * kFinTPT;
-  // Every load that does not depend on the particle count is issued before
-  // that count arrives: this block's compaction-tile counters (up to the
-  // launch's tile bound; entries past the count are masked below) and the
-  // step counters.  All loads come before any store (the arguments may alias).
-  uint32_t va[kFinTPT], vb[kFinTPT];
-#pragma unroll
-  for (uint32_t k = 0; k < kFinTPT; ++k) {
-    const uint32_t e = e0 + k;
-    va[k] = e < a.maxTiles ? a.tileAlive[e] : 0u;
-    vb[k] = e < a.maxTiles ? a.tileBirth[e] : 0u;
-  }
-  uint32_t stepPrev = 0;
+  const uint32_t e = t0 + threadIdx.x;
+  // every load that does not need another one's result is issued first
+  const uint32_t n = *a.dN;
+  const uint32_t dead = e < a.tilesCap ? a.deaths.tileDead[e] : 0u;
+  const uint32_t born = a.tileBirth && e < a.tilesCap ? a.tileBirth[e] : 0u;
+  uint32_t stepPrev = 0, status = 0;
   unsigned long long psPrev = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     stepPrev = *a.stepCount;
     psPrev = *a.particleSteps;
+    status = *a.status;
   }
-  const uint32_t n = *a.dN;
-  const uint32_t nTiles = (n + kCompactTile - 1) / kCompactTile;
-  if (blockIdx.x > 0 && t0 >= nTiles) return;
-#pragma unroll
-  for (uint32_t k = 0; k < kFinTPT; ++k) {
-    if (e0 + k >= nTiles) {
-      va[k] = 0u;
-      vb[k] = 0u;
-    }
-  }
+  if (e < a.tilesCap) a.tileDeadNext[e] = 0u;
+  if (blockIdx.x > 0 && t0 >= (n + kCompactTile - 1u) / kCompactTile) return;  // no particles here
+  uint32_t before = 0;
+  for (uint32_t q = threadIdx.x; q < t0; q += 1024u) before += a.deaths.tileDead[q];
   if (blockIdx.x == 0) {
     // replicas
-    uint32_t cN = 0, cA = 0, cB = 0;
+    uint32_t c[4] = {0u, 0u, 0u, 0u};
     for (uint32_t b = 0; b < (uint32_t)a.R; b += 1024) {
       const uint32_t r = b + threadIdx.x;
-      uint32_t alive = 0, births = 0, zc = 0, inj = 0;
+      uint32_t deaths = 0, alive = 0, births = 0, zc = 0, inj = 0;
       if (r < (uint32_t)a.R) {
-        alive = a.repCount[r] - a.repDeaths[r];
+        deaths = a.repDeaths[r];
+        alive = a.repCount[r] - deaths;
         births = a.repBirths[r];
         if (a.zCount) zc = a.zCount[r];
         if (a.injCount) inj = a.injCount[r];
       }
-      // new segment of replica r: [survivors, births, created, admitted]
-      const uint32_t v[3] = {alive + births + zc + inj, alive, births};
-      uint32_t ex[3], tot[3];
-      block_exscan1024_k<3>(v, ex, tot, wsum);
+      // replica r's next particles: [survivors, births, created, admitted]
+      const uint32_t gain = births + zc + inj;
+      const uint32_t v[4] = {alive + gain, deaths, gain, births};
+      uint32_t ex[4] = {0u, 0u, 0u, 0u}, tot[4] = {v[0], v[1], v[2], v[3]};  // one replica: no scan
+      if (a.R > 1) block_exscan1024_k<4>(v, ex, tot, wsum);
       if (r < (uint32_t)a.R) {
-        a.newOff[r] = cN + ex[0];
+        a.newOff[r] = c[0] + ex[0];
         a.newCount[r] = v[0];
-        a.aliveBase[r] = cA + ex[1];
-        a.birthBase[r] = cB + ex[2];
-        a.repAlive[r] = alive;
+        a.alive[r] = alive;
+        a.holeOff[r] = c[1] + ex[1];
+        a.holeN[r] = deaths;
+        a.extraOff[r] = c[2] + ex[2];
+        a.birthBase[r] = c[3] + ex[3];
         a.repDeaths[r] = 0;
         a.repBirths[r] = 0;
-        if (a.zCount) a.zeroBase[r] = alive + births;
+        if (a.zCount) a.zeroBase[r] = c[2] + ex[2] + births;
         if (a.injCount) {
-          a.injBase[r] = alive + births + zc;
+          a.injBase[r] = c[2] + ex[2] + births + zc;
           a.injCount[r] = 0;
         }
         if (a.retire) a.retire[r] = 0;
       }
-      cN += tot[0];
-      cA += tot[1];
-      cB += tot[2];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) c[k] += tot[k];
     }
     if (threadIdx.x == 0) {
-      a.newOff[a.R] = cN;
-      *a.dNnext = cN;
+      a.newOff[a.R] = c[0];
+      *a.dNnext = c[0];
       *a.particleSteps = psPrev + n;
+      if (status) __hip_atomic_store(a.hostStatus, status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       // the host reads the particle count after each step from this ring,
       // tagged with the step number (no copy or event in the stream)
       const uint32_t st = stepPrev + 1u;
       *a.stepCount = st;
-      __hip_atomic_store(&a.countRing[st & a.ringMask], ((unsigned long long)st << 32) | cN, __ATOMIC_RELAXED,
+      __hip_atomic_store(&a.countRing[st & a.ringMask], ((unsigned long long)st << 32) | c[0], __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
-  // this block's compaction tiles: exclusive prefixes inside the block,
-  // counters reset, block totals for the scatter
-  uint32_t sum[2] = {0u, 0u};
-#pragma unroll
-  for (uint32_t k = 0; k < kFinTPT; ++k) {
-    const uint32_t e = e0 + k;
-    sum[0] += va[k];
-    sum[1] += vb[k];
-    if (e < nTiles) a.tileAlive[e] = 0;  // the birth counters are cleared by the scatter
+  if (!__syncthreads_or((dead | born) != 0u)) {
+    if (a.tileBirth && threadIdx.x == 0) a.blockSum[blockIdx.x] = 0u;
+    return;
   }
+  uint4 x[kCompactTile / 128];
+  if (dead) {
+    uint4* const bits = (uint4*)(a.deaths.bits + (size_t)e * (kCompactTile / 32));
+#pragma unroll
+    for (int q = 0; q < kCompactTile / 128; ++q) x[q] = bits[q];
+#pragma unroll
+    for (int q = 0; q < kCompactTile / 128; ++q) bits[q] = make_uint4(0u, 0u, 0u, 0u);
+  }
+  before = wave_sum(before);
+  if ((threadIdx.x & 63u) == 0u) s_base[threadIdx.x >> 6] = before;
+  const uint32_t v[2] = {dead, born};
   uint32_t ex[2], tot[2];
-  block_exscan1024_k<2>(sum, ex, tot, wsum);
-  uint32_t ra = ex[0], rb = ex[1];
+  block_exscan1024_k<2>(v, ex, tot, wsum);
+  if (dead) {
+    uint32_t at = ex[0];
 #pragma unroll
-  for (uint32_t k = 0; k < kFinTPT; ++k) {
-    const uint32_t e = e0 + k;
-    if (e < nTiles) {
-      a.tileAlivePre[e] = ra;
-      a.tileBirthPre[e] = rb;
+    for (uint32_t q = 0; q < 16u; ++q) at += s_base[q];
+#pragma unroll
+    for (int q = 0; q < kCompactTile / 128; ++q) {
+      const uint32_t w[4] = {x[q].x, x[q].y, x[q].z, x[q].w};
+#pragma unroll
+      for (uint32_t k = 0; k < 4u; ++k) {
+        for (uint32_t m = w[k]; m; m &= m - 1u)
+          a.holes[at++] = e * kCompactTile + q * 128u + k * 32u + (uint32_t)__ffs((int)m) - 1u;
+      }
     }
-    ra += va[k];
-    rb += vb[k];
   }
-  if (threadIdx.x == 0) {
-    a.blockSum[blockIdx.x] = tot[0];
-    a.blockSum[a.blockStride + blockIdx.x] = tot[1];
+  if (a.tileBirth) {
+    if (e < a.tilesCap) a.tileBirthPre[e] = ex[1];
+    if (threadIdx.x == 0) a.blockSum[blockIdx.x] = tot[1];
   }
 }
 
 // ---------------------------------------------------------------------------
-// Scatter: order-preserving compaction (the intent of compactPosAndTypeD,
-// particles_kernel.cu:97-123, done out of place).  Replica r's new segment is
-// [survivors of r in index order, births of r in parent index order].
+// Births go behind their replica's survivors in parent index order (the order
+// of compactPosAndTypeD, particles_kernel.cu:97-123).  A wave looks after 16
+// tiles and reads the birth types of those with births.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_scatter(ScatterArgs a, const uint32_t* __restrict__ repOff) {
-  __shared__ uint32_t s_wa[16], s_wb[16];
+constexpr uint32_t kBirthTiles = 16;
+static_assert(kFinBlockTiles % kBirthTiles == 0, "a wave's tiles lie in one finalize block");
+
+__global__ __launch_bounds__(256) void k_births(BirthArgs a, const uint32_t* __restrict__ repOff) {
   const uint32_t n = *a.dN;
-  const uint32_t tile = blockIdx.x;
-  if (tile * kCompactTile >= n) return;
-  const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t tile0 = (blockIdx.x * 4u + (threadIdx.x >> 6)) * kBirthTiles;
+  if (tile0 >= (n + kCompactTile - 1u) / kCompactTile) return;
+  const uint32_t mine = lane < kBirthTiles && (tile0 + lane) * kCompactTile < n ? a.tileBirth[tile0 + lane] : 0u;
+  uint64_t some = __ballot(mine != 0u);
+  if (some == 0) return;
+  uint32_t base = 0;
+  for (uint32_t q = lane; q < tile0 / kFinBlockTiles; q += 64) base += a.blockSum[q];
+  base = wave_sum(base);
   const uint64_t lt = lanemask_lt();
-  constexpr int kItems = kCompactTile / 256;  // chunks of 64 per wave
-  constexpr uint32_t kWaveSpan = kCompactTile / 4;  // consecutive elements per wave
-  bool al[kItems], bi[kItems];
-  uint32_t ra[kItems], rb[kItems];
-  float4 pv[kItems];
-  float wv[kItems];
-  int bt[kItems];
-  uint32_t ca = 0, cb = 0;
-  // every load of the survivors' data before the first store (a wait for a
-  // load also waits for the stores issued before it)
-  const uint32_t tileBirths = a.tileBirth[tile];  // births the producer counted here
+  constexpr int kItems = kCompactTile / 64;
+  while (some) {
+    const uint32_t tile = tile0 + (uint32_t)__ffsll((unsigned long long)some) - 1u;
+    some &= some - 1u;
+    uint32_t rank = base + a.tileBirthPre[tile];
+    const uint32_t e0 = tile * kCompactTile;
+    int bt[kItems];
 #pragma unroll
-  for (int it = 0; it < kItems; ++it) {
-    const uint32_t e = tile * kCompactTile + w * kWaveSpan + it * 64 + lane;
-    const bool v = e < n;
-    pv[it] = v ? a.pt[e] : make_float4(0.f, 0.f, 0.f, 0.f);
-    wv[it] = v ? a.w[e] : 0.0f;
-  }
-  // birth types are read only in tiles with births (zero everywhere else)
+    for (int it = 0; it < kItems; ++it) {
+      const uint32_t e = e0 + it * 64 + lane;
+      bt[it] = e < n ? a.birthType[e] : 0;
+    }
+    // replica of the tile's first slot (last r with repOff[r] <= e0); the
+    // lanes move forward from there
+    int r = 0;
+    {
+      int hi = a.R;
+      while (hi - r > 1) {
+        const int mid = (r + hi) >> 1;
+        if (repOff[mid] <= e0) r = mid;
+        else hi = mid;
+      }
+    }
 #pragma unroll
-  for (int it = 0; it < kItems; ++it) {
-    const uint32_t e = tile * kCompactTile + w * kWaveSpan + it * 64 + lane;
-    bt[it] = (tileBirths != 0u && e < n) ? a.birthType[e] : 0;
-  }
-#pragma unroll
-  for (int it = 0; it < kItems; ++it) {
-    const uint32_t e = tile * kCompactTile + w * kWaveSpan + it * 64 + lane;
-    const bool v = e < n;
-    al[it] = v && __float_as_int(pv[it].w) > 0;
-    bi[it] = v && bt[it] > 0;
-    const uint64_t am = __ballot(al[it]);
-    const uint64_t bm = __ballot(bi[it]);
-    ra[it] = ca + (uint32_t)__popcll(am & lt);
-    rb[it] = cb + (uint32_t)__popcll(bm & lt);
-    ca += (uint32_t)__popcll(am);
-    cb += (uint32_t)__popcll(bm);
-  }
-  uint32_t pa = a.tileAlivePre[tile], pb = a.tileBirthPre[tile];
-  // totals of the finalize blocks before this tile's block
-  {
-    const uint32_t g = tile / kFinBlockTiles;
-    uint32_t sa = 0, sb = 0;
-    for (uint32_t q = lane; q < g; q += 64) {
-      sa += a.blockSum[q];
-      sb += a.blockSum[a.blockStride + q];
-    }
-    pa += wave_sum(sa);
-    pb += wave_sum(sb);
-  }
-  if (lane == 0) {
-    s_wa[w] = ca;
-    s_wb[w] = cb;
-  }
-  __syncthreads();
-  for (uint32_t k = 0; k < w; ++k) {
-    pa += s_wa[k];
-    pb += s_wb[k];
-  }
-  // replica of the wave's first element (last r with repOff[r] <= e), by a
-  // wave-uniform search through the scalar cache; each lane's elements only
-  // move forward through the replicas from there
-  int r = 0;
-  {
-    const uint32_t e0 = tile * kCompactTile + w * kWaveSpan;
-    int lo = 0, hi = a.R;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (repOff[mid] <= e0) lo = mid;
-      else hi = mid;
-    }
-    r = lo;
-  }
-  // the replica's offsets in registers, reloaded only when the walk moves on
-  uint32_t nOff = a.newOff[r], aBase = a.aliveBase[r], bBase = a.birthBase[r], rAlive = a.repAlive[r];
-  uint32_t nextOff = r + 1 < a.R ? repOff[r + 1] : 0xFFFFFFFFu;
-#pragma unroll
-  for (int it = 0; it < kItems; ++it) {
-    const uint32_t e = tile * kCompactTile + w * kWaveSpan + it * 64 + lane;
-    if (!(al[it] || bi[it])) continue;
-    while (nextOff <= e) {
-      ++r;
-      nOff = a.newOff[r];
-      aBase = a.aliveBase[r];
-      bBase = a.birthBase[r];
-      rAlive = a.repAlive[r];
-      nextOff = r + 1 < a.R ? repOff[r + 1] : 0xFFFFFFFFu;
-    }
-    if (al[it]) {
-      const uint32_t dst = nOff + (pa + ra[it] - aBase);
-      a.ptOut[dst] = pv[it];
-      a.wOut[dst] = wv[it];
-    }
-    if (bi[it]) {
-      const uint32_t dst = nOff + rAlive + (pb + rb[it] - bBase);
-      const float4 q = a.addedPos[e];
-      a.ptOut[dst] = make_float4(q.x, q.y, q.z, __int_as_float(bt[it]));
-      a.wOut[dst] = q.w;
-      a.birthType[e] = 0;  // taken: zero again for the next step
+    for (int it = 0; it < kItems; ++it) {
+      const uint64_t bm = __ballot(bt[it] > 0);
+      if (bt[it] > 0) {
+        const uint32_t e = e0 + it * 64 + lane;
+        while (r + 1 < a.R && repOff[r + 1] <= e) ++r;
+        const uint32_t dst = a.extraOff[r] + rank + (uint32_t)__popcll(bm & lt) - a.birthBase[r];
+        const float4 q = a.addedPos[e];
+        a.extra[dst] = make_float4(q.x, q.y, q.z, __int_as_float((a.extraW ? 0 : __float_as_int(q.w)) | bt[it]));
+        if (a.extraW) a.extraW[dst] = q.w;
+        a.birthType[e] = 0;  // taken: zero again for the next step
+      }
+      rank += (uint32_t)__popcll(bm);
     }
   }
-  if (threadIdx.x == 0 && tileBirths != 0u) a.tileBirth[tile] = 0;
+  if (mine) a.tileBirth[tile0 + lane] = 0;
+}
+
+// Where particle il of replica r is (CanonMap).
+__device__ __forceinline__ uint32_t canon_index(const CanonMap& m, uint32_t r, uint32_t il) {
+  const uint32_t so = m.srcOff[r], na = m.alive[r];
+  if (il >= na) return m.extraBase + m.extraOff[r] + il - na;
+  return so + il + holes_before(m.holes + m.holeOff[r], m.holeN[r], so, il);
+}
+
+// The replica that holds canonical particle i (last r with repOff[r] <= i).
+__device__ __forceinline__ uint32_t replica_of(const uint32_t* __restrict__ repOff, int R, uint32_t i) {
+  int lo = 0, hi = R;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (repOff[mid] <= i) lo = mid;
+    else hi = mid;
+  }
+  return (uint32_t)lo;
+}
+
+__global__ __launch_bounds__(256) void k_export(ExportArgs a) {
+  const uint32_t k = blockIdx.x * 256 + threadIdx.x;
+  const uint32_t n = a.rep >= 0 ? a.repCount[a.rep] : a.repOff[a.R];
+  if (k == 0 && a.header) *a.header = n;
+  if (k >= a.cap || k + a.begin >= n) return;
+  uint32_t r = (uint32_t)a.rep, il = k + a.begin;
+  if (a.rep < 0) {
+    r = replica_of(a.repOff, a.R, il);
+    il -= a.repOff[r];
+  }
+  const uint32_t src = canon_index(a.map, r, il);
+  const float4 p = a.pt[src];
+  const int word = __float_as_int(p.w);
+  if (a.pos4) a.pos4[k] = make_float4(p.x, p.y, p.z, a.w ? a.w[src] : __int_as_float(word & ~kTypeMask));
+  if (a.types) a.types[k] = word & kTypeMask;
+}
+
+__global__ __launch_bounds__(256) void k_compact(ExportArgs a, float4* __restrict__ out, float* __restrict__ wOut) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.repOff[a.R]) return;
+  const uint32_t r = replica_of(a.repOff, a.R, i);
+  const uint32_t src = canon_index(a.map, r, i - a.repOff[r]);
+  out[i] = a.pt[src];
+  if (wOut) wOut[i] = a.w[src];
+}
+
+__global__ __launch_bounds__(256) void k_identity_map(int R, const uint32_t* __restrict__ repOff,
+                                                      const uint32_t* __restrict__ repCount,
+                                                      uint32_t* __restrict__ srcOff, uint32_t* __restrict__ alive,
+                                                      uint32_t* __restrict__ holeN) {
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r >= R) return;
+  srcOff[r] = repOff[r];
+  alive[r] = repCount[r];
+  holeN[r] = 0u;
+}
+
+__global__ __launch_bounds__(256) void k_split_w(float4* __restrict__ pt, float* __restrict__ w, uint32_t n) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int word = __float_as_int(pt[i].w);
+  w[i] = __int_as_float(word & ~kTypeMask);
+  pt[i].w = __int_as_float(word & kTypeMask);
 }
 
 // ---------------------------------------------------------------------------
@@ -1544,10 +1606,10 @@ __global__ __launch_bounds__(256) void k_inject(InjectArgs a) {
   const uint32_t q = blockIdx.x * 256 + threadIdx.x;
   if (q >= a.nInj) return;
   const int r = a.injRep[q];
-  const uint32_t dst = a.newOff[r] + a.injBase[r] + (q - a.injSrcOff[r]);
+  const uint32_t dst = a.injBase[r] + (q - a.injSrcOff[r]);
   const float4 p = a.injPos[q];
-  a.ptOut[dst] = make_float4(p.x, p.y, p.z, __int_as_float(a.injType[q]));
-  a.wOut[dst] = p.w;
+  a.extra[dst] = make_float4(p.x, p.y, p.z, __int_as_float((a.extraW ? 0 : __float_as_int(p.w)) | a.injType[q]));
+  if (a.extraW) a.extraW[dst] = p.w;
 }
 
 // ---------------------------------------------------------------------------
@@ -1607,27 +1669,17 @@ __global__ __launch_bounds__(64) void k_zero(ZeroArgs a) {
 __global__ __launch_bounds__(64) void k_zero_place(const ReplicaTables* __restrict__ tables,
                                                    const float4* __restrict__ zPos, const int* __restrict__ zType,
                                                    const uint32_t* __restrict__ zCount,
-                                                   const uint32_t* __restrict__ newOff,
-                                                   const uint32_t* __restrict__ zeroBase, float4* __restrict__ ptOut,
-                                                   float* __restrict__ wOut) {
+                                                   const uint32_t* __restrict__ zeroBase, float4* __restrict__ extra,
+                                                   float* __restrict__ extraW) {
   const int r = blockIdx.x;
   const uint32_t c = zCount[r];
   if (c == 0) return;
-  const uint32_t src = tables[r].zeroOff, dst = newOff[r] + zeroBase[r];
+  const uint32_t src = tables[r].zeroOff, dst = zeroBase[r];
   for (uint32_t j = threadIdx.x; j < c; j += 64) {
     const float4 p = zPos[src + j];
-    ptOut[dst + j] = make_float4(p.x, p.y, p.z, __int_as_float(zType[src + j]));
-    wOut[dst + j] = p.w;
+    extra[dst + j] = make_float4(p.x, p.y, p.z, __int_as_float((extraW ? 0 : __float_as_int(p.w)) | zType[src + j]));
+    if (extraW) extraW[dst + j] = p.w;
   }
-}
-
-__global__ __launch_bounds__(256) void k_unpack(const float4* __restrict__ pt, const float* __restrict__ w, uint32_t n,
-                                                float4* __restrict__ pos4, int* __restrict__ type) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const float4 p = pt[i];
-  pos4[i] = make_float4(p.x, p.y, p.z, w[i]);
-  type[i] = __float_as_int(p.w);
 }
 
 __global__ __launch_bounds__(256) void k_mt_init_range(uint32_t* __restrict__ st, const uint32_t* __restrict__ seeds,
@@ -2070,7 +2122,7 @@ __global__ __launch_bounds__(256) void k_seg_down(const uint32_t* __restrict__ k
           // the record carries its particle's index above the type bits
           if (dk[q] < deadKey)
             gatherDst[dd[q]] = make_float4(rec[q].x, rec[q].y, rec[q].z,
-                                           __int_as_float(pack_index_type(dv[q], __float_as_int(rec[q].w))));
+                                           __int_as_float(pack_index_type(dv[q], __float_as_int(rec[q].w) & kTypeMask)));
         } else {
           valsOut[dd[q]] = dv[q];
           if (dk[q] < deadKey) gatherDst[dd[q]] = rec[q];
@@ -2116,12 +2168,16 @@ hipError_t launch_producer(const ProducerArgs& a, int blockSize, hipStream_t str
   // the stream of global id g is g's in every shape: the results do not
   // depend on the block size; one more workgroup for the tile table
   const unsigned extra = a.segTilesOn ? 1u : 0u;
-  if (blockSize == 512)
-    hipLaunchKernelGGL(k_producer<512>, dim3(cdiv(a.Stot, 512) + extra), dim3(512), 0, stream, a, a.tables);
-  else if (blockSize == 128)
-    hipLaunchKernelGGL(k_producer<128>, dim3(cdiv(a.Stot, 128) + extra), dim3(128), 0, stream, a, a.tables);
-  else
-    hipLaunchKernelGGL(k_producer<256>, dim3(cdiv(a.Stot, 256) + extra), dim3(256), 0, stream, a, a.tables);
+#define SMD_PRODUCER(BS)                                                                                          \
+  {                                                                                                               \
+    const dim3 grid(cdiv(a.Stot, BS) + extra), blk(BS);                                                           \
+    if (a.w) hipLaunchKernelGGL((k_producer<BS, true>), grid, blk, 0, stream, a, a.tables);                       \
+    else hipLaunchKernelGGL((k_producer<BS, false>), grid, blk, 0, stream, a, a.tables);                          \
+  }
+  if (blockSize == 512) SMD_PRODUCER(512)
+  else if (blockSize == 128) SMD_PRODUCER(128)
+  else SMD_PRODUCER(256)
+#undef SMD_PRODUCER
   return hipGetLastError();
 }
 
@@ -2467,16 +2523,45 @@ hipError_t launch_resolve(const ResolveArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-uint32_t finalize_blocks(uint32_t maxN) {
-  return std::max<uint32_t>(1u, cdiv(cdiv(maxN, kCompactTile), kFinBlockTiles));
+uint32_t finalize_blocks(uint32_t capacity) {
+  return std::max<uint32_t>(1u, cdiv(cdiv(capacity, kCompactTile), kFinBlockTiles));
 }
 
-hipError_t launch_finalize(const FinalizeArgs& args, uint32_t maxN, hipStream_t stream) {
-  const uint32_t g = finalize_blocks(maxN);
-  if (g > args.blockStride) return hipErrorInvalidValue;
-  FinalizeArgs a = args;
-  a.maxTiles = cdiv(maxN, kCompactTile);
-  hipLaunchKernelGGL(k_finalize, dim3(g), dim3(1024), 0, stream, a);
+hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t stream) {
+  // over all tiles of the capacity: the other parity's counts are cleared
+  hipLaunchKernelGGL(k_finalize, dim3(std::max(1u, cdiv(a.tilesCap, kFinBlockTiles))), dim3(1024), 0, stream, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_births(const BirthArgs& a, uint32_t maxN, hipStream_t stream) {
+  if (maxN == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_births, dim3(cdiv(cdiv(maxN, kCompactTile), 4 * kBirthTiles)), dim3(256), 0, stream, a,
+                     a.repOff);
+  return hipGetLastError();
+}
+
+hipError_t launch_export(const ExportArgs& a, uint32_t maxN, hipStream_t stream) {
+  hipLaunchKernelGGL(k_export, dim3(std::max(1u, cdiv(maxN, 256))), dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_compact(const ExportArgs& a, uint32_t maxN, float4* out, float* wOut, hipStream_t stream) {
+  if (maxN == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_compact, dim3(cdiv(maxN, 256)), dim3(256), 0, stream, a, out, wOut);
+  return hipGetLastError();
+}
+
+hipError_t launch_identity_map(int R, const uint32_t* repOff, const uint32_t* repCount, uint32_t* srcOff,
+                               uint32_t* alive, uint32_t* holeN, hipStream_t stream) {
+  if (R <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_identity_map, dim3(cdiv(R, 256)), dim3(256), 0, stream, R, repOff, repCount, srcOff, alive,
+                     holeN);
+  return hipGetLastError();
+}
+
+hipError_t launch_split_w(float4* pt, float* w, uint32_t n, hipStream_t stream) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_split_w, dim3(cdiv(n, 256)), dim3(256), 0, stream, pt, w, n);
   return hipGetLastError();
 }
 
@@ -2493,17 +2578,10 @@ hipError_t launch_zero(const ZeroArgs& a, hipStream_t stream) {
 }
 
 hipError_t launch_zero_place(int R, const ReplicaTables* tables, const float4* zPos, const int* zType,
-                             const uint32_t* zCount, const uint32_t* newOff, const uint32_t* zeroBase, float4* ptOut,
-                             float* wOut, hipStream_t stream) {
+                             const uint32_t* zCount, const uint32_t* zeroBase, float4* extra, float* extraW,
+                             hipStream_t stream) {
   if (R <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_zero_place, dim3(R), dim3(64), 0, stream, tables, zPos, zType, zCount, newOff, zeroBase,
-                     ptOut, wOut);
-  return hipGetLastError();
-}
-
-hipError_t launch_unpack(const float4* pt, const float* w, uint32_t n, float4* pos4, int* type, hipStream_t stream) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_unpack, dim3(cdiv(n, 256)), dim3(256), 0, stream, pt, w, n, pos4, type);
+  hipLaunchKernelGGL(k_zero_place, dim3(R), dim3(64), 0, stream, tables, zPos, zType, zCount, zeroBase, extra, extraW);
   return hipGetLastError();
 }
 
@@ -2511,13 +2589,6 @@ hipError_t launch_mt_init_range(uint32_t* st, const uint32_t* seeds, uint32_t St
                                 hipStream_t stream) {
   if (count == 0) return hipSuccess;
   hipLaunchKernelGGL(k_mt_init_range, dim3(cdiv(count, 256)), dim3(256), 0, stream, st, seeds, Stot, off, count);
-  return hipGetLastError();
-}
-
-
-hipError_t launch_scatter(const ScatterArgs& a, uint32_t maxN, hipStream_t stream) {
-  if (maxN == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_scatter, dim3(cdiv(maxN, kCompactTile)), dim3(256), 0, stream, a, a.repOff);
   return hipGetLastError();
 }
 

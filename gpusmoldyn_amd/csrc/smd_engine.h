@@ -59,7 +59,10 @@ class Engine {
   int* dBucketRep = nullptr;  // replica of each 2^repShift-bucket chunk (nullptr: search bucketStart)
   uint32_t repShift = 0;
   uint32_t *dRepOff = nullptr, *dRepCount = nullptr, *dNewOff = nullptr, *dNewCount = nullptr;
-  uint32_t *dAliveBase = nullptr, *dBirthBase = nullptr, *dRepAlive = nullptr;
+  // where the particles entering the next step are (CanonMap; dNewOff holds
+  // the slots' replica offsets)
+  uint32_t *dAlive = nullptr, *dHoleOff = nullptr, *dHoleN = nullptr, *dExtraOff = nullptr, *dHoles = nullptr;
+  uint32_t* dBirthBase = nullptr;
   uint32_t *dRepDeaths = nullptr, *dRepBirths = nullptr;
   uint32_t* dCounters = nullptr;
   unsigned long long* dParticleSteps = nullptr;  // running sum of particles entering each step
@@ -67,10 +70,14 @@ class Engine {
   uint32_t *dMtState = nullptr, *dMtPar = nullptr;
   float* dGauss = nullptr;
   uint32_t* dFirst = nullptr;
-  // canonical particle state, ping-ponged by the compaction: (x, y, z, type
-  // bits) and the fourth position component
+  // canonical particle state: the producer reads one buffer through the map
+  // and writes the other densely.  Records (x, y, z, type and fourth
+  // component); the fourth components apart (dW) only when they do not pack.
+  // Each buffer holds cap slots, then extraCap for the particles a step gains.
   float4* dPT[2] = {nullptr, nullptr};
   float* dW[2] = {nullptr, nullptr};
+  bool wApart = false;
+  uint32_t extraCap = 0;
   float4* dAddedPos = nullptr;
   int* dBirthType = nullptr;
   float4* dSortedPT = nullptr;
@@ -79,10 +86,13 @@ class Engine {
   int* dViewType = nullptr;
   uint32_t viewCap = 0;
   SortBuffers sb = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, nullptr, nullptr, 0, 0};
-  uint32_t *dTileAlive = nullptr, *dTileBirth = nullptr, *dTileAlivePre = nullptr, *dTileBirthPre = nullptr;
-  uint32_t* dBlockSum = nullptr;  // finalize block totals, [2][blockStride]
-  uint32_t blockStride = 0;
-  uint32_t* dStatus = nullptr;  // sticky kernel error bits
+  uint32_t* dDeadBits = nullptr;                // a bit per slot removed in this step
+  uint32_t* dTileDead[2] = {nullptr, nullptr};  // removed per tile, one per step parity (cur)
+  uint32_t *dTileBirth = nullptr, *dTileBirthPre = nullptr;
+  uint32_t* dBlockSum = nullptr;  // births per finalize block
+  uint32_t* dStatus = nullptr;    // sticky kernel error bits
+  uint32_t* hostStatus = nullptr;   // their copy in host memory, written by the finalize kernel
+  uint32_t* dHostStatus = nullptr;  // its device address
   // order-0 creation: one stream per replica, a per-step creation buffer
   uint32_t *dZMt = nullptr, *dZPar = nullptr, *dZCount = nullptr, *dZeroBase = nullptr;
   float4* dZPos = nullptr;
@@ -151,6 +161,13 @@ class Engine {
   hipError_t sort_keys(uint32_t maxN, bool tilesLaid, StageTimer* timer, bool debug);
   smd_status step_graph(int pairs);
   smd_status alloc_particle_buffers(uint32_t c);
+  smd_status alloc_apart();
+  smd_status take_apart(const float* pos4, size_t n);
+  CanonMap canon_map() const;
+  ProducerArgs producer_args() const;
+  ExportArgs export_args(int r) const;
+  smd_status set_dense();
+  smd_status view_buffers(uint32_t n);
   void free_particle_buffers();
   void refresh_bound(bool block);
   smd_status grow(uint64_t need);

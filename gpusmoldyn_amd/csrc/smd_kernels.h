@@ -25,6 +25,27 @@ struct SegTilesArgs {
   uint32_t* status;
 };
 
+// Where the particles that enter a step are.  The step that wrote them left
+// removed ones in place: replica r's survivors are the slots from srcOff[r]
+// on, in order, except the holes [holeOff[r], holeOff[r] + holeN[r]) of the
+// sorted hole list; behind its alive[r] survivors come the particles it
+// gained, at extraBase + extraOff[r] of the same array.
+struct CanonMap {
+  const uint32_t* srcOff;
+  const uint32_t* alive;
+  const uint32_t* holeOff;
+  const uint32_t* holeN;
+  const uint32_t* holes;
+  const uint32_t* extraOff;
+  uint32_t extraBase;
+};
+
+// Particles removed in a step: a bit per slot and a count per tile.
+struct DeathMarks {
+  uint32_t* bits;
+  uint32_t* tileDead;
+};
+
 struct ProducerArgs {
   const ReplicaTables* tables;
   const int* streamReplica;   // per global stream: replica id (padding lanes of a replica included), -1 none
@@ -34,15 +55,18 @@ struct ProducerArgs {
   const uint32_t* mtPar;      // [3][Stot]
   uint32_t Stot;
   const float* gauss;         // entries 1 to 2048 of the 4096-entry table (gauss_entry)
-  float4* pt;                 // canonical (x, y, z, type bits), updated in place; also the pair-search source
-  float* w;                   // canonical fourth position component (set to 0 for offset products)
+  const float4* ptIn;         // canonical records entering the step, through map
+  CanonMap map;
+  float4* pt;                 // canonical records of the step, dense; also the pair-search source
+  const float* wIn;           // fourth position components, as ptIn and pt (nullptr: in the records)
+  float* w;
   float4* addedPos;
   int* birthType;
   uint32_t* key;
   uint32_t deadKey;
   uint32_t* repDeaths;
   uint32_t* repBirths;
-  uint32_t* tileAlive;
+  DeathMarks deaths;
   uint32_t* tileBirth;
   const uint32_t* retire;     // per replica: remove every particle this step (nullptr: none)
   // 1: one extra workgroup of the launch lays out the segmented sort's tiles
@@ -157,9 +181,9 @@ struct ResolveArgs {
   const uint32_t* vals;
   int packed;  // sortedPT carries the particles' indices (vals unused)
   float4* pt;
-  float* w;
+  float* w;  // nullptr: in the records
   uint32_t* repDeaths;
-  uint32_t* tileAlive;
+  DeathMarks deaths;
 };
 
 struct FinalizeArgs {
@@ -169,27 +193,32 @@ struct FinalizeArgs {
   uint32_t* repBirths;
   uint32_t* newOff;     // [R+1]
   uint32_t* newCount;
-  uint32_t* aliveBase;
-  uint32_t* birthBase;
-  uint32_t* repAlive;
+  // the map of the next step (CanonMap) and where the gained particles go
+  uint32_t* alive;
+  uint32_t* holeOff;
+  uint32_t* holeN;
+  uint32_t* holes;
+  uint32_t* extraOff;
+  uint32_t* birthBase;  // births of earlier replicas
   uint32_t* dNnext;
   const uint32_t* dN;
-  uint32_t* tileAlive;
-  uint32_t* tileBirth;
-  uint32_t* tileAlivePre;
+  DeathMarks deaths;    // the bits are cleared here
+  uint32_t* tileDeadNext;  // the other step parity's counts: cleared here
+  uint32_t* tileBirth;     // nullptr: no particle can be born
   uint32_t* tileBirthPre;
   unsigned long long* particleSteps;  // += particles entering the step
   uint32_t* stepCount;                // steps completed (incremented here)
   unsigned long long* countRing;      // host-visible: slot (steps & ringMask) = steps << 32 | particles
   uint32_t ringMask;
+  const uint32_t* status;  // sticky error bits, and their host-visible copy
+  uint32_t* hostStatus;
   const uint32_t* zCount;  // per replica: particles created this step (nullptr: none)
-  uint32_t* zeroBase;      // per replica: alive + births, where created particles go
+  uint32_t* zeroBase;      // per replica: where its created particles go (from extraBase)
   uint32_t* injCount;      // per replica: particles admitted this step (nullptr: none); reset
-  uint32_t* injBase;       // per replica: alive + births + created, where admitted particles go
+  uint32_t* injBase;       // per replica: where its admitted particles go (from extraBase)
   uint32_t* retire;        // per replica retire flags (nullptr: none); reset
-  uint32_t* blockSum;      // [2][blockStride]: alive and birth totals of each 1024-tile block
-  uint32_t blockStride;    // at least finalize_blocks(maxN)
-  uint32_t maxTiles;       // compaction tiles of the launch bound (set by launch_finalize)
+  uint32_t* blockSum;      // births of each 1024-tile block
+  uint32_t tilesCap;       // tiles of the allocated capacity
 };
 
 struct ZeroArgs {
@@ -209,31 +238,41 @@ struct InjectArgs {
   const int* injRep;          // replica of each admitted particle
   const uint32_t* injSrcOff;  // first admitted particle of each replica
   uint32_t nInj;
-  const uint32_t* newOff;
   const uint32_t* injBase;
-  float4* ptOut;
-  float* wOut;
+  float4* extra;   // gained particles' records and fourth components (nullptr: in the records)
+  float* extraW;
 };
 
-struct ScatterArgs {
+// Births of a step, in parent order behind their replica's survivors.
+struct BirthArgs {
   int R;
   const uint32_t* dN;
   const uint32_t* repOff;
-  const uint32_t* newOff;
-  const uint32_t* aliveBase;
   const uint32_t* birthBase;
-  const uint32_t* repAlive;
-  const uint32_t* tileAlivePre;
+  const uint32_t* extraOff;
   const uint32_t* tileBirthPre;
-  const float4* pt;
-  const float* w;
   const float4* addedPos;
   int* birthType;          // nonzero only at births; cleared as they are taken
-  uint32_t* tileBirth;     // births per compaction tile (producer); cleared here
-  float4* ptOut;
-  float* wOut;
-  const uint32_t* blockSum;  // the finalize blocks' totals (FinalizeArgs::blockSum)
-  uint32_t blockStride;
+  uint32_t* tileBirth;     // births per tile (producer); cleared here
+  const uint32_t* blockSum;
+  float4* extra;
+  float* extraW;           // nullptr: in the records
+};
+
+// Reads replica rep's canonical particles (all replicas, as one array, when
+// rep < 0) through the map into pos4 / types (either may be nullptr); header
+// gets the particle count and the status bits.
+struct ExportArgs {
+  const float4* pt;
+  const float* w;  // nullptr: in the records
+  CanonMap map;
+  const uint32_t* repOff;    // [R+1]
+  const uint32_t* repCount;
+  int R, rep;
+  uint32_t begin, cap;       // particles [begin, begin + cap) of the replica
+  float4* pos4;
+  int* types;
+  uint32_t* header;          // nullptr: none
 };
 
 hipError_t launch_mt_init(uint32_t* st, const uint32_t* seeds, uint32_t S, hipStream_t stream);
@@ -282,19 +321,24 @@ hipError_t launch_gather(const uint32_t* keys, const uint32_t* vals, const float
 // blockSize: 64, 128 or 256 threads (identical results)
 hipError_t launch_candidates(const CandArgs& a, uint32_t maxN, int blockSize, hipStream_t stream);
 hipError_t launch_resolve(const ResolveArgs& a, hipStream_t stream);
-// Finalize workgroups for a step of at most maxN particles (one per 4096
-// compaction tiles).
-uint32_t finalize_blocks(uint32_t maxN);
-hipError_t launch_finalize(const FinalizeArgs& a, uint32_t maxN, hipStream_t stream);
-hipError_t launch_scatter(const ScatterArgs& a, uint32_t maxN, hipStream_t stream);
+// Finalize workgroups for a capacity (one per 1024 tiles).
+uint32_t finalize_blocks(uint32_t capacity);
+hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t stream);
+hipError_t launch_births(const BirthArgs& a, uint32_t maxN, hipStream_t stream);
+hipError_t launch_export(const ExportArgs& a, uint32_t maxN, hipStream_t stream);
+// Dense copy of the canonical records (and fourth components) through the
+// map, and the map of dense records.
+hipError_t launch_compact(const ExportArgs& a, uint32_t maxN, float4* out, float* wOut, hipStream_t stream);
+hipError_t launch_identity_map(int R, const uint32_t* repOff, const uint32_t* repCount, uint32_t* srcOff,
+                               uint32_t* alive, uint32_t* holeN, hipStream_t stream);
+// Moves the fourth components out of n records into w.
+hipError_t launch_split_w(float4* pt, float* w, uint32_t n, hipStream_t stream);
 hipError_t launch_inject(const InjectArgs& a, hipStream_t stream);
 hipError_t launch_zero(const ZeroArgs& a, hipStream_t stream);
-// Appends replica r's created particles after its survivors and births.
+// Replica r's created particles, behind its survivors and births.
 hipError_t launch_zero_place(int R, const ReplicaTables* tables, const float4* zPos, const int* zType,
-                             const uint32_t* zCount, const uint32_t* newOff, const uint32_t* zeroBase, float4* ptOut,
-                             float* wOut, hipStream_t stream);
-// pos4[i] = (pt[i].xyz, w[i]), type[i] = type bits of pt[i], i < n.
-hipError_t launch_unpack(const float4* pt, const float* w, uint32_t n, float4* pos4, int* type, hipStream_t stream);
+                             const uint32_t* zCount, const uint32_t* zeroBase, float4* extra, float* extraW,
+                             hipStream_t stream);
 hipError_t launch_mt_init_range(uint32_t* st, const uint32_t* seeds, uint32_t Stot, uint32_t off, uint32_t count,
                                 hipStream_t stream);
 

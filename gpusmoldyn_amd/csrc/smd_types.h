@@ -15,7 +15,11 @@ constexpr int kMtMM = 9;         // middle word offset (MersenneTwister.cuh:29)
 constexpr int kMtWords = 20;     // 19 state words + iState, stored word-major (SoA)
 constexpr int kMtParamSets = 32768;  // records in MersenneTwister.dat (MersenneTwister.h:31)
 constexpr int kGaussDim = 4096;  // particles_kernel.cuh:43
-constexpr int kCompactTile = 1024;   // elements per compaction tile (4 waves x 4 chunks of 64)
+constexpr int kCompactTile = 1024;   // particle slots per tile of the death and birth counters
+// The fourth word of a canonical record holds the particle's type in its low
+// kIndexShift bits and, above them, the bits of its fourth position component
+// where every particle's component has zeros there (1.0, 0.0 and the like);
+// otherwise the components live in arrays of their own and these bits are 0.
 // Sorted particle records may carry the particle's index above its type:
 // w bits = index << kIndexShift | type (types stay below 2^kIndexShift), for
 // indices below kMaxPackedIndex.
