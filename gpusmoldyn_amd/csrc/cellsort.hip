@@ -45,7 +45,7 @@ constexpr uint32_t kIndexMask = (1u << kIndexBits) - 1u;
 constexpr int kLow = 7, kHigh = kCellSliceBits - kLow;  // digits of the ordered path's passes over the list
 // Cells of at most this many particles are put in order by comparing
 // neighbours in the list; a fuller one sends the slice to the ordered path.
-constexpr uint32_t kFew = 20;
+constexpr uint32_t kFew = 32;
 
 struct CsLds {
   uint32_t hist[kCellSlice];               // counts per cell, then where each cell's next particle goes

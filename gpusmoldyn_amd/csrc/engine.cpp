@@ -129,6 +129,7 @@ void Engine::free_particle_buffers() {
   dfree(dBirthType);
   dfree(dSortedPT);
   dfree(dCand);
+  dfree(dCandList);
   dfree(dViewPos);
   dfree(dViewType);
   viewCap = 0;
@@ -184,6 +185,8 @@ smd_status Engine::alloc_particle_buffers(uint32_t c) {
   HIPCHK(dalloc(&dBirthType, cap));
   HIPCHK(dalloc(&dSortedPT, cap));
   HIPCHK(dalloc(&dCand, cap));
+  HIPCHK(hipMemsetAsync(dCand, 0, (size_t)cap * sizeof(uint2), stream));  // tag 0: no step's
+  HIPCHK(dalloc(&dCandList, pair_list_size()));
   // the cell sort reads keys as whole vectors of four
   HIPCHK(dalloc(&sb.keys, (size_t)cap + 4));
   HIPCHK(dalloc(&sb.vals, cap));
@@ -361,6 +364,7 @@ smd_status Engine::finalize(uint32_t capacity) {
   HIPCHK(hipMemset(dRepDeaths, 0, R * sizeof(uint32_t)));
   HIPCHK(hipMemset(dRepBirths, 0, R * sizeof(uint32_t)));
   HIPCHK(dalloc(&dCounters, 8));
+  HIPCHK(hipMemset(dCounters, 0, 8 * sizeof(uint32_t)));
   HIPCHK(dalloc(&dParticleSteps, 1));
   HIPCHK(hipMemset(dParticleSteps, 0, sizeof(unsigned long long)));
   dN = dCounters;
@@ -821,6 +825,40 @@ ProducerArgs Engine::producer_args() const {
   return pa;
 }
 
+CandArgs Engine::cand_args() const {
+  CandArgs a;
+  a.tables = dTables;
+  a.bucketStart = dBucketStart;
+  a.bucketRep = dBucketRep;
+  a.repShift = repShift;
+  a.R = (int)R;
+  a.keys = sb.keys;
+  a.sortedPT = dSortedPT;
+  a.first = dFirst;
+  a.dLive = dLive;
+  a.cand = CandList{dCand, dCandList, dCounters + 3, dCounters + 4, dStepCount};
+  return a;
+}
+
+ResolveArgs Engine::resolve_args() const {
+  ResolveArgs a;
+  a.tables = dTables;
+  a.streamReplica = dStreamReplica;
+  a.mtState = dMtState;
+  a.mtPar = dMtPar;
+  a.Stot = Stot;
+  a.first = dFirst;
+  a.cand = CandList{dCand, dCandList, dCounters + 3, dCounters + 4, dStepCount};
+  a.sortedPT = dSortedPT;
+  a.vals = sb.vals;
+  a.packed = sb.packIndex;
+  a.pt = dPT[cur ^ 1];
+  a.w = dW[cur ^ 1];
+  a.repDeaths = dRepDeaths;
+  a.deaths = DeathMarks{dDeadBits, dTileDead[cur]};
+  return a;
+}
+
 smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
   auto mark = [&](int stage) {
     if (timer) (void)hipEventRecord(timer->ev[stage], stream);
@@ -858,35 +896,9 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
     sb.packIndex = (sb.algo == 1 && cap <= kMaxPackedIndex) ? 1 : 0;
     HIPCHK(sort_keys(maxN, tilesLaid, timer, false));
     mark(3);
-    CandArgs ca;
-    ca.tables = dTables;
-    ca.bucketStart = dBucketStart;
-    ca.bucketRep = dBucketRep;
-    ca.repShift = repShift;
-    ca.R = (int)R;
-    ca.keys = sb.keys;
-    ca.sortedPT = dSortedPT;
-    ca.first = dFirst;
-    ca.dLive = dLive;
-    ca.cand = dCand;
-    HIPCHK(launch_candidates(ca, maxN, pairBlock, stream));
+    HIPCHK(launch_candidates(cand_args(), maxN, pairBlock, stream));
     mark(4);
-    ResolveArgs ra;
-    ra.tables = dTables;
-    ra.streamReplica = dStreamReplica;
-    ra.mtState = dMtState;
-    ra.mtPar = dMtPar;
-    ra.Stot = Stot;
-    ra.first = dFirst;
-    ra.cand = dCand;
-    ra.sortedPT = dSortedPT;
-    ra.vals = sb.vals;
-    ra.packed = sb.packIndex;
-    ra.pt = dPT[cur ^ 1];
-    ra.w = dW[cur ^ 1];
-    ra.repDeaths = dRepDeaths;
-    ra.deaths = pa.deaths;
-    HIPCHK(launch_resolve(ra, stream));
+    HIPCHK(launch_resolve(resolve_args(), stream));
     mark(5);
   } else {
     for (int s = 2; s <= 5; ++s) mark(s);
@@ -910,6 +922,8 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
   fa.tileDeadNext = dTileDead[cur ^ 1];
   fa.tileBirth = anySplit ? dTileBirth : nullptr;
   fa.tileBirthPre = dTileBirthPre;
+  fa.candCount = anyBim ? dCounters + 3 : nullptr;
+  fa.candActing = dCounters + 4;
   fa.particleSteps = dParticleSteps;
   fa.stepCount = dStepCount;
   fa.countRing = dCountRing;
@@ -1378,37 +1392,9 @@ smd_status Engine::debug_stage(int stage, float* pos4, int* types, uint32_t* key
     HIPCHK(sort_keys(maxN, false, nullptr, true));
   }
   if (stage >= 3) {
-    CandArgs ca;
-    ca.tables = dTables;
-    ca.bucketStart = dBucketStart;
-    ca.bucketRep = dBucketRep;
-    ca.repShift = repShift;
-    ca.R = (int)R;
-    ca.keys = sb.keys;
-    ca.sortedPT = dSortedPT;
-    ca.first = dFirst;
-    ca.dLive = dLive;
-    ca.cand = dCand;
-    HIPCHK(launch_candidates(ca, maxN, pairBlock, stream));
+    HIPCHK(launch_candidates(cand_args(), maxN, pairBlock, stream));
   }
-  if (stage >= 4) {
-    ResolveArgs ra;
-    ra.tables = dTables;
-    ra.streamReplica = dStreamReplica;
-    ra.mtState = dMtState;
-    ra.mtPar = dMtPar;
-    ra.Stot = Stot;
-    ra.first = dFirst;
-    ra.cand = dCand;
-    ra.sortedPT = dSortedPT;
-    ra.vals = sb.vals;
-    ra.packed = 0;
-    ra.pt = dPT[cur ^ 1];
-    ra.w = dW[cur ^ 1];
-    ra.repDeaths = dRepDeaths;
-    ra.deaths = pa.deaths;
-    HIPCHK(launch_resolve(ra, stream));
-  }
+  if (stage >= 4) HIPCHK(launch_resolve(resolve_args(), stream));
   HIPCHK(hipStreamSynchronize(stream));
   if (stage >= 2) HIPCHK(hipMemcpy(&live, dLive, sizeof(uint32_t), hipMemcpyDeviceToHost));
   if (nTotal) *nTotal = n;
@@ -1441,7 +1427,13 @@ smd_status Engine::debug_stage(int stage, float* pos4, int* types, uint32_t* key
       HIPCHK(hipMemcpy(keysSorted, sb.keys, n * sizeof(uint32_t), hipMemcpyDeviceToHost));
     if (stage >= 2 && valsSorted)
       HIPCHK(hipMemcpy(valsSorted, sb.vals, n * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    if (stage >= 3 && cand && live) HIPCHK(hipMemcpy(cand, dCand, live * sizeof(int), hipMemcpyDeviceToHost));
+    if (stage >= 3 && cand && live) {
+      std::vector<uint2> cd(live);
+      uint32_t steps = 0;
+      HIPCHK(hipMemcpy(cd.data(), dCand, live * sizeof(uint2), hipMemcpyDeviceToHost));
+      HIPCHK(hipMemcpy(&steps, dStepCount, sizeof(uint32_t), hipMemcpyDeviceToHost));
+      for (uint32_t j = 0; j < live; ++j) cand[j] = cd[j].y == steps + 1u ? (int)cd[j].x : -1;
+    }
   }
   return SMD_OK;
 }

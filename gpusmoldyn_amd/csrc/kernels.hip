@@ -963,6 +963,9 @@ __global__ __launch_bounds__(256) void k_gather(const uint32_t* __restrict__ key
   sortedPT[j] = src[vals[j]];
 }
 
+// Possible pairs up to which the pair step works on their list (k_resolve).
+constexpr uint32_t kPairList = 1024;
+
 // ---------------------------------------------------------------------------
 // Candidate search (collideD/collideCell, particles_kernel.cu:316-411,
 // :443-497): for each live sorted particle j, the nearest particle k != j in
@@ -1190,6 +1193,10 @@ __global__ __launch_bounds__(BS) void k_candidates(CandArgs a, const uint32_t* _
                                                    const int* __restrict__ bucketRep,
                                                    const ReplicaTables* __restrict__ tables) {
   const uint32_t nLive = *a.dLive;
+  const uint32_t tag = *a.cand.stepCount + 1u;
+  // whether this step keeps a list (a count that passes the limit meanwhile
+  // may end it early: the pair step sees that count too)
+  const bool listed = *a.cand.count <= kPairList;
   const uint32_t nBlocks = (nLive + BS - 1u) / BS;
   if (blockIdx.x >= nBlocks) return;
   // neighbouring blocks on one XCD: the cells they both search share its L2
@@ -1213,108 +1220,199 @@ __global__ __launch_bounds__(BS) void k_candidates(CandArgs a, const uint32_t* _
     wave_search(tables[rw], a, j, wbase, lane, active, key, p, best, true);  // one replica: scalar table loads
   else
     wave_search(tables[r], a, j, wbase, lane, active, key, p, best, false);
-  if (active) a.cand[j] = best;
+  // few particles have a partner: those write their candidate, the lower one
+  // of a possible pair also enters the list
+  if (best >= 0) a.cand.cand[j] = make_uint2((uint32_t)best, tag);
+  if (!listed) return;
+  const uint64_t lower = __ballot(best > (int)j);
+  if (lower != 0) {
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(a.cand.count, (uint32_t)__popcll(lower));
+    at = __builtin_amdgcn_readfirstlane(at) + lanes_below(lower);
+    if (best > (int)j && at < kPairList) {
+      const ReplicaTables& T = tables[r];
+      a.cand.list[at] = make_uint4(j, (uint32_t)best, T.streamOff + (j - a.first[T.bucketOff]) % T.numStreams,
+                                   (uint32_t)r);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
-// Resolve: thread g owns stream g and walks the sorted particles
-// j = s, s + S, ... of its replica.  A pair (j, c) reacts when each is the
-// other's candidate; the lower sorted index j draws (coin for prob < 1, then
-// theta, phi, chi) and performs bimReact (reaction_kernel.cuh:202-258),
-// writing products into the unsorted arrays at the original indices.
-// Stream state is loaded only by threads that actually draw.
+// Resolve: a pair (j, c) reacts when each is the other's candidate; the lower
+// sorted index j draws (coin for prob < 1, then theta, phi, chi) from stream
+// (j - first particle of the replica) mod S and performs bimReact
+// (reaction_kernel.cuh:202-258), writing products into the unsorted arrays at
+// the original indices.  Draws of one stream happen in increasing j.
+//
+// Usually a few particles of millions have a candidate: a few workgroups then
+// work on the list of possible pairs, the thread of an acting pair first
+// making sure that its stream has no earlier one (later ones of the stream it
+// performs too).  With more than kPairList possible pairs, thread g walks the
+// sorted particles j = s, s + S, ... of stream g, 8 bytes per particle.
+// Bound by the chain of loads (count, list, partner's candidate, records and
+// tables, stream state).
 // ---------------------------------------------------------------------------
+constexpr uint32_t kPairWgs = 64;     // workgroups that share a list (by stream)
+constexpr uint32_t kPairGrid = 1024;  // workgroups of the launch, for the walk
+
 __global__ __launch_bounds__(kBS) void k_resolve(ResolveArgs a, const ReplicaTables* __restrict__ tables) {
   __shared__ uint32_t lds_mt[kMtNN * kBS];
-  const uint32_t g = blockIdx.x * kBS + threadIdx.x;
-  if (g >= a.Stot) return;
-  // a wave never spans two replicas (stream ranges are 64-aligned), so the
-  // table fields load through the scalar cache
-  const int r = __builtin_amdgcn_readfirstlane(a.streamReplica[g]);
-  if (r < 0) return;
-  const ReplicaTables& T = tables[r];
-  if (!T.hasBim) return;
-  const uint32_t S = T.numStreams;
-  const uint32_t s = g - T.streamOff;
-  if (s >= S) return;
-  const uint32_t lo = a.first[T.bucketOff];
-  const uint32_t hi = a.first[T.bucketOff + T.numBuckets];
+  __shared__ uint4 s_pair[kPairList];  // acting pairs of this workgroup's streams, as listed
+  __shared__ uint32_t s_n;
+  const uint32_t L = *a.cand.count;
+  if (L == 0) return;
+  const uint32_t tag = *a.cand.stepCount + 1u;
   Mt m;
-  bool loaded = false;
-  uint32_t deaths = 0;
-  // candidates of eight consecutive particles of the stream are loaded
-  // together; the particles are still handled in increasing j
-  constexpr int kAhead = 8;
-  int cq[kAhead];
-  for (uint32_t j0 = lo + s; j0 < hi; j0 += kAhead * S) {
+
+  // performs the pair (j, c) of replica r; returns its deaths
+  auto react = [&](const ReplicaTables& T, uint32_t j, uint32_t c) __attribute__((always_inline)) -> uint32_t {
+    const float4 p1 = a.sortedPT[j];
+    const float4 p2 = a.sortedPT[c];
+    const int t1 = __float_as_int(p1.w) & kTypeMask, t2 = __float_as_int(p2.w) & kTypeMask;
+    const int rx = T.pairRxn[t1 * kMaxTypes + t2];
+    const float pr = T.prob[rx];
+    if (!(pr == 1.0f || rand_real(mt_draw<kBS>(m)) < pr)) return 0u;
+    const float dc1 = T.D[t1], dc2 = T.D[t2];
+    const float x = (dc1 == 0.0f && dc2 == 0.0f) ? 0.5f : dc2 / (dc1 + dc2);
+    // pos2 taken at its image nearest pos1 on periodic axes
+    const float q0 = nearest_image(p1.x, p2.x, T, 0);
+    const float q1 = nearest_image(p1.y, p2.y, T, 1);
+    const float q2 = nearest_image(p1.z, p2.z, T, 2);
+    const float omx = 1.0f - x;
+    float rp[3] = {fmaf(x, p1.x, omx * q0), fmaf(x, p1.y, omx * q1), fmaf(x, p1.z, omx * q2)};
+    const float th = smd_theta(rand_real(mt_draw<kBS>(m)));
+    const float ph = rand_real(mt_draw<kBS>(m)) * 6.28318548f;
+    const float ch = rand_real(mt_draw<kBS>(m)) * 6.28318548f;
+    float v1[3], v2[3];
+    rotate_offsets(th, ph, ch, T.prodPos[rx], v1, v2);
+    const uint32_t mol1 = a.packed ? unpack_index(p1.w) : a.vals[j];
+    const uint32_t mol2 = a.packed ? unpack_index(p2.w) : a.vals[c];
+    float n1[3] = {rp[0] + v1[0], rp[1] + v1[1], rp[2] + v1[2]};
+    float n2[3] = {rp[0] + v2[0], rp[1] + v2[1], rp[2] + v2[2]};
 #pragma unroll
-    for (int q = 0; q < kAhead; ++q) {
-      const uint32_t jq = j0 + (uint32_t)q * S;
-      cq[q] = jq < hi ? a.cand[jq] : -1;
-    }
-#pragma unroll
-    for (int q = 0; q < kAhead; ++q) {
-      const uint32_t j = j0 + (uint32_t)q * S;
-      const int c = cq[q];
-      if (c <= (int)j) continue;
-      if (a.cand[c] != (int)j) continue;
-      const float4 p1 = a.sortedPT[j];
-      const float4 p2 = a.sortedPT[c];
-      const int t1 = __float_as_int(p1.w) & kTypeMask, t2 = __float_as_int(p2.w) & kTypeMask;
-      const int rx = T.pairRxn[t1 * kMaxTypes + t2];
-      if (!loaded) {
-        mt_load<kBS>(m, &lds_mt[threadIdx.x], a.mtState, a.mtPar, a.Stot, g);
-        loaded = true;
+    for (int d = 0; d < 3; ++d) {
+      if (T.periodic[d]) {
+        if (n1[d] >= T.hi[d]) n1[d] -= T.L[d];
+        else if (n1[d] < T.lo[d]) n1[d] += T.L[d];
+        if (n2[d] >= T.hi[d]) n2[d] -= T.L[d];
+        else if (n2[d] < T.lo[d]) n2[d] += T.L[d];
       }
-      const float pr = T.prob[rx];
-      if (!(pr == 1.0f || rand_real(mt_draw<kBS>(m)) < pr)) continue;
-      const float dc1 = T.D[t1], dc2 = T.D[t2];
-      const float x = (dc1 == 0.0f && dc2 == 0.0f) ? 0.5f : dc2 / (dc1 + dc2);
-      // pos2 taken at its image nearest pos1 on periodic axes
-      const float q0 = nearest_image(p1.x, p2.x, T, 0);
-      const float q1 = nearest_image(p1.y, p2.y, T, 1);
-      const float q2 = nearest_image(p1.z, p2.z, T, 2);
-      const float omx = 1.0f - x;
-      float rp[3] = {fmaf(x, p1.x, omx * q0), fmaf(x, p1.y, omx * q1), fmaf(x, p1.z, omx * q2)};
-      const float th = smd_theta(rand_real(mt_draw<kBS>(m)));
-      const float ph = rand_real(mt_draw<kBS>(m)) * 6.28318548f;
-      const float ch = rand_real(mt_draw<kBS>(m)) * 6.28318548f;
-      float v1[3], v2[3];
-      rotate_offsets(th, ph, ch, T.prodPos[rx], v1, v2);
-      const uint32_t mol1 = a.packed ? unpack_index(p1.w) : a.vals[j];
-      const uint32_t mol2 = a.packed ? unpack_index(p2.w) : a.vals[c];
-      float n1[3] = {rp[0] + v1[0], rp[1] + v1[1], rp[2] + v1[2]};
-      float n2[3] = {rp[0] + v2[0], rp[1] + v2[1], rp[2] + v2[2]};
-  #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        if (T.periodic[d]) {
-          if (n1[d] >= T.hi[d]) n1[d] -= T.L[d];
-          else if (n1[d] < T.lo[d]) n1[d] += T.L[d];
-          if (n2[d] >= T.hi[d]) n2[d] -= T.L[d];
-          else if (n2[d] < T.lo[d]) n2[d] += T.L[d];
+    }
+    const int nt1 = T.prodX[rx], nt2 = T.prodY[rx];
+    a.pt[mol1] = make_float4(n1[0], n1[1], n1[2], __int_as_float(nt1 & kTypeMask));
+    a.pt[mol2] = make_float4(n2[0], n2[1], n2[2], __int_as_float(nt2 & kTypeMask));
+    if (a.w) {
+      a.w[mol1] = 0.0f;
+      a.w[mol2] = 0.0f;
+    }
+    uint32_t deaths = 0;
+    if (nt1 <= 0) {
+      ++deaths;
+      mark_removed(a.deaths, mol1, 1ull);
+      count_tiles(a.deaths.tileDead, mol1, 1ull);
+    }
+    if (nt2 <= 0) {
+      ++deaths;
+      mark_removed(a.deaths, mol2, 1ull);
+      count_tiles(a.deaths.tileDead, mol2, 1ull);
+    }
+    return deaths;
+  };
+
+  if (L <= kPairList) {
+    if (blockIdx.x >= kPairWgs) return;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < L; k += kBS) {
+      const uint4 p = a.cand.list[k];
+      if (p.z % kPairWgs != blockIdx.x) continue;  // another workgroup's stream
+      const uint2 back = a.cand.cand[p.y];
+      if (back.y == tag && back.x == p.x) s_pair[atomicAdd(&s_n, 1u)] = p;
+    }
+    __syncthreads();
+    const uint32_t n = s_n;
+    for (uint32_t k = threadIdx.x; k < n; k += kBS) {
+      const uint4 p = s_pair[k];
+      const uint32_t g = p.z;
+      uint32_t j = p.x;
+      mt_load<kBS>(m, &lds_mt[threadIdx.x], a.mtState, a.mtPar, a.Stot, g);
+      // the stream's pairs before and after this one
+      bool leads = true, more = false;
+      for (uint32_t q = 0; q < n; ++q) {
+        const uint4 o = s_pair[q];
+        leads = leads && !(o.z == g && o.x < j);
+        more = more || (o.z == g && o.x > j);
+      }
+      if (!leads) continue;
+      const ReplicaTables& T = tables[p.w];
+      uint32_t deaths = react(T, j, p.y);
+      while (more) {
+        uint4 next = make_uint4(0xFFFFFFFFu, 0u, 0u, 0u);
+        for (uint32_t q = 0; q < n; ++q) {
+          const uint4 o = s_pair[q];
+          if (o.z == g && o.x > j && o.x < next.x) next = o;
+        }
+        more = next.x != 0xFFFFFFFFu;
+        if (more) {
+          j = next.x;
+          deaths += react(T, j, next.y);
         }
       }
-      const int nt1 = T.prodX[rx], nt2 = T.prodY[rx];
-      a.pt[mol1] = make_float4(n1[0], n1[1], n1[2], __int_as_float(nt1 & kTypeMask));
-      a.pt[mol2] = make_float4(n2[0], n2[1], n2[2], __int_as_float(nt2 & kTypeMask));
-      if (a.w) {
-        a.w[mol1] = 0.0f;
-        a.w[mol2] = 0.0f;
+      mt_store<kBS>(m, a.mtState, a.Stot, g);
+      if (deaths) atomicAdd(&a.repDeaths[p.w], deaths);
+    }
+    return;
+  }
+
+  if (threadIdx.x == 0) s_n = 0;  // acting pairs
+  __syncthreads();
+  for (uint32_t b = blockIdx.x; b * kBS < a.Stot; b += gridDim.x) {
+    const uint32_t g = b * kBS + threadIdx.x;
+    if (g >= a.Stot) break;
+    // a wave never spans two replicas (stream ranges are 64-aligned), so the
+    // table fields load through the scalar cache
+    const int r = __builtin_amdgcn_readfirstlane(a.streamReplica[g]);
+    if (r < 0) continue;
+    const ReplicaTables& T = tables[r];
+    if (!T.hasBim) continue;
+    const uint32_t S = T.numStreams;
+    const uint32_t s = g - T.streamOff;
+    if (s >= S) continue;
+    const uint32_t lo = a.first[T.bucketOff];
+    const uint32_t hi = a.first[T.bucketOff + T.numBuckets];
+    bool loaded = false;
+    uint32_t deaths = 0, acting = 0;
+    // candidates of eight consecutive particles of the stream are loaded
+    // together; the particles are still handled in increasing j
+    constexpr int kAhead = 8;
+    for (uint32_t j0 = lo + s; j0 < hi; j0 += kAhead * S) {
+      uint2 cq[kAhead];
+#pragma unroll
+      for (int q = 0; q < kAhead; ++q) {
+        const uint32_t jq = j0 + (uint32_t)q * S;
+        cq[q] = jq < hi ? a.cand.cand[jq] : make_uint2(0u, 0u);
       }
-      if (nt1 <= 0) {
-        ++deaths;
-        mark_removed(a.deaths, mol1, 1ull);
-        count_tiles(a.deaths.tileDead, mol1, 1ull);
-      }
-      if (nt2 <= 0) {
-        ++deaths;
-        mark_removed(a.deaths, mol2, 1ull);
-        count_tiles(a.deaths.tileDead, mol2, 1ull);
+#pragma unroll
+      for (int q = 0; q < kAhead; ++q) {
+        const uint32_t j = j0 + (uint32_t)q * S;
+        const uint32_t c = cq[q].x;
+        if (cq[q].y != tag || c <= j) continue;
+        const uint2 back = a.cand.cand[c];
+        if (back.y != tag || back.x != j) continue;
+        ++acting;
+        if (!loaded) {
+          mt_load<kBS>(m, &lds_mt[threadIdx.x], a.mtState, a.mtPar, a.Stot, g);
+          loaded = true;
+        }
+        deaths += react(T, j, c);
       }
     }
+    if (loaded) mt_store<kBS>(m, a.mtState, a.Stot, g);
+    if (deaths) atomicAdd(&a.repDeaths[r], deaths);
+    if (acting) atomicAdd(&s_n, acting);
   }
-  if (loaded) mt_store<kBS>(m, a.mtState, a.Stot, g);
-  if (deaths) atomicAdd(&a.repDeaths[r], deaths);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_n) atomicAdd(a.cand.acting, s_n);
 }
 
 // Exclusive scans of K values per thread over the 1024-thread workgroup in
@@ -1374,12 +1472,16 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
   const uint32_t n = *a.dN;
   const uint32_t dead = e < a.tilesCap ? a.deaths.tileDead[e] : 0u;
   const uint32_t born = a.tileBirth && e < a.tilesCap ? a.tileBirth[e] : 0u;
-  uint32_t stepPrev = 0, status = 0;
+  uint32_t stepPrev = 0, status = 0, pairs = 0, acting = 0;
   unsigned long long psPrev = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     stepPrev = *a.stepCount;
     psPrev = *a.particleSteps;
     status = *a.status;
+    if (a.candCount) {
+      pairs = *a.candCount;
+      acting = *a.candActing;
+    }
   }
   if (e < a.tilesCap) a.tileDeadNext[e] = 0u;
   if (blockIdx.x > 0 && t0 >= (n + kCompactTile - 1u) / kCompactTile) return;  // no particles here
@@ -1424,6 +1526,11 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
       for (int k = 0; k < 4; ++k) c[k] += tot[k];
     }
     if (threadIdx.x == 0) {
+      if (a.candCount) {
+        // a list again once half of it would do
+        *a.candCount = pairs > kPairList && acting > kPairList / 2u ? kPairList + 1u : 0u;
+        *a.candActing = 0u;
+      }
       a.newOff[a.R] = c[0];
       *a.dNnext = c[0];
       *a.particleSteps = psPrev + n;
@@ -2518,8 +2625,11 @@ hipError_t launch_candidates(const CandArgs& a, uint32_t maxN, int blockSize, hi
   return hipGetLastError();
 }
 
+size_t pair_list_size() { return kPairList; }
+
 hipError_t launch_resolve(const ResolveArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL(k_resolve, dim3(cdiv(a.Stot, kBS)), dim3(kBS), 0, stream, a, a.tables);
+  hipLaunchKernelGGL(k_resolve, dim3(std::max(kPairWgs, std::min(kPairGrid, cdiv(a.Stot, kBS)))), dim3(kBS), 0,
+                     stream, a, a.tables);
   return hipGetLastError();
 }
 

@@ -81,7 +81,8 @@ class Engine {
   float4* dAddedPos = nullptr;
   int* dBirthType = nullptr;
   float4* dSortedPT = nullptr;
-  int* dCand = nullptr;
+  uint2* dCand = nullptr;           // pair candidates (CandList)
+  uint4* dCandList = nullptr;
   float4* dViewPos = nullptr;  // view() buffers
   int* dViewType = nullptr;
   uint32_t viewCap = 0;
@@ -164,6 +165,8 @@ class Engine {
   smd_status alloc_apart();
   smd_status take_apart(const float* pos4, size_t n);
   CanonMap canon_map() const;
+  CandArgs cand_args() const;
+  ResolveArgs resolve_args() const;
   ProducerArgs producer_args() const;
   ExportArgs export_args(int r) const;
   smd_status set_dense();

@@ -156,6 +156,21 @@ struct CellSortArgs {
   uint32_t* status;
 };
 
+// Pair candidates of a step: cand[j] = (partner, step tag) for the sorted
+// particles that have one; entries whose tag is not *stepCount + 1 are of
+// earlier steps.  The list holds, in any order, the possible pairs by their
+// lower index: (j, its candidate c > j, stream that j draws from, replica).
+struct CandList {
+  uint2* cand;
+  uint4* list;
+  // entries of the list; the finalize kernel sets it to 0 for the next step,
+  // or past pair_list_size() where the step had too many pairs for a list:
+  // then none is kept
+  uint32_t* count;
+  uint32_t* acting;  // reacting pairs found without a list; reset likewise
+  const uint32_t* stepCount;
+};
+
 struct CandArgs {
   const ReplicaTables* tables;
   const uint32_t* bucketStart;  // per replica bucketOff, [R] = deadKey
@@ -166,7 +181,7 @@ struct CandArgs {
   const float4* sortedPT;
   const uint32_t* first;
   const uint32_t* dLive;
-  int* cand;
+  CandList cand;
 };
 
 struct ResolveArgs {
@@ -176,7 +191,7 @@ struct ResolveArgs {
   const uint32_t* mtPar;
   uint32_t Stot;
   const uint32_t* first;
-  const int* cand;
+  CandList cand;
   const float4* sortedPT;
   const uint32_t* vals;
   int packed;  // sortedPT carries the particles' indices (vals unused)
@@ -206,6 +221,8 @@ struct FinalizeArgs {
   uint32_t* tileDeadNext;  // the other step parity's counts: cleared here
   uint32_t* tileBirth;     // nullptr: no particle can be born
   uint32_t* tileBirthPre;
+  uint32_t* candCount;   // CandList::count and acting (nullptr: no pairs)
+  uint32_t* candActing;
   unsigned long long* particleSteps;  // += particles entering the step
   uint32_t* stepCount;                // steps completed (incremented here)
   unsigned long long* countRing;      // host-visible: slot (steps & ringMask) = steps << 32 | particles
@@ -320,6 +337,8 @@ hipError_t launch_gather(const uint32_t* keys, const uint32_t* vals, const float
                          uint32_t maxN, uint32_t deadKey, float4* sortedPT, hipStream_t stream);
 // blockSize: 64, 128 or 256 threads (identical results)
 hipError_t launch_candidates(const CandArgs& a, uint32_t maxN, int blockSize, hipStream_t stream);
+// Entries of CandList::list.
+size_t pair_list_size();
 hipError_t launch_resolve(const ResolveArgs& a, hipStream_t stream);
 // Finalize workgroups for a capacity (one per 1024 tiles).
 uint32_t finalize_blocks(uint32_t capacity);

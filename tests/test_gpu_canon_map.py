@@ -109,3 +109,41 @@ def test_admitted_components_of_any_value(smd, orc, gpu):
         rp, rt = sim.state()
         assert np.array_equal(gt, rt) and np.array_equal(gp.view(np.uint32), rp.view(np.uint32)), slot
     e.close()
+
+
+@pytest.mark.parametrize("n,streams,kf,prob", [(3000, 1, 5.0, 0.0), (3000, 7, 5.0, 0.5), (3000, 3000, 5.0, 0.0),
+                                               (30000, 1, 5.0, 0.0), (30000, 70, 5.0, 0.5), (30000, 30000, 5.0, 0.0)])
+def test_pairs_of_one_stream_in_order(smd, orc, gpu, n, streams, kf, prob):
+    """Reacting pairs drawn from few streams, worked off from the list of
+    candidates (small systems) and by the walk over all particles (dense
+    ones), with and without a coin per pair."""
+    rx = dict(order=2, reactants=[1, 2], products=[3, 1], rate=kf)
+    if prob:
+        rx["prob"] = prob
+    spec = configs.make_spec(
+        D=[0.0, 1.0, 1.0, 0.5], dt=1e-3, reactions=[rx, dict(order=2, reactants=[1, 3], products=[2], rate=kf)],
+        box_lo=[0.0] * 3, box_hi=[16.0] * 3, faces=[smd.BC_REFLECT] * 6, grid_bits=(4, 5, 5), num_streams=streams,
+        seed=9)
+    rng = np.random.default_rng(n + streams)
+    pos = configs.uniform_box(rng, n, 0.0, 16.0)
+    types = rng.integers(1, 4, size=n).astype(np.int32)
+    print(f"pairs n={n} streams={streams} prob={prob}", flush=True)
+    e = smd.Engine(0)
+    e.add_replica(spec, pos, types)
+    e.finalize()
+    d = smd.Engine(0)
+    d.add_replica(spec, pos, types)
+    d.finalize()
+    st = d.debug_stage(3, n)
+    d.close()
+    some = int((st["cand"] >= 0).sum())
+    assert (some > 2200) == (n == 30000) and some > 40  # possible pairs: about half
+    e.step(5)
+    gp, gt = e.get(0)
+    gs = e.get_streams(0)
+    e.close()
+    sim = orc.sim_for(smd, spec, pos, types)
+    sim.step(smd.gauss_table(), 5)
+    rp, rt = sim.state()
+    assert np.array_equal(gt, rt) and np.array_equal(gp.view(np.uint32), rp.view(np.uint32))
+    assert gs.shape[0] == streams and len(rt) < n
