@@ -649,6 +649,7 @@ bool derive_tables(const smd_sim_spec& sp, ReplicaTables& T, smd_rxn_derived* de
       T.partnerMask[a] |= 1u << b;
       T.maxBindR2[a] = std::fmax(T.maxBindR2[a], T.bindR2[r]);
     }
+    T.maxBind[a] = std::sqrt(T.maxBindR2[a]);
   }
 
   // Geometry.
@@ -693,6 +694,7 @@ bool derive_tables(const smd_sim_spec& sp, ReplicaTables& T, smd_rxn_derived* de
     }
     if (cs < maxBind) { err = "cell size smaller than the largest binding radius"; return false; }
     T.cellSize[d] = cs;
+    T.invCell[d] = 1.0f / cs;
     T.origin[d] = T.periodic[d] ? sp.box_lo[d] : sp.origin[d];
   }
   if (totalBits > 28) { err = "grid too large"; return false; }

@@ -65,6 +65,7 @@ struct ReplicaTables {
   // largest squared binding radius over those reactions (pair-search filters)
   uint32_t partnerMask[kMaxTypes];
   float maxBindR2[kMaxTypes];
+  float maxBind[kMaxTypes];  // its square root
   // geometry
   float lo[3], hi[3];
   float L[3], halfL[3];
@@ -77,6 +78,7 @@ struct ReplicaTables {
   // uniform (wrapped) hash grid (particles_kernel.cu:169-186)
   float origin[3];
   float cellSize[3];
+  float invCell[3];        // 1 / cellSize
   uint32_t gbits[3];       // log2 of the grid dimension per axis
   uint32_t bucketOff;      // first global bucket of this replica
   uint32_t numBuckets;     // 2^(gbits sum)
