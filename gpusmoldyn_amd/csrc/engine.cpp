@@ -115,7 +115,7 @@ Engine::~Engine() {
   dfree(dInjType);
   dfree(dInjRep);
   if (countRing) (void)hipHostFree(countRing);
-  if (hostStatus) (void)hipHostFree(hostStatus);
+  if (stage) (void)hipHostFree(stage);
   dfree(dStepCount);
   if (stream) (void)hipStreamDestroy(stream);
 }
@@ -476,14 +476,33 @@ smd_status Engine::finalize(uint32_t capacity) {
                        hipHostMallocMapped | hipHostMallocCoherent));
   std::memset(countRing, 0, kRing * sizeof(unsigned long long));
   HIPCHK(hipHostGetDevicePointer((void**)&dCountRing, countRing, 0));
-  HIPCHK(hipHostMalloc((void**)&hostStatus, sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
-  *hostStatus = 0;
-  HIPCHK(hipHostGetDevicePointer((void**)&dHostStatus, hostStatus, 0));
+  st = alloc_stage();
+  if (st != SMD_OK) return st;
+  lastN = cnt;
   HIPCHK(dalloc(&dStepCount, 1));
   HIPCHK(hipMemset(dStepCount, 0, sizeof(uint32_t)));
   lastSeen = 0;
   HIPCHK(hipStreamSynchronize(stream));
   finalized = true;
+  return SMD_OK;
+}
+
+smd_status Engine::alloc_stage() {
+  stageCap = std::min(kStage, cap);
+  const size_t head = 256, pos = (size_t)stageCap * sizeof(float4);
+  HIPCHK(hipHostMalloc((void**)&stage, head + pos + (size_t)stageCap * sizeof(int),
+                       hipHostMallocMapped | hipHostMallocCoherent));
+  char* dev = nullptr;
+  HIPCHK(hipHostGetDevicePointer((void**)&dev, stage, 0));
+  std::memset(stage, 0, head);
+  hostStatus = (uint32_t*)stage;
+  dHostStatus = (uint32_t*)dev;
+  stageHead = (uint32_t*)(stage + 64);
+  dStageHead = (uint32_t*)(dev + 64);
+  stagePos = (float4*)(stage + head);
+  dStagePos = (float4*)(dev + head);
+  stageType = (int*)(stage + head + pos);
+  dStageType = (int*)(dev + head + pos);
   return SMD_OK;
 }
 
@@ -558,7 +577,7 @@ smd_status Engine::enqueue_step(StageTimer* timer) {
 void Engine::drop_graph(int which) {
   const int lo = which < 0 ? 0 : which, hi = which < 0 ? 1 : which;
   bool any = false;
-  for (int p = lo; p <= hi; ++p) any = any || gexec[p];
+  for (int p = lo; p <= hi; ++p) any = any || gexec[p] || oneExec[p];
   if (!any) return;
   // A launch of the graph may still be queued or running: the executable
   // graph (and the kernel arguments it owns) must outlive it.
@@ -568,8 +587,9 @@ void Engine::drop_graph(int which) {
   }
   for (int p = lo; p <= hi; ++p) {
     if (gexec[p]) (void)hipGraphExecDestroy(gexec[p]);
-    gexec[p] = nullptr;
-    gMaxN[p] = 0;
+    if (oneExec[p]) (void)hipGraphExecDestroy(oneExec[p]);
+    gexec[p] = oneExec[p] = nullptr;
+    gMaxN[p] = oneMaxN[p] = 0;
   }
 }
 
@@ -586,6 +606,62 @@ void Engine::restore(const HostSnapshot& s) {
   dN = s.n;
   dNnext = s.nnext;
   sb = s.sb;
+}
+
+// Captures `steps` steps of at most maxN particles; the host-side buffer
+// selection stays as it is (after: what the steps would make of it).
+smd_status Engine::capture(int steps, uint32_t maxN, hipGraphExec_t* exec, HostSnapshot* after) {
+  const HostSnapshot before = snapshot();
+  hipGraph_t g = nullptr;
+  HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+  smd_status st = SMD_OK;
+  for (int k = 0; k < steps && st == SMD_OK; ++k) st = enqueue_kernels(maxN, nullptr);
+  hipError_t e = hipStreamEndCapture(stream, &g);
+  // nothing ran: the host-side buffer selection goes back to where it was
+  if (after) *after = snapshot();
+  restore(before);
+  if (st != SMD_OK) {
+    if (g) (void)hipGraphDestroy(g);
+    return st;
+  }
+  HIPCHK(e);
+  hipGraphExec_t x = nullptr;
+  e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
+  (void)hipGraphDestroy(g);
+  if (e != hipSuccess) {
+    if (x) (void)hipGraphExecDestroy(x);
+    HIPCHK(e);
+  }
+  *exec = x;
+  return SMD_OK;
+}
+
+// One step: launch by launch the first time (a capture costs more than it
+// saves then), from a graph after that (the loop of a program that looks at
+// the particles after every step: 5 launches as one).
+smd_status Engine::step_one() {
+  smd_status st = ensure_capacity();
+  if (st != SMD_OK) return st;
+  const int p = cur;
+  if (!useGraphs || !oneSeen[p]) {
+    oneSeen[p] = true;
+    return enqueue_step(nullptr);
+  }
+  if (oneExec[p] && Nub > oneMaxN[p]) refresh_bound(true);
+  if (oneExec[p] && Nub > oneMaxN[p]) drop_graph(p);
+  if (!oneExec[p]) {
+    // headroom where the bound only follows stale counts
+    const uint32_t maxN = (uint32_t)std::min<uint64_t>(Nub + Nub / 2, cap);
+    st = capture(1, maxN, &oneExec[p], &oneAfter[p]);
+    if (st != SMD_OK) return st;
+    oneMaxN[p] = maxN;
+  }
+  HIPCHK(hipGraphLaunch(oneExec[p], stream));
+  restore(oneAfter[p]);
+  std::fill(slotPending.begin(), slotPending.end(), (uint8_t)0);
+  ++stepsDone;
+  Nub = std::min<uint64_t>(step_bound(Nub), (uint64_t)cap);
+  return SMD_OK;
 }
 
 // Two consecutive steps captured as one hipGraph: after two steps every
@@ -620,27 +696,8 @@ smd_status Engine::step_graph(int pairs) {
     }
     if (!gexec[p]) {
       const uint32_t maxN = (uint32_t)std::min<uint64_t>(want, cap);
-      const HostSnapshot before = snapshot();
-      hipGraph_t g = nullptr;
-      HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      smd_status st = enqueue_kernels(maxN, nullptr);
-      if (st == SMD_OK) st = enqueue_kernels(maxN, nullptr);
-      hipError_t e = hipStreamEndCapture(stream, &g);
-      // nothing ran: the host-side buffer selection goes back to where it was
-      restore(before);
-      if (st != SMD_OK) {
-        if (g) (void)hipGraphDestroy(g);
-        return st;
-      }
-      HIPCHK(e);
-      hipGraphExec_t x = nullptr;
-      e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (e != hipSuccess) {
-        if (x) (void)hipGraphExecDestroy(x);
-        HIPCHK(e);
-      }
-      gexec[p] = x;
+      smd_status st = capture(2, maxN, &gexec[p], nullptr);
+      if (st != SMD_OK) return st;
       gMaxN[p] = maxN;
     }
     HIPCHK(hipGraphLaunch(gexec[p], stream));
@@ -1006,9 +1063,7 @@ smd_status Engine::step(int nsteps) {
     nsteps -= 2 * (nsteps / 2);
   }
   for (int s = 0; s < nsteps; ++s) {
-    smd_status st = ensure_capacity();
-    if (st != SMD_OK) return st;
-    st = enqueue_step(nullptr);
+    smd_status st = step_one();
     if (st != SMD_OK) return st;
   }
   return SMD_OK;
@@ -1265,6 +1320,10 @@ smd_status Engine::particle_steps(unsigned long long* out) {
 smd_status Engine::counts(uint32_t* out) {
   smd_status st = sync();
   if (st != SMD_OK) return st;
+  if (count_known()) {
+    out[0] = (uint32_t)knownN;
+    return SMD_OK;
+  }
   HIPCHK(hipMemcpy(out, dRepCount, R * sizeof(uint32_t), hipMemcpyDeviceToHost));
   return SMD_OK;
 }
@@ -1278,7 +1337,6 @@ ExportArgs Engine::export_args(int r) const {
   a.repCount = dRepCount;
   a.R = (int)R;
   a.rep = r;
-  a.begin = 0;
   a.cap = 0xFFFFFFFFu;
   a.pos4 = nullptr;
   a.types = nullptr;
@@ -1301,13 +1359,37 @@ smd_status Engine::get(int r, float* pos4, int* types, uint32_t capN, uint32_t* 
     set_error("replica id out of range");
     return SMD_ERR_INVALID;
   }
+  const bool wants = capN && (pos4 || types);
+  uint32_t n = 0;
+  if (wants && lastN[r] <= stageCap) {
+    // a few particles: the export kernel writes them and their number into
+    // host memory, one launch and one wait
+    HIPCHK(hipSetDevice(device));
+    ExportArgs a = export_args(r);
+    a.cap = std::min(capN, stageCap);
+    a.pos4 = pos4 ? dStagePos : nullptr;
+    a.types = types ? dStageType : nullptr;
+    a.header = dStageHead;
+    HIPCHK(launch_export(a, a.cap, stream));
+    smd_status st = sync();
+    if (st != SMD_OK) return st;
+    n = lastN[r] = __atomic_load_n(stageHead, __ATOMIC_ACQUIRE);
+    if (nOut) *nOut = n;
+    const uint32_t m = std::min(n, capN);
+    if (m <= stageCap) {
+      if (pos4) std::memcpy(pos4, stagePos, m * sizeof(float4));
+      if (types) std::memcpy(types, stageType, m * sizeof(int));
+      return SMD_OK;
+    }
+  }
   smd_status st = sync();
   if (st != SMD_OK) return st;
-  uint32_t n = 0;
-  HIPCHK(hipMemcpy(&n, dRepCount + r, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  if (count_known()) n = (uint32_t)knownN;
+  else HIPCHK(hipMemcpy(&n, dRepCount + r, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  lastN[r] = n;
   if (nOut) *nOut = n;
   const uint32_t m = std::min(n, capN);
-  if (!m || !(pos4 || types)) return SMD_OK;
+  if (!m || !wants) return SMD_OK;
   st = view_buffers(m);
   if (st != SMD_OK) return st;
   ExportArgs a = export_args(r);

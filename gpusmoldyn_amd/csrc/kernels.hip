@@ -1359,18 +1359,18 @@ __global__ __launch_bounds__(kBS) void k_resolve(ResolveArgs a, const ReplicaTab
       }
       if (!leads) continue;
       const ReplicaTables& T = tables[p.w];
-      uint32_t deaths = react(T, j, p.y);
-      while (more) {
+      uint32_t deaths = 0, c = p.y;
+      for (;;) {
+        deaths += react(T, j, c);
+        if (!more) break;
         uint4 next = make_uint4(0xFFFFFFFFu, 0u, 0u, 0u);
         for (uint32_t q = 0; q < n; ++q) {
           const uint4 o = s_pair[q];
           if (o.z == g && o.x > j && o.x < next.x) next = o;
         }
-        more = next.x != 0xFFFFFFFFu;
-        if (more) {
-          j = next.x;
-          deaths += react(T, j, next.y);
-        }
+        if (next.x == 0xFFFFFFFFu) break;
+        j = next.x;
+        c = next.y;
       }
       mt_store<kBS>(m, a.mtState, a.Stot, g);
       if (deaths) atomicAdd(&a.repDeaths[p.w], deaths);
@@ -1677,8 +1677,8 @@ __global__ __launch_bounds__(256) void k_export(ExportArgs a) {
   const uint32_t k = blockIdx.x * 256 + threadIdx.x;
   const uint32_t n = a.rep >= 0 ? a.repCount[a.rep] : a.repOff[a.R];
   if (k == 0 && a.header) *a.header = n;
-  if (k >= a.cap || k + a.begin >= n) return;
-  uint32_t r = (uint32_t)a.rep, il = k + a.begin;
+  if (k >= a.cap || k >= n) return;
+  uint32_t r = (uint32_t)a.rep, il = k;
   if (a.rep < 0) {
     r = replica_of(a.repOff, a.R, il);
     il -= a.repOff[r];

@@ -92,7 +92,16 @@ class Engine {
   uint32_t *dTileBirth = nullptr, *dTileBirthPre = nullptr;
   uint32_t* dBlockSum = nullptr;  // births per finalize block
   uint32_t* dStatus = nullptr;    // sticky kernel error bits
-  uint32_t* hostStatus = nullptr;   // their copy in host memory, written by the finalize kernel
+  // host memory that kernels write: the error bits' copy (finalize kernel),
+  // and particles read back a few at a time (get)
+  static constexpr uint32_t kStage = 1u << 15;  // particles
+  uint32_t* hostStatus = nullptr;
+  float4* stagePos = nullptr;
+  int* stageType = nullptr;
+  uint32_t* stageHead = nullptr;
+  uint32_t stageCap = 0;
+  char* stage = nullptr;            // the allocation behind them
+  std::vector<uint32_t> lastN;      // per replica: a recent count (which way get() takes)
   uint32_t* dHostStatus = nullptr;  // its device address
   // order-0 creation: one stream per replica, a per-step creation buffer
   uint32_t *dZMt = nullptr, *dZPar = nullptr, *dZCount = nullptr, *dZeroBase = nullptr;
@@ -137,15 +146,21 @@ class Engine {
   uint64_t cellGroupsN = 0;         // particles (all replicas) up to which they serve
   uint32_t cellBinBits = 0;         // cells per bin (log2) when segments are bins of the high key bits
 
-  // hipGraph replay of two-step pairs, one executable graph per ping-pong
-  // parity (an eager step between pairs flips the parity)
+  // hipGraph replay of two-step pairs and of single steps, one executable
+  // graph per ping-pong parity (a single step flips the parity)
   bool useGraphs = true;
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
   uint32_t gMaxN[2] = {0, 0};
+  hipGraphExec_t oneExec[2] = {nullptr, nullptr};
+  uint32_t oneMaxN[2] = {0, 0};
+  bool oneSeen[2] = {false, false};  // a single step of this parity has been launched
   // Waits for the stream, then destroys the executable graph of parity
   // `which` (-1: both).
   void drop_graph(int which = -1);
 
+  // one replica's count is the total that the finalize kernel published
+  // (after sync)
+  bool count_known() const { return R == 1 && !slotsMode && lastSeen >= stepsDone; }
   bool seg_sorted() const;  // this engine's step sorts replica by replica
 
  private:
@@ -171,6 +186,10 @@ class Engine {
   ExportArgs export_args(int r) const;
   smd_status set_dense();
   smd_status view_buffers(uint32_t n);
+  smd_status alloc_stage();
+  float4* dStagePos = nullptr;
+  int* dStageType = nullptr;
+  uint32_t* dStageHead = nullptr;
   void free_particle_buffers();
   void refresh_bound(bool block);
   smd_status grow(uint64_t need);
@@ -187,6 +206,9 @@ class Engine {
   };
   HostSnapshot snapshot() const;
   void restore(const HostSnapshot& s);
+  HostSnapshot oneAfter[2] = {};  // the selection after a single-step graph
+  smd_status capture(int steps, uint32_t maxN, hipGraphExec_t* exec, HostSnapshot* after);
+  smd_status step_one();
 };
 
 }  // namespace smd

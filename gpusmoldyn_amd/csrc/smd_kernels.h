@@ -277,8 +277,8 @@ struct BirthArgs {
 };
 
 // Reads replica rep's canonical particles (all replicas, as one array, when
-// rep < 0) through the map into pos4 / types (either may be nullptr); header
-// gets the particle count and the status bits.
+// rep < 0) through the map into pos4 / types (either may be nullptr, both may
+// be host memory); header gets the particle count.
 struct ExportArgs {
   const float4* pt;
   const float* w;  // nullptr: in the records
@@ -286,7 +286,7 @@ struct ExportArgs {
   const uint32_t* repOff;    // [R+1]
   const uint32_t* repCount;
   int R, rep;
-  uint32_t begin, cap;       // particles [begin, begin + cap) of the replica
+  uint32_t cap;              // the first cap particles
   float4* pos4;
   int* types;
   uint32_t* header;          // nullptr: none
