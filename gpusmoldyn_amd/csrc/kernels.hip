@@ -49,7 +49,7 @@ __global__ __launch_bounds__(kBS) void k_mt_fill(uint32_t* __restrict__ st, cons
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= nStreams) return;
   Mt m;
-  mt_load<kBS>(m, &lds[threadIdx.x], st, par, S, g);
+  mt_load<kBS>(m, lds, st, par, S, g);
   int k = 0;
   if (batch3) {
     for (; k + 3 <= count; k += 3) {
@@ -75,6 +75,18 @@ __global__ __launch_bounds__(kBS) void k_mt_fill(uint32_t* __restrict__ st, cons
 // that used to move every record and fourth component once more per step (40
 // bytes per particle: 67 us of 474 for 9.36M particles, 33 of 315 for 4M) is
 // gone for a few registers here.
+//
+// What bounds it: with many streams (512 replicas of 2k to 64k) memory, 541 MB
+// in 110 us; with few (100k particles on 12.5k streams, one wave on a fifth of
+// the SIMDs) the instructions of one wave after another, 1 us per particle.
+// So the loop body stands once, is kept short - 165 vector instructions per
+// particle for a system without order-1 reactions, 250 with the faces tried one
+// by one, the grid divisions and the index wrap by comparison - and the faces
+// are looked at only by waves that hold a particle beyond one.  us before /
+// after: 100k 16.0 / 13.5, 1M periodic 22.6 / 19.8, 4M clustered 59 / 50, 48 of
+// 4k to 131k 28 / 24, the 512 replicas 117 / 110.  Tried without gain: three or
+// eight records requested at once, nine draws at once (100k no faster, 125
+// VGPRs), faces by selects without a branch (the 512 replicas 136).
 // ---------------------------------------------------------------------------
 // Per-type and per-reaction entries the producer indexes per particle, staged
 // in LDS for each wave's replica (a few hundred bytes per wave).
@@ -186,7 +198,7 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
     // the replica's box, grid and reaction flags in registers for the loop
     const BoxGeom G = box_geom(T);
     const int hasUni = T.hasUni, unbindOffsets = T.unbindOffsets, numSpheres = T.numSpheres;
-    // Records are requested one pair of particles ahead, from where the last
+    // Records are requested one particle ahead, from where the last
     // step left them: behind the holes of the particles it removed.  Lane q
     // holds, for the wave's iteration 64 * block + q, the holes before lane
     // 0's particle and how many survivors precede the next hole; a wave whose
@@ -221,10 +233,10 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
       src = src_index(it);
       return (laneOK && s + it * S < n) ? a.ptIn[src] : make_float4(0.f, 0.f, 0.f, 0.f);
     };
-    uint32_t i0, i1;
-    float4 p0 = rec(0, i0), p1 = rec(1, i1);
+    uint32_t i0;
+    float4 p0 = rec(0, i0);
     Mt m;
-    if (laneOK && !kill) mt_load<BS>(m, &lds_mt[threadIdx.x], a.mtState, a.mtPar, a.Stot, g);
+    if (laneOK && !kill) mt_load<BS>(m, lds_mt, a.mtState, a.mtPar, a.Stot, g);
     // the stream parameters are complete before the loop, so no wait inside
     // it covers them (such a wait would also cover the records in flight)
     asm volatile("" ::"v"(m.a), "v"(m.mb), "v"(m.mc), "v"(m.mti1));
@@ -247,44 +259,40 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
         mt_draw3<BS>(m, u0, u1, u2);
         const float rt = L.rate[t];
         float np[3];
-        np[0] = fmaf(rt, gauss_entry(lds_gauss, u0 & (kGaussDim - 1)), p.x);
-        np[1] = fmaf(rt, gauss_entry(lds_gauss, u1 & (kGaussDim - 1)), p.y);
-        np[2] = fmaf(rt, gauss_entry(lds_gauss, u2 & (kGaussDim - 1)), p.z);
+        np[0] = fmaf(rt, gauss_entry(lds_gauss, u0), p.x);
+        np[1] = fmaf(rt, gauss_entry(lds_gauss, u1), p.y);
+        np[2] = fmaf(rt, gauss_entry(lds_gauss, u2), p.z);
         bool wZero = false;  // the fourth component becomes 0 (offset products)
-        int bt = 0;
-        float bp[3] = {np[0], np[1], np[2]};
-        float bw = 0.0f;
-        if (t > 0 && hasUni) {
+        if (hasUni && t > 0) {
           const int cnt = L.uniCount[t];
           const int base = L.uniStart[t];
           for (int j = 0; j < cnt; ++j) {
             const int rx = L.uniList[base + j];
             if (rand_real(mt_draw<BS>(m)) < L.prob[rx]) {
-              if (L.prodX[rx] <= 0) {
-                t = 0;
-              } else {
-                t = L.prodX[rx];
-                const int t2 = L.prodY[rx];
-                if (t2 > 0) {
-                  bt = t2;
-                  if (unbindOffsets) {
-                    const float th = smd_theta(rand_real(mt_draw<BS>(m)));
-                    const float ph = rand_real(mt_draw<BS>(m)) * 6.28318548f;
-                    const float ch = rand_real(mt_draw<BS>(m)) * 6.28318548f;
-                    float v1[3], v2[3];
-                    rotate_offsets(th, ph, ch, T.prodPos[rx], v1, v2);
-                    bp[0] = np[0] + v2[0];
-                    bp[1] = np[1] + v2[1];
-                    bp[2] = np[2] + v2[2];
-                    np[0] = np[0] + v1[0];
-                    np[1] = np[1] + v1[1];
-                    np[2] = np[2] + v1[2];
-                    wZero = true;
-                  } else {
-                    // the birth inherits the parent's fourth component
-                    bw = APART ? a.wIn[src] : __int_as_float(word & ~kTypeMask);
-                  }
+              t = max(L.prodX[rx], 0);
+              const int t2 = L.prodY[rx];
+              if (t > 0 && t2 > 0) {
+                birth = true;
+                float4 bp;
+                if (unbindOffsets) {
+                  const float th = smd_theta(rand_real(mt_draw<BS>(m)));
+                  const float ph = rand_real(mt_draw<BS>(m)) * 6.28318548f;
+                  const float ch = rand_real(mt_draw<BS>(m)) * 6.28318548f;
+                  float v1[3], v2[3];
+                  rotate_offsets(th, ph, ch, T.prodPos[rx], v1, v2);
+                  bp = make_float4(np[0] + v2[0], np[1] + v2[1], np[2] + v2[2], 0.0f);
+                  np[0] = np[0] + v1[0];
+                  np[1] = np[1] + v1[1];
+                  np[2] = np[2] + v1[2];
+                  wZero = true;
+                } else {
+                  // the birth inherits the parent's fourth component
+                  bp = make_float4(np[0], np[1], np[2], APART ? a.wIn[src] : __int_as_float(word & ~kTypeMask));
                 }
+                // birth types are zero except where there is a birth to take
+                // (it clears them again), so only births are written
+                a.birthType[i] = t2;
+                a.addedPos[i] = bp;
               }
               break;
             }
@@ -293,24 +301,17 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
         uint32_t key = a.deadKey;
         if (t > 0) {
           const float o[3] = {p.x, p.y, p.z};
-          if (!apply_box(G, np)) {
+          if (!inside_box(G, np) && !apply_box(T, np)) {
             t = 0;
           } else {
             if (numSpheres) apply_spheres(T, o, np);
-            key = bucketOff + grid_hash(G, np[0], np[1], np[2]);
+            key = bucketOff + grid_hash(G, T, np);
           }
         }
         a.pt[i] = make_float4(np[0], np[1], np[2], __int_as_float((wZero ? 0 : word & ~kTypeMask) | t));
         if (APART) a.w[i] = wZero ? 0.0f : a.wIn[src];
         a.key[i] = key;
-        // birth types are zero except where the scatter has a birth to take
-        // (it clears them again), so only births are written
-        if (bt) {
-          a.birthType[i] = bt;
-          a.addedPos[i] = make_float4(bp[0], bp[1], bp[2], bw);
-        }
         alive = t > 0;
-        birth = bt > 0;
         db += (alive ? 0ull : 1ull) + (birth ? (1ull << 32) : 0ull);
       }
       // removed particles and births, by slot: lanes hold consecutive slots
@@ -326,20 +327,16 @@ __global__ __launch_bounds__(BS) void k_producer(ProducerArgs a, const ReplicaTa
       }
       return db;
     };
-    uint32_t it = 0;
     uint64_t db = 0;
-    for (; it + 2 <= iters; it += 2) {
-      // this pair's records were requested one pair ago; the next pair's are
-      // requested before this pair's stores, so waiting for them later does
-      // not wait for those stores
-      const float4 c0 = p0, c1 = p1;
-      const uint32_t j0 = i0, j1 = i1;
-      p0 = rec(it + 2, i0);
-      p1 = rec(it + 3, i1);
+#pragma unroll 1
+    for (uint32_t it = 0; it < iters; ++it) {
+      // this record was requested a particle ago; the next one's is requested
+      // before this one's stores, so waiting for it does not wait for those
+      const float4 c0 = p0;
+      const uint32_t j0 = i0;
+      p0 = rec(it + 1, i0);
       db += step_one(c0, it, j0);
-      db += step_one(c1, it + 1, j1);
     }
-    if (it < iters) db += step_one(p0, it, i0);
     nDeaths += (uint32_t)db;
     nBirths += (uint32_t)(db >> 32);
     if (laneOK && !kill) mt_store<BS>(m, a.mtState, a.Stot, g);
@@ -1349,7 +1346,7 @@ __global__ __launch_bounds__(kBS) void k_resolve(ResolveArgs a, const ReplicaTab
       const uint4 p = s_pair[k];
       const uint32_t g = p.z;
       uint32_t j = p.x;
-      mt_load<kBS>(m, &lds_mt[threadIdx.x], a.mtState, a.mtPar, a.Stot, g);
+      mt_load<kBS>(m, lds_mt, a.mtState, a.mtPar, a.Stot, g);
       // the stream's pairs before and after this one
       bool leads = true, more = false;
       for (uint32_t q = 0; q < n; ++q) {
@@ -1415,7 +1412,7 @@ __global__ __launch_bounds__(kBS) void k_resolve(ResolveArgs a, const ReplicaTab
         if (back.y != tag || back.x != j) continue;
         ++acting;
         if (!loaded) {
-          mt_load<kBS>(m, &lds_mt[threadIdx.x], a.mtState, a.mtPar, a.Stot, g);
+          mt_load<kBS>(m, lds_mt, a.mtState, a.mtPar, a.Stot, g);
           loaded = true;
         }
         deaths += react(T, j, c);
@@ -1756,7 +1753,7 @@ __global__ __launch_bounds__(64) void k_zero(ZeroArgs a) {
     return;
   }
   Mt m;
-  mt_load<64>(m, &lds_mt[threadIdx.x], a.zMt, a.zPar, (uint32_t)a.R, (uint32_t)r);
+  mt_load<64>(m, lds_mt, a.zMt, a.zPar, (uint32_t)a.R, (uint32_t)r);
   const uint32_t cap = T.zeroMax;
   uint32_t cnt = 0;
   bool over = false;

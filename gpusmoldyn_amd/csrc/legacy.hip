@@ -88,12 +88,12 @@ inline unsigned cdiv(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
 // AoS stream records: load the 19 words into the workgroup's LDS state.
 // ---------------------------------------------------------------------------
 template <int BS>
-__device__ __forceinline__ void aos_load(Mt& m, uint32_t* lds_lane, const uint32_t* rec, const uint32_t* table,
+__device__ __forceinline__ void aos_load(Mt& m, uint32_t* lds, const uint32_t* rec, const uint32_t* table,
                                          uint32_t s) {
-  m.s = lds_lane;
+  m.s = lds;
 #pragma unroll
-  for (int w = 0; w < kMtNN; ++w) lds_lane[w * BS] = rec[w];
-  m.i = (int)rec[19];
+  for (int w = 0; w < kMtNN; ++w) lds[w * BS + threadIdx.x] = rec[w];
+  m.at = mt_offset<BS>(rec[19]);
   m.mti1 = rec[20];
   m.a = table[4 * s];
   m.mb = table[4 * s + 1];
@@ -103,8 +103,8 @@ __device__ __forceinline__ void aos_load(Mt& m, uint32_t* lds_lane, const uint32
 template <int BS>
 __device__ __forceinline__ void aos_store(const Mt& m, uint32_t* rec) {
 #pragma unroll
-  for (int w = 0; w < kMtNN; ++w) rec[w] = m.s[w * BS];
-  rec[19] = (uint32_t)m.i;
+  for (int w = 0; w < kMtNN; ++w) rec[w] = m.s[w * BS + threadIdx.x];
+  rec[19] = mt_index<BS>(m);
   rec[20] = m.mti1;
 }
 
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(kLBS) void k_legacy_integrate(IntegrateArgs a) {
   if (s >= (uint32_t)kLegacyStreams || s >= a.n) return;
   Mt m;
   uint32_t* rec = a.st + (size_t)kAosWords * s;
-  aos_load<kLBS>(m, &lds_mt[threadIdx.x], rec, a.table, s);
+  aos_load<kLBS>(m, lds_mt, rec, a.table, s);
   for (uint32_t i = s; i < a.n; i += kLegacyStreams) {
     float4 p = a.pos[i];
     const int type = a.types[i];
@@ -327,7 +327,7 @@ __global__ __launch_bounds__(kLBS) void k_legacy_resolve(CollideArgs a) {
     const int c = a.cand[j];
     if (c <= (int)j || a.cand[c] != (int)j) continue;
     if (!loaded) {
-      aos_load<kLBS>(m, &lds_mt[threadIdx.x], rec, a.mtTable, s);
+      aos_load<kLBS>(m, lds_mt, rec, a.mtTable, s);
       loaded = true;
     }
     const uint32_t m1 = a.index[j], m2 = a.index[c];

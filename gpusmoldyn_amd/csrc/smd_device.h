@@ -19,15 +19,28 @@ namespace smd {
 // lanes of a workgroup live in LDS, word-major: word w of lane t is at
 // lds[w * BS + t], so a wave's accesses to one word index are bank-conflict
 // free.  `mti1` caches lds[iState] exactly like the reference's state->mti1.
+// The state index is kept as the byte offset of the lane's word: a word k
+// further on is at mt_word(m, k), a sum and a minimum.
 // ---------------------------------------------------------------------------
 struct Mt {
-  uint32_t* s;     // &lds[threadIdx.x]
-  int i;           // iState
+  uint32_t* s;     // the workgroup's array
+  uint32_t at;     // (iState * BS + threadIdx.x) * 4
   uint32_t mti1;
   uint32_t a, mb, mc;
 };
 
-__device__ __forceinline__ int wrap19(int x) { return x >= kMtNN ? x - kMtNN : x; }
+template <int BS>
+__device__ __forceinline__ uint32_t mt_offset(uint32_t iState) { return (iState * BS + threadIdx.x) * 4u; }
+template <int BS>
+__device__ __forceinline__ uint32_t mt_index(const Mt& m) { return m.at / (BS * 4u); }
+
+// Offset of word iState + k (mod 19), k < 19.
+template <int BS>
+__device__ __forceinline__ uint32_t mt_at(const Mt& m, uint32_t k) {
+  const uint32_t x = m.at + k * (BS * 4u);
+  return min(x, x - kMtNN * BS * 4u);  // the difference wraps past x below 19 words
+}
+__device__ __forceinline__ uint32_t& mt_word(const Mt& m, uint32_t at) { return *(uint32_t*)((char*)m.s + at); }
 
 __device__ __forceinline__ uint32_t mt_temper(uint32_t x, uint32_t mb, uint32_t mc) {
   x ^= x >> 12;
@@ -44,14 +57,13 @@ __device__ __forceinline__ uint32_t mt_twist(uint32_t cur, uint32_t next, uint32
 
 template <int BS>
 __device__ __forceinline__ uint32_t mt_draw(Mt& m) {
-  int i1 = wrap19(m.i + 1);
-  int iM = wrap19(m.i + kMtMM);
-  uint32_t next = m.s[i1 * BS];
-  uint32_t mid = m.s[iM * BS];
-  uint32_t x = mt_twist(m.mti1, next, mid, m.a);
-  m.s[m.i * BS] = x;
+  const uint32_t i1 = mt_at<BS>(m, 1);
+  const uint32_t next = mt_word(m, i1);
+  const uint32_t mid = mt_word(m, mt_at<BS>(m, kMtMM));
+  const uint32_t x = mt_twist(m.mti1, next, mid, m.a);
+  mt_word(m, m.at) = x;
   m.mti1 = next;
-  m.i = i1;
+  m.at = i1;
   return mt_temper(x, m.mb, m.mc);
 }
 
@@ -60,19 +72,18 @@ __device__ __forceinline__ uint32_t mt_draw(Mt& m) {
 // i..i+2; none of the reads hits a word written earlier in the batch.
 template <int BS>
 __device__ __forceinline__ void mt_draw3(Mt& m, uint32_t& o0, uint32_t& o1, uint32_t& o2) {
-  const int i0 = m.i;
-  const int i1 = wrap19(i0 + 1), i2 = wrap19(i0 + 2), i3 = wrap19(i0 + 3);
-  const int m1 = wrap19(i0 + 9), m2 = wrap19(i0 + 10), m3 = wrap19(i0 + 11);
-  const uint32_t r1 = m.s[i1 * BS], r2 = m.s[i2 * BS], r3 = m.s[i3 * BS];
-  const uint32_t q1 = m.s[m1 * BS], q2 = m.s[m2 * BS], q3 = m.s[m3 * BS];
+  const uint32_t i1 = mt_at<BS>(m, 1), i2 = mt_at<BS>(m, 2), i3 = mt_at<BS>(m, 3);
+  const uint32_t r1 = mt_word(m, i1), r2 = mt_word(m, i2), r3 = mt_word(m, i3);
+  const uint32_t q1 = mt_word(m, mt_at<BS>(m, kMtMM)), q2 = mt_word(m, mt_at<BS>(m, kMtMM + 1)),
+                 q3 = mt_word(m, mt_at<BS>(m, kMtMM + 2));
   const uint32_t x1 = mt_twist(m.mti1, r1, q1, m.a);
   const uint32_t x2 = mt_twist(r1, r2, q2, m.a);
   const uint32_t x3 = mt_twist(r2, r3, q3, m.a);
-  m.s[i0 * BS] = x1;
-  m.s[i1 * BS] = x2;
-  m.s[i2 * BS] = x3;
+  mt_word(m, m.at) = x1;
+  mt_word(m, i1) = x2;
+  mt_word(m, i2) = x3;
   m.mti1 = r3;
-  m.i = i3;
+  m.at = i3;
   o0 = mt_temper(x1, m.mb, m.mc);
   o1 = mt_temper(x2, m.mb, m.mc);
   o2 = mt_temper(x3, m.mb, m.mc);
@@ -81,13 +92,13 @@ __device__ __forceinline__ void mt_draw3(Mt& m, uint32_t& o0, uint32_t& o1, uint
 // Global SoA stream state: word w of stream g at st[w * S + g] (w = 19 holds
 // iState); per-stream parameters at par[k * S + g] (matrix_a, mask_b, mask_c).
 template <int BS>
-__device__ __forceinline__ void mt_load(Mt& m, uint32_t* lds_lane, const uint32_t* __restrict__ st,
+__device__ __forceinline__ void mt_load(Mt& m, uint32_t* lds, const uint32_t* __restrict__ st,
                                         const uint32_t* __restrict__ par, uint32_t S, uint32_t g) {
-  m.s = lds_lane;
+  m.s = lds;
 #pragma unroll
-  for (int w = 0; w < kMtNN; ++w) lds_lane[w * BS] = st[(size_t)w * S + g];
-  m.i = (int)st[(size_t)kMtNN * S + g];
-  m.mti1 = lds_lane[m.i * BS];
+  for (int w = 0; w < kMtNN; ++w) lds[w * BS + threadIdx.x] = st[(size_t)w * S + g];
+  m.at = mt_offset<BS>(st[(size_t)kMtNN * S + g]);
+  m.mti1 = mt_word(m, m.at);
   m.a = par[g];
   m.mb = par[(size_t)S + g];
   m.mc = par[(size_t)2 * S + g];
@@ -96,8 +107,8 @@ __device__ __forceinline__ void mt_load(Mt& m, uint32_t* lds_lane, const uint32_
 template <int BS>
 __device__ __forceinline__ void mt_store(const Mt& m, uint32_t* __restrict__ st, uint32_t S, uint32_t g) {
 #pragma unroll
-  for (int w = 0; w < kMtNN; ++w) st[(size_t)w * S + g] = m.s[w * BS];
-  st[(size_t)kMtNN * S + g] = (uint32_t)m.i;
+  for (int w = 0; w < kMtNN; ++w) st[(size_t)w * S + g] = m.s[w * BS + threadIdx.x];
+  st[(size_t)kMtNN * S + g] = mt_index<BS>(m);
 }
 
 // ---------------------------------------------------------------------------
@@ -206,17 +217,15 @@ __device__ __forceinline__ float min_image(float d, const ReplicaTables& T, int 
 // ---------------------------------------------------------------------------
 // Box faces (per axis: upper face first, then lower face, as in
 // particles_kernel.cu:73-86) and reflective spheres.  Returns false when an
-// absorbing face removes the particle.  Geo is ReplicaTables or BoxGeom.
+// absorbing face removes the particle.
 // ---------------------------------------------------------------------------
 
 // The box and grid fields of a replica's tables, copied once into registers
 // by a loop that moves many particles of one replica (read through the
 // scalar cache otherwise, once per particle).
 struct BoxGeom {
-  float lo[3], hi[3], L[3];
-  int32_t face[6];
-  float particleRadius;
-  float origin[3], cellSize[3];
+  float inLo[3], inHi[3];  // positions in [inLo, inHi) that no face acts on
+  float origin[3], invCell[3];
   uint32_t gbits[3];
 };
 
@@ -224,21 +233,26 @@ __device__ __forceinline__ BoxGeom box_geom(const ReplicaTables& T) {
   BoxGeom G;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    G.lo[d] = T.lo[d];
-    G.hi[d] = T.hi[d];
-    G.L[d] = T.L[d];
+    const bool per = T.face[2 * d + 1] == kPeriodic;
+    G.inLo[d] = !per && T.face[2 * d] == kClamp ? T.lo[d] + T.particleRadius : T.lo[d];
+    G.inHi[d] = T.face[2 * d + 1] == kClamp ? T.hi[d] - T.particleRadius : T.hi[d];
     G.origin[d] = T.origin[d];
-    G.cellSize[d] = T.cellSize[d];
+    G.invCell[d] = T.invCell[d];
     G.gbits[d] = T.gbits[d];
   }
-#pragma unroll
-  for (int f = 0; f < 6; ++f) G.face[f] = T.face[f];
-  G.particleRadius = T.particleRadius;
   return G;
 }
 
-template <class Geo>
-__device__ __forceinline__ bool apply_box(const Geo& T, float* p) {
+// Whether no face acts on the position (a particle moves about a hundredth of
+// the box, so few waves hold one that meets a face).
+__device__ __forceinline__ bool inside_box(const BoxGeom& G, const float* p) {
+  bool in = true;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) in = in && p[d] >= G.inLo[d] && p[d] < G.inHi[d];
+  return in;
+}
+
+__device__ __forceinline__ bool apply_box(const ReplicaTables& T, float* p) {
   bool alive = true;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
@@ -312,14 +326,30 @@ __device__ __forceinline__ void apply_spheres(const ReplicaTables& T, const floa
 
 // calcGridPos + calcGridHash (particles_kernel.cu:169-186), local to a
 // replica's grid; the caller adds the replica's bucket offset.
-template <class Geo>
-__device__ __forceinline__ uint32_t grid_hash(const Geo& T, float x, float y, float z) {
-  const int gx = (int)floorf((x - T.origin[0]) / T.cellSize[0]);
-  const int gy = (int)floorf((y - T.origin[1]) / T.cellSize[1]);
-  const int gz = (int)floorf((z - T.origin[2]) / T.cellSize[2]);
-  const uint32_t mx = (1u << T.gbits[0]) - 1u, my = (1u << T.gbits[1]) - 1u, mz = (1u << T.gbits[2]) - 1u;
-  return (((uint32_t)gz & mz) << (T.gbits[0] + T.gbits[1])) | (((uint32_t)gy & my) << T.gbits[0]) |
-         ((uint32_t)gx & mx);
+// The cell number is floor((x - origin) / cellSize) with the quotient rounded
+// as the division rounds it.  The product with the reciprocal is within
+// 1.5 * 2^-23 of that quotient (relatively), so where it is further than
+// kCellMargin of itself from a whole number both have the same floor; the few
+// other positions divide.  (Three divisions are 33 instructions, a tenth of
+// what the producer runs for a particle.)
+constexpr float kCellMargin = 4.76837158203125e-7f;  // 2^-21
+__device__ __forceinline__ uint32_t grid_hash(const BoxGeom& G, const ReplicaTables& T, const float* p) {
+  uint32_t g[3];
+  bool sure = true;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const float q = (p[d] - G.origin[d]) * G.invCell[d];
+    const float f = floorf(q);
+    g[d] = (uint32_t)(int)f;
+    sure = sure && fabsf((q - f) - 0.5f) < fmaf(fabsf(q), -kCellMargin, 0.5f);
+  }
+  if (!sure) {
+    asm volatile("");  // or the compiler divides for everyone and selects
+#pragma unroll
+    for (int d = 0; d < 3; ++d) g[d] = (uint32_t)(int)floorf((p[d] - T.origin[d]) / T.cellSize[d]);
+  }
+  const uint32_t mx = (1u << G.gbits[0]) - 1u, my = (1u << G.gbits[1]) - 1u, mz = (1u << G.gbits[2]) - 1u;
+  return ((g[2] & mz) << (G.gbits[0] + G.gbits[1])) | ((g[1] & my) << G.gbits[0]) | (g[0] & mx);
 }
 
 __device__ __forceinline__ uint64_t lanemask_lt() {
@@ -337,12 +367,15 @@ __device__ __forceinline__ uint32_t unpack_index(float w) { return __float_as_ui
 // antisymmetric and then rotated right by one: t[u] = -t[kGaussDim + 1 - u]
 // for 2 <= u < kGaussDim and t[0] = -t[1].  Its half h[j] = t[j + 1],
 // j < kGaussDim / 2, holds all of it: t[u] = h[u - 1] for 1 <= u <=
-// kGaussDim / 2, otherwise -h[(kGaussDim - u) mod kGaussDim / 2].
+// kGaussDim / 2, otherwise -h[(kGaussDim - u) mod kGaussDim / 2].  Only the
+// low kGaussBits bits of u count.
 __device__ __forceinline__ float gauss_entry(const float* h, uint32_t u) {
-  const uint32_t k = u - 1u;  // wraps for u = 0
-  const bool lower = k < (uint32_t)(kGaussDim / 2);
-  const float v = h[lower ? k : (((uint32_t)kGaussDim - u) & (uint32_t)(kGaussDim / 2 - 1))];
-  return lower ? v : -v;
+  // below the middle entry k = u - 1 is stored; above it (and for u = 0) the
+  // entry kGaussDim - 1 - k, all bits of k turned, with the other sign
+  const uint32_t k = u - 1u;
+  const uint32_t upper = (uint32_t)((int32_t)(k << (32 - kGaussBits)) >> 31);
+  const float v = h[(k ^ upper) & (uint32_t)(kGaussDim / 2 - 1)];
+  return __uint_as_float(__float_as_uint(v) ^ (upper & 0x80000000u));
 }
 
 // Number of set bits of m at lanes below this one (v_mbcnt).

@@ -14,7 +14,8 @@ constexpr int kMtNN = 19;        // dcmt MEXP 607 state words (MersenneTwister.h
 constexpr int kMtMM = 9;         // middle word offset (MersenneTwister.cuh:29)
 constexpr int kMtWords = 20;     // 19 state words + iState, stored word-major (SoA)
 constexpr int kMtParamSets = 32768;  // records in MersenneTwister.dat (MersenneTwister.h:31)
-constexpr int kGaussDim = 4096;  // particles_kernel.cuh:43
+constexpr int kGaussBits = 12;
+constexpr int kGaussDim = 1 << kGaussBits;  // particles_kernel.cuh:43
 constexpr int kCompactTile = 1024;   // particle slots per tile of the death and birth counters
 // The fourth word of a canonical record holds the particle's type in its low
 // kIndexShift bits and, above them, the bits of its fourth position component
