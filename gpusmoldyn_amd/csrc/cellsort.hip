@@ -37,6 +37,12 @@ constexpr uint32_t T = kCellThreads;
 constexpr uint32_t W = T / 64;                        // waves
 constexpr uint32_t kVecs = 2;                         // vectors of four keys per thread per counting round
 constexpr uint32_t kVecRound = T * kVecs;
+// With at most a workgroup per CU, registers are free and the key reads are a
+// chain of latencies: step of one system, us, in rounds / kept: 8k particles
+// 26.4 / 25.6, 16k 27.2 / 26.0, 32k 33.9 / 32.4, 48k 40.0 / 38.2.  With more
+// workgroups four of them share a CU, which 148 VGPRs would not allow.
+constexpr uint32_t kKeepGroups = 256;
+constexpr int kKeepVecs = 24;
 constexpr uint32_t kRounds = 64;                      // counting rounds that a wave remembers
 constexpr int kKeys = 4;                              // keys per thread per round of the ordered path
 constexpr uint32_t kRound = T * kKeys;
@@ -159,8 +165,11 @@ __device__ __forceinline__ void cs_digit_pass(CsLds& s, uint32_t n, int shift) {
 
 // PART: segments are the bins of a digit pass (a.vals holds the particles'
 // indices, a.binTotals the bin sizes); otherwise the replicas.
-template <bool PART>
-__global__ __launch_bounds__(T, 8) void k_cell_sort(CellSortArgs a, const ReplicaTables* __restrict__ tables,
+// KEEP > 0: the keys of a segment of at most KEEP * T vectors stay in registers
+// between counting and the list, requested at once; a larger segment reads them
+// again, in rounds.
+template <bool PART, int KEEP>
+__global__ __launch_bounds__(T, KEEP ? 2 : 8) void k_cell_sort(CellSortArgs a, const ReplicaTables* __restrict__ tables,
                                                     const uint32_t* __restrict__ keys,
                                                     const float4* __restrict__ src) {
   __shared__ CsLds s;
@@ -261,23 +270,52 @@ __global__ __launch_bounds__(T, 8) void k_cell_sort(CellSortArgs a, const Replic
   };
   uint32_t below = 0, kk[4 * kVecs];
   uint64_t mine = 0;  // rounds in which this wave met keys of the slice
-  loadv(0u, kk);
-  for (uint32_t r = 0; r < rounds; ++r) {
-    // the next round's keys are requested before this round's are counted
-    uint32_t kn[4 * kVecs];
-    if (r + 1u < rounds) loadv(r + 1u, kn);
-    uint64_t any = 0;
+  uint4 kept[KEEP ? KEEP : 1];
+  auto count = [&](uint32_t key) __attribute__((always_inline)) {
+    const uint32_t c = key - key0;
+    below += key < key0 ? 1u : 0u;
+    if (c < nc) atomicAdd(&s.hist[c], 1u);
+  };
+  // the segment's keys fit the registers of the workgroup
+  const bool keeps = KEEP > 0 && v1 - v0 <= (uint32_t)KEEP * T;
+  if (keeps) {
 #pragma unroll
-    for (uint32_t q = 0; q < 4 * kVecs; ++q) {
-      const uint32_t c = kk[q] - key0;
-      below += kk[q] < key0 ? 1u : 0u;
-      any |= __ballot(c < nc);
-      if (c < nc) atomicAdd(&s.hist[c], 1u);
+    for (uint32_t q = 0; q < KEEP; ++q) {
+      const uint32_t v = v0 + q * T + t;
+      kept[q] = v < v1 ? keys4[v] : make_uint4(~0u, ~0u, ~0u, ~0u);
     }
-    if (any != 0 && r < kRounds) mine |= 1ull << r;
-    if (r + 1u == rounds) break;  // kk keeps the last round's keys
 #pragma unroll
-    for (uint32_t q = 0; q < 4 * kVecs; ++q) kk[q] = kn[q];
+    for (uint32_t q = 0; q < KEEP; ++q) {
+      if (v0 + q * T >= v1) break;
+      const uint32_t v = v0 + q * T + t, e = 4u * v - off;
+      if (v == v0 || v + 1u == v1) {  // keys of the neighbouring segments in the end vectors
+        if (e >= n) kept[q].x = ~0u;
+        if (e + 1u >= n) kept[q].y = ~0u;
+        if (e + 2u >= n) kept[q].z = ~0u;
+        if (e + 3u >= n) kept[q].w = ~0u;
+      }
+      count(kept[q].x);
+      count(kept[q].y);
+      count(kept[q].z);
+      count(kept[q].w);
+    }
+  } else {
+    loadv(0u, kk);
+    for (uint32_t r = 0; r < rounds; ++r) {
+      // the next round's keys are requested before this round's are counted
+      uint32_t kn[4 * kVecs];
+      if (r + 1u < rounds) loadv(r + 1u, kn);
+      uint64_t any = 0;
+#pragma unroll
+      for (uint32_t q = 0; q < 4 * kVecs; ++q) {
+        any |= __ballot(kk[q] - key0 < nc);
+        count(kk[q]);
+      }
+      if (any != 0 && r < kRounds) mine |= 1ull << r;
+      if (r + 1u == rounds) break;  // kk keeps the last round's keys
+#pragma unroll
+      for (uint32_t q = 0; q < 4 * kVecs; ++q) kk[q] = kn[q];
+    }
   }
   below = wave_sum(below);
   if (lane == 0u) s.red[0][w] = below;
@@ -353,24 +391,40 @@ __global__ __launch_bounds__(T, 8) void k_cell_sort(CellSortArgs a, const Replic
       s.padded[t] = 0u;
       list[have + t] = 0xFFFFFFFFu;
     }
-    bool ready = false;  // kk holds the round's keys (the last round's are still there)
-    while (mine) {
-      const uint32_t r = 63u - (uint32_t)__clzll((long long)mine);
-      mine &= ~(1ull << r);
-      uint32_t kn[4 * kVecs];
-      if (r + 1u != rounds && !ready) loadv(r, kk);
-      if (mine) loadv(63u - (uint32_t)__clzll((long long)mine), kn);
+    if (keeps) {
+      auto place = [&](uint32_t key, uint32_t idx) __attribute__((always_inline)) {
+        const uint32_t c = key - key0;
+        if (c < nc) list[atomicAdd(&s.hist[c], 1u)] = (c << kIndexBits) | idx;
+      };
 #pragma unroll
-      for (uint32_t q = 0; q < 4 * kVecs; ++q) {
-        const uint32_t c = kk[q] - key0;
-        if (c < nc)
-          list[atomicAdd(&s.hist[c], 1u)] =
-              (c << kIndexBits) |
-              (4u * (v0 + r * kVecRound + q / 4 * T + t) + q % 4 - off);
+      for (uint32_t q = 0; q < KEEP; ++q) {
+        if (v0 + q * T >= v1) break;
+        const uint32_t e = 4u * (v0 + q * T + t) - off;
+        place(kept[q].x, e);
+        place(kept[q].y, e + 1u);
+        place(kept[q].z, e + 2u);
+        place(kept[q].w, e + 3u);
       }
+    } else {
+      bool ready = false;  // kk holds the round's keys (the last round's are still there)
+      while (mine) {
+        const uint32_t r = 63u - (uint32_t)__clzll((long long)mine);
+        mine &= ~(1ull << r);
+        uint32_t kn[4 * kVecs];
+        if (r + 1u != rounds && !ready) loadv(r, kk);
+        if (mine) loadv(63u - (uint32_t)__clzll((long long)mine), kn);
 #pragma unroll
-      for (uint32_t q = 0; q < 4 * kVecs; ++q) kk[q] = kn[q];
-      ready = true;
+        for (uint32_t q = 0; q < 4 * kVecs; ++q) {
+          const uint32_t c = kk[q] - key0;
+          if (c < nc)
+            list[atomicAdd(&s.hist[c], 1u)] =
+                (c << kIndexBits) |
+                (4u * (v0 + r * kVecRound + q / 4 * T + t) + q % 4 - off);
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < 4 * kVecs; ++q) kk[q] = kn[q];
+        ready = true;
+      }
     }
     __syncthreads();
     for (uint32_t p0 = t; p0 < have; p0 += 4u * T) {
@@ -495,8 +549,10 @@ __global__ __launch_bounds__(T) void k_cell_sort_removed(const uint32_t* __restr
 hipError_t launch_cell_sort(const CellSortArgs& a, bool part, uint32_t workgroups, hipStream_t stream) {
   if (workgroups == 0) return hipSuccess;
   const dim3 grid(workgroups), blk(T);
-  if (part) hipLaunchKernelGGL(k_cell_sort<true>, grid, blk, 0, stream, a, a.tables, a.keys, a.src);
-  else hipLaunchKernelGGL(k_cell_sort<false>, grid, blk, 0, stream, a, a.tables, a.keys, a.src);
+  if (part) hipLaunchKernelGGL((k_cell_sort<true, 0>), grid, blk, 0, stream, a, a.tables, a.keys, a.src);
+  else if (workgroups <= kKeepGroups)
+    hipLaunchKernelGGL((k_cell_sort<false, kKeepVecs>), grid, blk, 0, stream, a, a.tables, a.keys, a.src);
+  else hipLaunchKernelGGL((k_cell_sort<false, 0>), grid, blk, 0, stream, a, a.tables, a.keys, a.src);
   return hipGetLastError();
 }
 
