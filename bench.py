@@ -54,27 +54,30 @@ def log(msg):
 PACKED_INDEX_MAX = 1 << 27
 
 
-def stage_bytes(name, n, S, nb, passes, packed=True):
+def stage_bytes(name, n, S, nb, passes, packed=True, form="digits"):
     """Algorithmic bytes of one launch of each stage for n particles, S RNG
-    streams, nb buckets (compulsory reads + writes, each datum once)."""
+    streams, nb buckets (compulsory reads + writes, each datum once).  form:
+    the sort's ("replica" or "bins": the counting sort, which writes the cell
+    table too; "digits": digit passes and a pass for the table)."""
     if name == "producer":
         # record (x, y, z, type) 16 in; record 16, key 4 out (birth type and position only at
         # births); stream state
         return 36 * n + 172 * S
+    if name == "sort" and form != "digits":
+        # keys 4 in; key 4 and record 16 + 16 in sorted order (the particle's index in the record, or
+        # as a value of its own); the table; bins: one digit pass before (count 4, scatter 4 in, 8 out)
+        # and values 4 in
+        return 40 * n + (0 if packed else 4 * n) + 4 * (nb + 1) + (20 * n if form == "bins" else 0)
     if name == "sort":
         # per digit pass: count (key 4) + scatter (key, value 8 in, 8 out); first pass values implicit;
         # the last pass also copies the packed record of each particle into sorted order (16 + 16),
         # with the particle's index in the record instead of a sorted value written (4 less)
         return 20 * n * passes - 4 * n + 32 * n - (4 * n if packed else 0)
-    if name == "first":
+    if name == "first" and form == "digits":
         return 4 * (nb + 1) + 4 * n
     if name == "candidates":
         return 24 * n
-    if name == "resolve":
-        return 4 * n
-    if name == "scatter":
-        # record 16 + fourth component 4 in, the same out (birth types only in tiles with births)
-        return 40 * n
+    # pairs, bookkeeping and the particles gained: a few records
     return 0
 
 
@@ -126,8 +129,7 @@ def timed(e, steps):
 
 
 # stages that are one kernel each, and that kernel's name in the profiles
-SINGLE_KERNEL = {"producer": "k_producer", "first": "k_first", "candidates": "k_candidates", "resolve": "k_resolve",
-                 "scatter": "k_scatter"}
+SINGLE_KERNEL = {"producer": "k_producer", "first": "k_first", "candidates": "k_candidates", "resolve": "k_resolve"}
 PROFILE = {"c2": "step_kernels_c2_1M.md", "c3": "step_kernels_c3_4M.md", "c4": "step_kernels_c4_9M.md",
            "c5": "step_kernels_c5_mix8.md"}
 SERVING_RESIDENT = 8  # jobs resident in the serving engine's measured mix
@@ -159,7 +161,7 @@ def stage_graph_bytes(e, steps, ps):
     return n * (140 + 16 * P) + 12 * lay["total_buckets"] + 336 * lay["total_streams"]
 
 
-def roofline(e, cfg, nprof=5, streams=None, buckets=None):
+def roofline(e, cfg, nprof=5, streams=None, buckets=None, algo=1):
     """Per-stage HIP-event times of `nprof` eager steps (on the engine's
     stream) and the dominant single kernel's roofline.  streams / buckets:
     the streams and buckets in use when they are fewer than the engine's
@@ -170,10 +172,15 @@ def roofline(e, cfg, nprof=5, streams=None, buckets=None):
     S = streams if streams is not None else lay["total_streams"]
     nb = buckets if buckets is not None else lay["total_buckets"]
     passes = e.sort_plan()[0]  # two for an ensemble sorted replica by replica
+    # the form the engine takes for these workloads: slots and other digit widths sort by digits,
+    # c2 and c3 by bins
+    form = {"c2": "bins", "c3": "bins"}.get(cfg, "replica")
+    if streams is not None or e.radix_bits() != 8 or algo == 0:
+        form = "digits"
     packed = lay["capacity"] <= PACKED_INDEX_MAX
     rows = {}
     for k, us in prof.items():
-        b = stage_bytes(k, n, S, nb, passes, packed)
+        b = stage_bytes(k, n, S, nb, passes, packed, form)
         rows[k] = dict(us=us, bytes=b, gbs=(b / (us * 1e-6) / 1e9) if us > 0 else 0.0)
     dom = max((k for k in rows if k in SINGLE_KERNEL), key=lambda k: rows[k]["us"])
     step_us = sum(r["us"] for r in rows.values())
@@ -182,7 +189,7 @@ def roofline(e, cfg, nprof=5, streams=None, buckets=None):
     # the kernels with a launch-shape knob are templates on their block size
     kname = SINGLE_KERNEL[dom]
     if dom == "producer":
-        kname += f"<{e.get_knob(smd.KNOB_PRODUCER_BLOCK)}>"
+        kname += f"<{e.get_knob(smd.KNOB_PRODUCER_BLOCK)}, false>"  # fourth components in the records
     elif dom == "candidates":
         kname += f"<{e.get_knob(smd.KNOB_PAIR_BLOCK)}>"
     traffic, prof_us, prof_file = profiled_traffic(cfg, kname)
@@ -488,7 +495,7 @@ def c5_line(args):
 
 
 def base_line(cfg, args, e, steps, ps, secs, desc):
-    rl, step = roofline(e, cfg)
+    rl, step = roofline(e, cfg, algo=args.sort)
     out = {
         "metric": METRIC,
         "value": ps / secs,

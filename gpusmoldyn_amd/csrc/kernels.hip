@@ -2,9 +2,11 @@
 //
 // One step over an ensemble of R >= 1 replicas (a plain simulation is R = 1):
 //   k_producer    diffuse + unimolecular reactions + boundaries + hash   (one thread per RNG stream)
-//   k_sort_*      stable LSD radix sort of (bucket key, particle index); the last digit pass
-//                 also copies each particle's (x, y, z, type) record into sorted order
-//   k_first       lower bound of every bucket in the sorted keys
+//   k_cell_sort   (cellsort.hip) records sorted by bucket and the lower bound of every bucket;
+//                 for one large system behind one k_sort_* pass over the keys' high bits
+//   k_sort_*      for slot engines and other digit widths: stable LSD radix sort of (bucket key,
+//                 particle index); the last digit pass also copies each particle's record into
+//                 sorted order, and k_first finds the lower bound of every bucket
 //   k_candidates  neighbour-cell search for each particle's nearest reactive partner
 //   k_resolve     mutual-nearest pairs react (bimReact)                (one thread per RNG stream)
 //   k_finalize    per-replica counts and offsets, the sorted list of removed particles
