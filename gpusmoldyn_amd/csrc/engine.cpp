@@ -1318,6 +1318,10 @@ smd_status Engine::particle_steps(unsigned long long* out) {
 }
 
 smd_status Engine::counts(uint32_t* out) {
+  if (R && !finalized) {  // finalize failed: no count has been published
+    set_error("engine not finalized");
+    return SMD_ERR_INVALID;
+  }
   smd_status st = sync();
   if (st != SMD_OK) return st;
   if (count_known()) {
@@ -1357,6 +1361,10 @@ smd_status Engine::view_buffers(uint32_t n) {
 smd_status Engine::get(int r, float* pos4, int* types, uint32_t capN, uint32_t* nOut) {
   if (r < 0 || (uint32_t)r >= R) {
     set_error("replica id out of range");
+    return SMD_ERR_INVALID;
+  }
+  if (!finalized) {  // finalize failed after it had set R
+    set_error("engine not finalized");
     return SMD_ERR_INVALID;
   }
   const bool wants = capN && (pos4 || types);
