@@ -1367,6 +1367,7 @@ smd_status Engine::get(int r, float* pos4, int* types, uint32_t capN, uint32_t* 
     set_error("engine not finalized");
     return SMD_ERR_INVALID;
   }
+  std::lock_guard<std::mutex> lock(readMutex);
   const bool wants = capN && (pos4 || types);
   uint32_t n = 0;
   if (wants && lastN[r] <= stageCap) {

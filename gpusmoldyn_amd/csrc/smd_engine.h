@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <vector>
 
 #include "smd_kernels.h"
@@ -102,6 +103,7 @@ class Engine {
   uint32_t stageCap = 0;
   char* stage = nullptr;            // the allocation behind them
   std::vector<uint32_t> lastN;      // per replica: a recent count (which way get() takes)
+  std::mutex readMutex;             // several threads may read: one at a time uses this memory
   uint32_t* dHostStatus = nullptr;  // its device address
   // order-0 creation: one stream per replica, a per-step creation buffer
   uint32_t *dZMt = nullptr, *dZPar = nullptr, *dZCount = nullptr, *dZeroBase = nullptr;
