@@ -1348,16 +1348,6 @@ ExportArgs Engine::export_args(int r) const {
   return a;
 }
 
-smd_status Engine::view_buffers(uint32_t n) {
-  if (n <= viewCap && dViewPos) return SMD_OK;
-  dfree(dViewPos);
-  dfree(dViewType);
-  viewCap = std::max<uint32_t>(n, 1u);
-  HIPCHK(dalloc(&dViewPos, viewCap));
-  HIPCHK(dalloc(&dViewType, viewCap));
-  return SMD_OK;
-}
-
 smd_status Engine::get(int r, float* pos4, int* types, uint32_t capN, uint32_t* nOut) {
   if (r < 0 || (uint32_t)r >= R) {
     set_error("replica id out of range");
@@ -1399,16 +1389,18 @@ smd_status Engine::get(int r, float* pos4, int* types, uint32_t capN, uint32_t* 
   if (nOut) *nOut = n;
   const uint32_t m = std::min(n, capN);
   if (!m || !wants) return SMD_OK;
-  st = view_buffers(m);
-  if (st != SMD_OK) return st;
+  // into memory that only steps use: the other canonical buffer and, for the
+  // types, the sorted records (not the view, which its caller may still hold)
+  float4* const outPos = dPT[cur ^ 1];
+  int* const outType = (int*)dSortedPT;
   ExportArgs a = export_args(r);
   a.cap = m;
-  a.pos4 = pos4 ? dViewPos : nullptr;
-  a.types = types ? dViewType : nullptr;
+  a.pos4 = pos4 ? outPos : nullptr;
+  a.types = types ? outType : nullptr;
   HIPCHK(launch_export(a, m, stream));
   HIPCHK(hipStreamSynchronize(stream));
-  if (pos4) HIPCHK(hipMemcpy(pos4, dViewPos, m * sizeof(float4), hipMemcpyDeviceToHost));
-  if (types) HIPCHK(hipMemcpy(types, dViewType, m * sizeof(int), hipMemcpyDeviceToHost));
+  if (pos4) HIPCHK(hipMemcpy(pos4, outPos, m * sizeof(float4), hipMemcpyDeviceToHost));
+  if (types) HIPCHK(hipMemcpy(types, outType, m * sizeof(int), hipMemcpyDeviceToHost));
   return SMD_OK;
 }
 
@@ -1421,8 +1413,13 @@ smd_status Engine::view(float4** pos4, int** types, uint32_t* nOut) {
   if (st != SMD_OK) return st;
   uint32_t n = 0;
   HIPCHK(hipMemcpy(&n, dN, sizeof(uint32_t), hipMemcpyDeviceToHost));
-  st = view_buffers(n);
-  if (st != SMD_OK) return st;
+  if (n > viewCap || !dViewPos) {
+    dfree(dViewPos);
+    dfree(dViewType);
+    viewCap = std::max<uint32_t>(n, 1u);
+    HIPCHK(dalloc(&dViewPos, viewCap));
+    HIPCHK(dalloc(&dViewType, viewCap));
+  }
   ExportArgs a = export_args(-1);
   a.pos4 = dViewPos;
   a.types = dViewType;

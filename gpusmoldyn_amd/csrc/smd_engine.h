@@ -187,7 +187,6 @@ class Engine {
   ProducerArgs producer_args() const;
   ExportArgs export_args(int r) const;
   smd_status set_dense();
-  smd_status view_buffers(uint32_t n);
   smd_status alloc_stage();
   float4* dStagePos = nullptr;
   int* dStageType = nullptr;
