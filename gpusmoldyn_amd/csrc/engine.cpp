@@ -702,6 +702,7 @@ smd_status Engine::step_graph(int pairs) {
     }
     HIPCHK(hipGraphLaunch(gexec[p], stream));
     // two steps: every ping-pong selection is back where it was
+    std::fill(slotPending.begin(), slotPending.end(), (uint8_t)0);
     stepsDone += 2;
     Nub = std::min<uint64_t>(step_bound(step_bound(Nub)), (uint64_t)cap);
   }
