@@ -1485,6 +1485,10 @@ smd_status Engine::debug_stage(int stage, float* pos4, int* types, uint32_t* key
   }
   if (stage >= 4) HIPCHK(launch_resolve(resolve_args(), stream));
   HIPCHK(hipStreamSynchronize(stream));
+  // no finalize kernel ran to copy the error bits
+  uint32_t bits = 0;
+  HIPCHK(hipMemcpy(&bits, dStatus, sizeof(uint32_t), hipMemcpyDeviceToHost));
+  __atomic_store_n(hostStatus, bits, __ATOMIC_RELEASE);
   if (stage >= 2) HIPCHK(hipMemcpy(&live, dLive, sizeof(uint32_t), hipMemcpyDeviceToHost));
   if (nTotal) *nTotal = n;
   if (nLive) *nLive = live;
