@@ -211,8 +211,16 @@ smd_status Engine::alloc_particle_buffers(uint32_t c) {
   return SMD_OK;
 }
 
+// Both arrays or none: the kernels tell by the pointers whether components
+// live apart.
 smd_status Engine::alloc_apart() {
-  for (int k = 0; k < 2; ++k) HIPCHK(dalloc(&dW[k], (size_t)cap + extraCap));
+  float* w[2] = {nullptr, nullptr};
+  hipError_t e = hipSuccess;
+  for (int k = 0; k < 2 && e == hipSuccess; ++k) e = dalloc(&w[k], (size_t)cap + extraCap);
+  if (e != hipSuccess)
+    for (float*& x : w) dfree(x);
+  HIPCHK(e);
+  for (int k = 0; k < 2; ++k) dW[k] = w[k];
   return SMD_OK;
 }
 
