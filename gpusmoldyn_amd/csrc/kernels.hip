@@ -1617,63 +1617,71 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
 
 // ---------------------------------------------------------------------------
 // Births go behind their replica's survivors in parent index order (the order
-// of compactPosAndTypeD, particles_kernel.cu:97-123).  A wave looks after 16
-// tiles and reads the birth types of those with births.
+// of compactPosAndTypeD, particles_kernel.cu:97-123).  A wave looks after a
+// tile: without births it reads one word, otherwise the tile's birth types.
+// Bound by latency, so the tile's records are requested together, before the
+// first is placed.  us with births of 0 / 0.1% / 5% / 25% of the particles: 1M
+// 4.3 / 8.4 / 13 / 13, 4M 4.3 / 13 / 30 / 36.  A wave for 16 tiles, each record
+// loaded where it is placed: 1M 4.3 / 31 / 125 / 124, 4M 4.3 / 36 / 166 / 178;
+// for 4 tiles, 1M 4.4 / 15 / 31 / 32.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kBirthTiles = 16;
-static_assert(kFinBlockTiles % kBirthTiles == 0, "a wave's tiles lie in one finalize block");
-
-__global__ __launch_bounds__(256) void k_births(BirthArgs a, const uint32_t* __restrict__ repOff) {
+__global__ __launch_bounds__(256) void k_births(BirthArgs a, const uint32_t* __restrict__ repOff,
+                                                const float4* __restrict__ addedPos) {
   const uint32_t n = *a.dN;
   const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t tile0 = (blockIdx.x * 4u + (threadIdx.x >> 6)) * kBirthTiles;
-  if (tile0 >= (n + kCompactTile - 1u) / kCompactTile) return;
-  const uint32_t mine = lane < kBirthTiles && (tile0 + lane) * kCompactTile < n ? a.tileBirth[tile0 + lane] : 0u;
-  uint64_t some = __ballot(mine != 0u);
-  if (some == 0) return;
-  uint32_t base = 0;
-  for (uint32_t q = lane; q < tile0 / kFinBlockTiles; q += 64) base += a.blockSum[q];
-  base = wave_sum(base);
-  const uint64_t lt = lanemask_lt();
+  const uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6);
+  const uint32_t e0 = tile * kCompactTile;
+  if (e0 >= n || a.tileBirth[tile] == 0u) return;
   constexpr int kItems = kCompactTile / 64;
-  while (some) {
-    const uint32_t tile = tile0 + (uint32_t)__ffsll((unsigned long long)some) - 1u;
-    some &= some - 1u;
-    uint32_t rank = base + a.tileBirthPre[tile];
-    const uint32_t e0 = tile * kCompactTile;
-    int bt[kItems];
+  int bt[kItems];
 #pragma unroll
-    for (int it = 0; it < kItems; ++it) {
-      const uint32_t e = e0 + it * 64 + lane;
-      bt[it] = e < n ? a.birthType[e] : 0;
-    }
-    // replica of the tile's first slot (last r with repOff[r] <= e0); the
-    // lanes move forward from there
-    int r = 0;
-    {
-      int hi = a.R;
-      while (hi - r > 1) {
-        const int mid = (r + hi) >> 1;
-        if (repOff[mid] <= e0) r = mid;
-        else hi = mid;
-      }
-    }
+  for (int it = 0; it < kItems; ++it) {
+    const uint32_t e = e0 + it * 64 + lane;
+    bt[it] = e < n ? a.birthType[e] : 0;
+  }
+  float4 rec[kItems];
 #pragma unroll
-    for (int it = 0; it < kItems; ++it) {
-      const uint64_t bm = __ballot(bt[it] > 0);
-      if (bt[it] > 0) {
-        const uint32_t e = e0 + it * 64 + lane;
-        while (r + 1 < a.R && repOff[r + 1] <= e) ++r;
-        const uint32_t dst = a.extraOff[r] + rank + (uint32_t)__popcll(bm & lt) - a.birthBase[r];
-        const float4 q = a.addedPos[e];
-        a.extra[dst] = make_float4(q.x, q.y, q.z, __int_as_float((a.extraW ? 0 : __float_as_int(q.w)) | bt[it]));
-        if (a.extraW) a.extraW[dst] = q.w;
-        a.birthType[e] = 0;  // taken: zero again for the next step
-      }
-      rank += (uint32_t)__popcll(bm);
+  for (int it = 0; it < kItems; ++it)
+    if (bt[it] > 0) rec[it] = addedPos[e0 + it * 64 + lane];
+  // births of earlier tiles
+  uint32_t rank = 0;
+  for (uint32_t q = lane; q < tile / kFinBlockTiles; q += 64) rank += a.blockSum[q];
+  rank = wave_sum(rank) + a.tileBirthPre[tile];
+  // replica of the tile's first slot (last r with repOff[r] <= e0); the lanes
+  // move forward from there
+  int r = 0;
+  {
+    int hi = a.R;
+    while (hi - r > 1) {
+      const int mid = (r + hi) >> 1;
+      if (repOff[mid] <= e0) r = mid;
+      else hi = mid;
     }
   }
-  if (mine) a.tileBirth[tile0 + lane] = 0;
+  uint32_t next = r + 1 < a.R ? repOff[r + 1] : 0xFFFFFFFFu;
+  uint32_t to = a.extraOff[r] - a.birthBase[r];
+  const uint64_t lt = lanemask_lt();
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) {
+    const uint64_t bm = __ballot(bt[it] > 0);
+    if (bt[it] > 0) {
+      const uint32_t e = e0 + it * 64 + lane;
+      if (next <= e) {
+        do {
+          ++r;
+          next = r + 1 < a.R ? repOff[r + 1] : 0xFFFFFFFFu;
+        } while (next <= e);
+        to = a.extraOff[r] - a.birthBase[r];
+      }
+      const uint32_t dst = to + rank + (uint32_t)__popcll(bm & lt);
+      const float4 q = rec[it];
+      a.extra[dst] = make_float4(q.x, q.y, q.z, __int_as_float((a.extraW ? 0 : __float_as_int(q.w)) | bt[it]));
+      if (a.extraW) a.extraW[dst] = q.w;
+      a.birthType[e] = 0;  // taken: zero again for the next step
+    }
+    rank += (uint32_t)__popcll(bm);
+  }
+  if (lane == 0) a.tileBirth[tile] = 0u;
 }
 
 // Where particle il of replica r is (CanonMap).
@@ -2687,8 +2695,8 @@ hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t stream) {
 
 hipError_t launch_births(const BirthArgs& a, uint32_t maxN, hipStream_t stream) {
   if (maxN == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_births, dim3(cdiv(cdiv(maxN, kCompactTile), 4 * kBirthTiles)), dim3(256), 0, stream, a,
-                     a.repOff);
+  hipLaunchKernelGGL(k_births, dim3(cdiv(cdiv(maxN, kCompactTile), 4)), dim3(256), 0, stream, a,
+                     a.repOff, a.addedPos);
   return hipGetLastError();
 }
 
