@@ -199,7 +199,8 @@ smd_status Engine::alloc_particle_buffers(uint32_t c) {
   HIPCHK(dalloc(&dHoles, cap));
   HIPCHK(dalloc(&dTileBirth, nTilesCap));
   HIPCHK(dalloc(&dTileBirthPre, nTilesCap));
-  HIPCHK(dalloc(&dBlockSum, finalize_blocks(nTilesCap * kCompactTile)));
+  finBlockTiles = finalize_block_tiles(nTilesCap);
+  HIPCHK(dalloc(&dBlockSum, (size_t)nTilesCap / finBlockTiles + 1));
   if (segHigh) HIPCHK(dalloc(&dSegScratch, seg_sort_words(cap, (int)R, std::max(segLow, segHigh))));
   HIPCHK(hipMemsetAsync(dDeadBits, 0, words * sizeof(uint32_t), stream));
   for (int k = 0; k < 2; ++k) {
@@ -1002,6 +1003,7 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
   fa.injBase = dInjBase;
   fa.retire = dRetire;
   fa.blockSum = dBlockSum;
+  fa.blockTiles = finBlockTiles;
   fa.tilesCap = nTilesCap;
   HIPCHK(launch_finalize(fa, stream));
   mark(6);
@@ -1019,6 +1021,7 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
     ba.birthType = dBirthType;
     ba.tileBirth = dTileBirth;
     ba.blockSum = dBlockSum;
+    ba.blockTiles = finBlockTiles;
     ba.extra = extra;
     ba.extraW = extraW;
     HIPCHK(launch_births(ba, maxN, stream));

@@ -1490,23 +1490,42 @@ __device__ __forceinline__ void block_exscan1024_k(const uint32_t (&v)[K], uint3
 
 // ---------------------------------------------------------------------------
 // Finalize: per-step bookkeeping after the pair step.  The removed particles
-// stay where they are; the next step reads around them (CanonMap).  Workgroup
-// g turns the death bits of tiles [g * 1024, (g + 1) * 1024) into their part
-// of the sorted hole list (its place: the deaths of all earlier tiles), clears
-// them, and scans the tiles' births.  Workgroup 0 also lays out every
-// replica's particles for the next step and publishes the step's counts.
+// stay where they are; the next step reads around them (CanonMap).  A
+// workgroup turns the death bits of its tiles into their part of the sorted
+// hole list (its place: the deaths of all earlier tiles), clears them, and
+// scans the tiles' births.  Workgroup 0 also lays out every replica's
+// particles for the next step and publishes the step's counts.
+//
+// With few deaths it is the latency of a launch and of workgroup 0's chain of
+// loads; with many, the list's scattered writes, so these are spread over
+// sixteen threads a tile and a workgroup takes 64 tiles at a time: us at 1M
+// particles with 0.1% / 5% / 25% / 45% of them removed 10 / 9 / 15 / 22, at 4M
+// 12 / 13 / 26 / 40; a thread per tile and 1024 tiles per workgroup took 17 /
+// 41 / 143 / 248 and 18 / 42 / 148 / 257.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kFinBlockTiles = 1024;
+constexpr uint32_t kFinTiles = 64;                      // tiles at a time
+constexpr uint32_t kFinParts = 1024 / kFinTiles;        // threads per tile
+constexpr uint32_t kFinWords = kCompactTile / 32 / kFinParts;  // death words per thread
+static_assert(kFinWords == 2, "a thread reads its death words at once");
+// Every workgroup adds up the deaths of all tiles before its own, so beyond
+// this many workgroups they take more tiles each instead (MANY).
+constexpr uint32_t kFinBlocks = 512;
 
+template <bool MANY>
 __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
   __shared__ uint32_t wsum[4][16];
   __shared__ uint32_t s_base[16];
-  const uint32_t t0 = blockIdx.x * kFinBlockTiles;
-  const uint32_t e = t0 + threadIdx.x;
+  const uint32_t tiles = MANY ? a.blockTiles : kFinTiles;
+  const uint32_t t0 = blockIdx.x * tiles, t1 = min(t0 + tiles, a.tilesCap);
   // every load that does not need another one's result is issued first
   const uint32_t n = *a.dN;
-  const uint32_t dead = e < a.tilesCap ? a.deaths.tileDead[e] : 0u;
-  const uint32_t born = a.tileBirth && e < a.tilesCap ? a.tileBirth[e] : 0u;
+  const uint32_t part = threadIdx.x % kFinParts;
+  uint32_t tile = t0 + threadIdx.x / kFinParts, dead = 0, born = 0;
+  auto load_counts = [&]() __attribute__((always_inline)) {
+    dead = tile < t1 ? a.deaths.tileDead[tile] : 0u;  // 0 where no particles are
+    born = a.tileBirth && tile < t1 && part == 0u ? a.tileBirth[tile] : 0u;
+  };
+  load_counts();
   uint32_t stepPrev = 0, status = 0, pairs = 0, acting = 0;
   unsigned long long psPrev = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -1518,10 +1537,8 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
       acting = *a.candActing;
     }
   }
-  if (e < a.tilesCap) a.tileDeadNext[e] = 0u;
+  for (uint32_t q = t0 + threadIdx.x; q < t1; q += 1024u) a.tileDeadNext[q] = 0u;
   if (blockIdx.x > 0 && t0 >= (n + kCompactTile - 1u) / kCompactTile) return;  // no particles here
-  uint32_t before = 0;
-  for (uint32_t q = threadIdx.x; q < t0; q += 1024u) before += a.deaths.tileDead[q];
   if (blockIdx.x == 0) {
     // replicas
     uint32_t c[4] = {0u, 0u, 0u, 0u};
@@ -1578,41 +1595,39 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
                          __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
-  if (!__syncthreads_or((dead | born) != 0u)) {
-    if (a.tileBirth && threadIdx.x == 0) a.blockSum[blockIdx.x] = 0u;
-    return;
-  }
-  uint4 x[kCompactTile / 128];
-  if (dead) {
-    uint4* const bits = (uint4*)(a.deaths.bits + (size_t)e * (kCompactTile / 32));
-#pragma unroll
-    for (int q = 0; q < kCompactTile / 128; ++q) x[q] = bits[q];
-#pragma unroll
-    for (int q = 0; q < kCompactTile / 128; ++q) bits[q] = make_uint4(0u, 0u, 0u, 0u);
-  }
-  before = wave_sum(before);
-  if ((threadIdx.x & 63u) == 0u) s_base[threadIdx.x >> 6] = before;
-  const uint32_t v[2] = {dead, born};
-  uint32_t ex[2], tot[2];
-  block_exscan1024_k<2>(v, ex, tot, wsum);
-  if (dead) {
-    uint32_t at = ex[0];
-#pragma unroll
-    for (uint32_t q = 0; q < 16u; ++q) at += s_base[q];
-#pragma unroll
-    for (int q = 0; q < kCompactTile / 128; ++q) {
-      const uint32_t w[4] = {x[q].x, x[q].y, x[q].z, x[q].w};
-#pragma unroll
-      for (uint32_t k = 0; k < 4u; ++k) {
-        for (uint32_t m = w[k]; m; m &= m - 1u)
-          a.holes[at++] = e * kCompactTile + q * 128u + k * 32u + (uint32_t)__ffs((int)m) - 1u;
-      }
+  uint32_t c[2] = {0u, 0u};  // deaths and births so far, of this workgroup
+  bool placed = false;       // c[0] counts the earlier workgroups' deaths too
+  for (uint32_t tb = t0; tb < t1; tb = MANY ? tb + kFinTiles : t1, tile += kFinTiles) {
+    if (MANY && tb != t0) load_counts();
+    if (!__syncthreads_or((dead | born) != 0u)) continue;
+    uint2 x = make_uint2(0u, 0u);
+    if (dead) {
+      uint2* const bits = (uint2*)(a.deaths.bits + (size_t)tile * (kCompactTile / 32)) + part;
+      x = *bits;
+      *bits = make_uint2(0u, 0u);
     }
+    if (!placed) {
+      uint32_t before = 0;
+      for (uint32_t q = threadIdx.x; q < t0; q += 1024u) before += a.deaths.tileDead[q];
+      before = wave_sum(before);
+      if ((threadIdx.x & 63u) == 0u) s_base[threadIdx.x >> 6] = before;
+      __syncthreads();
+#pragma unroll
+      for (uint32_t q = 0; q < 16u; ++q) c[0] += s_base[q];
+      placed = true;
+    }
+    const uint32_t v[2] = {(uint32_t)__popc(x.x) + (uint32_t)__popc(x.y), born};
+    uint32_t ex[2], tot[2];
+    block_exscan1024_k<2>(v, ex, tot, wsum);
+    uint32_t at = c[0] + ex[0];
+    const uint32_t slot0 = tile * kCompactTile + part * (32u * kFinWords);
+    for (uint32_t m = x.x; m; m &= m - 1u) a.holes[at++] = slot0 + (uint32_t)__ffs((int)m) - 1u;
+    for (uint32_t m = x.y; m; m &= m - 1u) a.holes[at++] = slot0 + 32u + (uint32_t)__ffs((int)m) - 1u;
+    if (a.tileBirth && tile < t1 && part == 0u) a.tileBirthPre[tile] = c[1] + ex[1];
+    c[0] += tot[0];
+    c[1] += tot[1];
   }
-  if (a.tileBirth) {
-    if (e < a.tilesCap) a.tileBirthPre[e] = ex[1];
-    if (threadIdx.x == 0) a.blockSum[blockIdx.x] = tot[1];
-  }
+  if (a.tileBirth && threadIdx.x == 0) a.blockSum[blockIdx.x] = c[1];
 }
 
 // ---------------------------------------------------------------------------
@@ -1645,7 +1660,7 @@ __global__ __launch_bounds__(256) void k_births(BirthArgs a, const uint32_t* __r
     if (bt[it] > 0) rec[it] = addedPos[e0 + it * 64 + lane];
   // births of earlier tiles
   uint32_t rank = 0;
-  for (uint32_t q = lane; q < tile / kFinBlockTiles; q += 64) rank += a.blockSum[q];
+  for (uint32_t q = lane; q < tile / a.blockTiles; q += 64) rank += a.blockSum[q];
   rank = wave_sum(rank) + a.tileBirthPre[tile];
   // replica of the tile's first slot (last r with repOff[r] <= e0); the lanes
   // move forward from there
@@ -2683,13 +2698,15 @@ hipError_t launch_resolve(const ResolveArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-uint32_t finalize_blocks(uint32_t capacity) {
-  return std::max<uint32_t>(1u, cdiv(cdiv(capacity, kCompactTile), kFinBlockTiles));
+uint32_t finalize_block_tiles(uint32_t tiles) {
+  return kFinTiles * std::max(1u, cdiv(cdiv(tiles, kFinTiles), kFinBlocks));
 }
 
 hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t stream) {
   // over all tiles of the capacity: the other parity's counts are cleared
-  hipLaunchKernelGGL(k_finalize, dim3(std::max(1u, cdiv(a.tilesCap, kFinBlockTiles))), dim3(1024), 0, stream, a);
+  const dim3 grid(std::max(1u, cdiv(a.tilesCap, a.blockTiles))), blk(1024);
+  if (a.blockTiles == kFinTiles) hipLaunchKernelGGL(k_finalize<false>, grid, blk, 0, stream, a);
+  else hipLaunchKernelGGL(k_finalize<true>, grid, blk, 0, stream, a);
   return hipGetLastError();
 }
 

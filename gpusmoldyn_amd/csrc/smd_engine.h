@@ -91,7 +91,8 @@ class Engine {
   uint32_t* dDeadBits = nullptr;                // a bit per slot removed in this step
   uint32_t* dTileDead[2] = {nullptr, nullptr};  // removed per tile, one per step parity (cur)
   uint32_t *dTileBirth = nullptr, *dTileBirthPre = nullptr;
-  uint32_t* dBlockSum = nullptr;  // births per finalize block
+  uint32_t* dBlockSum = nullptr;  // births per finalize workgroup
+  uint32_t finBlockTiles = 0;     // its tiles
   uint32_t* dStatus = nullptr;    // sticky kernel error bits
   // host memory that kernels write: the error bits' copy (finalize kernel),
   // and particles read back a few at a time (get)

@@ -234,7 +234,8 @@ struct FinalizeArgs {
   uint32_t* injCount;      // per replica: particles admitted this step (nullptr: none); reset
   uint32_t* injBase;       // per replica: where its admitted particles go (from extraBase)
   uint32_t* retire;        // per replica retire flags (nullptr: none); reset
-  uint32_t* blockSum;      // births of each 1024-tile block
+  uint32_t* blockSum;      // births of each workgroup's tiles
+  uint32_t blockTiles;     // tiles per workgroup (finalize_block_tiles)
   uint32_t tilesCap;       // tiles of the allocated capacity
 };
 
@@ -272,6 +273,7 @@ struct BirthArgs {
   int* birthType;          // nonzero only at births; cleared as they are taken
   uint32_t* tileBirth;     // births per tile (producer); cleared here
   const uint32_t* blockSum;
+  uint32_t blockTiles;
   float4* extra;
   float* extraW;           // nullptr: in the records
 };
@@ -340,8 +342,8 @@ hipError_t launch_candidates(const CandArgs& a, uint32_t maxN, int blockSize, hi
 // Entries of CandList::list.
 size_t pair_list_size();
 hipError_t launch_resolve(const ResolveArgs& a, hipStream_t stream);
-// Finalize workgroups for a capacity (one per 1024 tiles).
-uint32_t finalize_blocks(uint32_t capacity);
+// Tiles per finalize workgroup when there are `tiles` of them.
+uint32_t finalize_block_tiles(uint32_t tiles);
 hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t stream);
 hipError_t launch_births(const BirthArgs& a, uint32_t maxN, hipStream_t stream);
 hipError_t launch_export(const ExportArgs& a, uint32_t maxN, hipStream_t stream);

@@ -83,3 +83,35 @@ def _stages(smd, n, p):
 def test_births_cost_less_than_the_move(smd, gpu):
     s = _stages(smd, 1 << 20, 0.05)
     assert s["scatter"] < 0.6 * s["producer"]
+
+
+@pytest.mark.parametrize("n", [65535, 65536, 65537, 200000])
+def test_holes_match_oracle(smd, orc, gpu, n):
+    """Around the 64 tiles that a bookkeeping workgroup takes; most particles
+    go in each step."""
+    print(f"holes, {n} particles", flush=True)
+    spec, pos, types = _system(smd, n, 0.3, 11)
+    spec.rxn[1].rate *= 0.2
+    _check(smd, orc, [(spec, pos, types)], 4)
+
+
+def test_many_tiles_per_workgroup(smd, orc, gpu):
+    """A capacity of more than 512 x 64 tiles: workgroups take several groups
+    of tiles each."""
+    print("holes, capacity 2^26", flush=True)
+    spec, pos, types = _system(smd, 150000, 0.2, 12)
+    e = smd.Engine(0)
+    e.add_replica(spec, pos, types)
+    e.finalize(1 << 26)
+    e.step(4)
+    gp, gt = e.get(0)
+    e.close()
+    sim = orc.sim_for(smd, spec, pos, types, cap=8 * len(types))
+    sim.step(smd.gauss_table(), 4)
+    rp, rt = sim.state()
+    assert np.array_equal(gt, rt) and np.array_equal(gp.view(np.uint32), rp.view(np.uint32))
+
+
+def test_holes_cost_less_than_the_move(smd, gpu):
+    s = _stages(smd, 1 << 20, 0.25)
+    assert s["finalize"] < 0.6 * s["producer"]
