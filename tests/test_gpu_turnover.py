@@ -115,3 +115,18 @@ def test_many_tiles_per_workgroup(smd, orc, gpu):
 def test_holes_cost_less_than_the_move(smd, gpu):
     s = _stages(smd, 1 << 20, 0.25)
     assert s["finalize"] < 0.6 * s["producer"]
+
+
+@pytest.mark.parametrize("n,p", [(4097, 0.5), (20000, 0.95), (20000, 0.995), (300, 1.0)])
+def test_most_particles_vanish(smd, orc, gpu, n, p):
+    """More holes than lanes between the particles of a wave."""
+    print(f"{n} particles, {p} of the C vanish", flush=True)
+    spec, pos, types = _system(smd, n, 0.25, 13)
+    spec.rxn[1].rate = 0.0
+    spec.rxn[2].rate = -math.log(max(1.0 - p, 1e-12)) / 1e-3
+    _check(smd, orc, [(spec, pos, types)], 3)
+
+
+def test_move_costs_the_same_with_many_holes(smd, gpu):
+    few, many = _stages(smd, 100000, 0.01), _stages(smd, 100000, 0.45)
+    assert many["producer"] < 1.6 * few["producer"]
