@@ -57,13 +57,13 @@ PACKED_INDEX_MAX = 1 << 27
 def stage_bytes(name, n, S, nb, passes, packed=True, form="digits"):
     """Algorithmic bytes of one launch of each stage for n particles, S RNG
     streams, nb buckets (compulsory reads + writes, each datum once).  form:
-    the sort's ("replica" or "bins": the counting sort, which writes the cell
-    table too; "digits": digit passes and a pass for the table)."""
+    the sort's ("replicas" or "bins": the counting sort, which writes the cell
+    table too; "digits" and "segments": digit passes and a pass for the table)."""
     if name == "producer":
         # record (x, y, z, type) 16 in; record 16, key 4 out (birth type and position only at
         # births); stream state
         return 36 * n + 172 * S
-    if name == "sort" and form != "digits":
+    if name == "sort" and form in ("replicas", "bins"):
         # keys 4 in; key 4 and record 16 + 16 in sorted order (the particle's index in the record, or
         # as a value of its own); the table; bins: one digit pass before (count 4, scatter 4 in, 8 out)
         # and values 4 in
@@ -73,7 +73,7 @@ def stage_bytes(name, n, S, nb, passes, packed=True, form="digits"):
         # the last pass also copies the packed record of each particle into sorted order (16 + 16),
         # with the particle's index in the record instead of a sorted value written (4 less)
         return 20 * n * passes - 4 * n + 32 * n - (4 * n if packed else 0)
-    if name == "first" and form == "digits":
+    if name == "first" and form in ("digits", "segments"):
         return 4 * (nb + 1) + 4 * n
     if name == "candidates":
         return 24 * n
@@ -161,7 +161,7 @@ def stage_graph_bytes(e, steps, ps):
     return n * (140 + 16 * P) + 12 * lay["total_buckets"] + 336 * lay["total_streams"]
 
 
-def roofline(e, cfg, nprof=5, streams=None, buckets=None, algo=1):
+def roofline(e, cfg, nprof=5, streams=None, buckets=None):
     """Per-stage HIP-event times of `nprof` eager steps (on the engine's
     stream) and the dominant single kernel's roofline.  streams / buckets:
     the streams and buckets in use when they are fewer than the engine's
@@ -172,11 +172,7 @@ def roofline(e, cfg, nprof=5, streams=None, buckets=None, algo=1):
     S = streams if streams is not None else lay["total_streams"]
     nb = buckets if buckets is not None else lay["total_buckets"]
     passes = e.sort_plan()[0]  # two for an ensemble sorted replica by replica
-    # the form the engine takes for these workloads: slots and other digit widths sort by digits,
-    # c2 and c3 by bins
-    form = {"c2": "bins", "c3": "bins"}.get(cfg, "replica")
-    if streams is not None or e.radix_bits() != 8 or algo == 0:
-        form = "digits"
+    form = e.sort_form()
     packed = lay["capacity"] <= PACKED_INDEX_MAX
     rows = {}
     for k, us in prof.items():
@@ -495,7 +491,7 @@ def c5_line(args):
 
 
 def base_line(cfg, args, e, steps, ps, secs, desc):
-    rl, step = roofline(e, cfg, algo=args.sort)
+    rl, step = roofline(e, cfg)
     out = {
         "metric": METRIC,
         "value": ps / secs,

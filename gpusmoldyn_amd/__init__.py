@@ -114,6 +114,7 @@ def lib():
         L.smd_engine_debug_stage.argtypes = [vp, ctypes.c_int, f32p, i32p, u32p, u32p, i32p,
                                              ctypes.POINTER(ctypes.c_uint), ctypes.POINTER(ctypes.c_uint)]
         L.smd_engine_layout.argtypes = [vp] + [ctypes.POINTER(ctypes.c_uint)] * 4
+        L.smd_engine_sort_form.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
         L.smd_engine_sort_plan.argtypes = [vp, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]
         L.smd_engine_profile_step.argtypes = [vp, ctypes.c_int, ctypes.POINTER(ctypes.c_double), ctypes.c_int,
                                               ctypes.c_char_p, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
@@ -351,6 +352,15 @@ class Engine:
 
     def radix_bits(self):
         return lib().smd_engine_radix_bits(self._h)
+
+    def sort_form(self):
+        """How the next step sorts its keys: "digits" (all keys), "segments"
+        (digits, replica by replica), "replicas" (keys counted per cell,
+        replica by replica) or "bins" (the same behind a digit pass over the
+        keys' high bits)."""
+        f = ctypes.c_int(0)
+        _check(lib().smd_engine_sort_form(self._h, ctypes.byref(f)), "smd_engine_sort_form")
+        return ("digits", "segments", "replicas", "bins")[f.value]
 
     def sort_plan(self):
         """(digit passes of the digit form of the step's key sort, True when it

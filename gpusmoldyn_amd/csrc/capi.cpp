@@ -341,6 +341,12 @@ smd_status smd_engine_layout(smd_engine* e, uint32_t* total_buckets, uint32_t* k
   return SMD_OK;
 }
 
+smd_status smd_engine_sort_form(const smd_engine* e, int* form) {
+  if (!e || !form || !e->impl->finalized) return SMD_ERR_INVALID;
+  *form = e->impl->form_now();
+  return SMD_OK;
+}
+
 smd_status smd_engine_sort_plan(const smd_engine* e, int* passes, int* segmented) {
   if (!e || !e->impl->finalized) return SMD_ERR_INVALID;
   const bool seg = e->impl->seg_sorted();

@@ -804,6 +804,14 @@ Engine::SortForm Engine::sort_form(uint32_t maxN) const {
   return cellBinBits ? SortForm::kCellsByBin : SortForm::kDigits;
 }
 
+smd_sort_form Engine::form_now() const {
+  switch (sort_form((uint32_t)std::max<uint64_t>(knownN, 1))) {
+    case SortForm::kCellsByReplica: return SMD_SORT_REPLICAS;
+    case SortForm::kCellsByBin: return SMD_SORT_BINS;
+    default: return seg_sorted() ? SMD_SORT_SEGMENTS : SMD_SORT_DIGITS;
+  }
+}
+
 hipError_t Engine::sort_keys(uint32_t maxN, bool tilesLaid, StageTimer* timer, bool debug) {
   const SortForm form = sort_form(maxN);
   hipError_t e;

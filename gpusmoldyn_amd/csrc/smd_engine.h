@@ -164,7 +164,8 @@ class Engine {
   // one replica's count is the total that the finalize kernel published
   // (after sync)
   bool count_known() const { return R == 1 && !slotsMode && lastSeen >= stepsDone; }
-  bool seg_sorted() const;  // this engine's step sorts replica by replica
+  bool seg_sorted() const;  // this engine's digit form sorts replica by replica
+  smd_sort_form form_now() const;
 
  private:
   smd_status enqueue_kernels(uint32_t maxN, StageTimer* timer);

@@ -238,10 +238,19 @@ smd_status smd_engine_debug_first(smd_engine* e, uint32_t* first, uint32_t cap, 
 /* Number of buckets (keys deadKey = total buckets) and key bits. */
 smd_status smd_engine_layout(smd_engine* e, uint32_t* total_buckets, uint32_t* key_bits, uint32_t* total_streams,
                              uint32_t* capacity);
+/* How the next step sorts its keys (every form gives the same order).  No
+ * counterpart in the reference. */
+typedef enum smd_sort_form {
+  SMD_SORT_DIGITS = 0,     /* digit passes over all keys */
+  SMD_SORT_SEGMENTS = 1,   /* two digit passes, replica by replica */
+  SMD_SORT_REPLICAS = 2,   /* keys counted per cell, replica by replica */
+  SMD_SORT_BINS = 3        /* keys counted per cell, behind a digit pass over their high bits */
+} smd_sort_form;
+smd_status smd_engine_sort_form(const smd_engine* e, int* form);
 /* The plan of the digit form of the step's key sort: *passes digit passes,
  * *segmented = 1 when each replica is sorted on its local cells
  * (SMD_KNOB_SEGMENTED_SORT applies), 0 for one sort over the global keys.
- * Where the step counts keys per cell instead, the order is the same.  No
+ * smd_engine_sort_form says whether the step takes the digit form.  No
  * counterpart in the reference. */
 smd_status smd_engine_sort_plan(const smd_engine* e, int* passes, int* segmented);
 /* Per-kernel timing of the last timed step (HIP events, microseconds):
