@@ -49,6 +49,9 @@ constexpr uint32_t kRound = T * kKeys;
 constexpr int kIndexBits = 32 - kCellSliceBits;       // list entry: cell << kIndexBits | index
 constexpr uint32_t kIndexMask = (1u << kIndexBits) - 1u;
 constexpr int kLow = 7, kHigh = kCellSliceBits - kLow;  // digits of the ordered path's passes over the list
+// About what a slice on the ordered path takes: this for each of its windows
+// (with the values to look up in bins), and 1 for each round over the keys.
+constexpr uint32_t kWindowHalfUs = 12, kWindowHalfUsBins = 15;
 // Cells of at most this many particles are put in order by comparing
 // neighbours in the list; a fuller one sends the slice to the ordered path.
 constexpr uint32_t kFew = 32;
@@ -459,8 +462,9 @@ __global__ __launch_bounds__(T, KEEP ? 2 : 8) void k_cell_sort(CellSortArgs a, c
   } else {
     // Windows of the segment whose keys fit the list, collected in index
     // order and put in cell order by stable digit passes.
-    uint32_t t0 = 0;
+    uint32_t t0 = 0, windows = 0;
     for (;;) {
+      ++windows;
       const uint32_t winBase = t0;
       uint32_t par = 0;
       have = 0;
@@ -516,6 +520,11 @@ __global__ __launch_bounds__(T, KEEP ? 2 : 8) void k_cell_sort(CellSortArgs a, c
         const uint32_t c = list[p] >> kIndexBits;
         if (p + 1u == have || (list[p + 1u] >> kIndexBits) != c) s.hist[c] += p + 1u;
       }
+    }
+    if (t == 0u) {
+      const uint32_t r = (n + kRound - 1u) / kRound;
+      atomicMax(&a.work[0], windows * (PART ? kWindowHalfUsBins : kWindowHalfUs) + r);
+      atomicAdd(&a.work[1], r);
     }
   }
   if (bad) atomicOr(a.status, kStatusSortLayout);

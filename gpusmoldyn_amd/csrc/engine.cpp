@@ -506,6 +506,8 @@ smd_status Engine::alloc_stage() {
   std::memset(stage, 0, head);
   hostStatus = (uint32_t*)stage;
   dHostStatus = (uint32_t*)dev;
+  hostSort = (unsigned long long*)(stage + 128);
+  dHostSort = (unsigned long long*)(dev + 128);
   stageHead = (uint32_t*)(stage + 64);
   dStageHead = (uint32_t*)(dev + 64);
   stagePos = (float4*)(stage + head);
@@ -566,6 +568,7 @@ smd_status Engine::grow(uint64_t need) {
 
 smd_status Engine::ensure_capacity() {
   refresh_bound(false);
+  watch_sort();
   const uint64_t needAfter = step_bound(Nub);
   if (needAfter <= cap) return SMD_OK;
   refresh_bound(true);
@@ -586,7 +589,8 @@ smd_status Engine::enqueue_step(StageTimer* timer) {
 void Engine::drop_graph(int which) {
   const int lo = which < 0 ? 0 : which, hi = which < 0 ? 1 : which;
   bool any = false;
-  for (int p = lo; p <= hi; ++p) any = any || gexec[p] || oneExec[p];
+  for (int f = 0; f < kForms; ++f)
+    for (int p = lo; p <= hi; ++p) any = any || gexec[f][p] || oneExec[f][p];
   if (!any) return;
   // A launch of the graph may still be queued or running: the executable
   // graph (and the kernel arguments it owns) must outlive it.
@@ -594,12 +598,13 @@ void Engine::drop_graph(int which) {
     (void)hipSetDevice(device);
     (void)hipStreamSynchronize(stream);
   }
-  for (int p = lo; p <= hi; ++p) {
-    if (gexec[p]) (void)hipGraphExecDestroy(gexec[p]);
-    if (oneExec[p]) (void)hipGraphExecDestroy(oneExec[p]);
-    gexec[p] = oneExec[p] = nullptr;
-    gMaxN[p] = oneMaxN[p] = 0;
-  }
+  for (int f = 0; f < kForms; ++f)
+    for (int p = lo; p <= hi; ++p) {
+      if (gexec[f][p]) (void)hipGraphExecDestroy(gexec[f][p]);
+      if (oneExec[f][p]) (void)hipGraphExecDestroy(oneExec[f][p]);
+      gexec[f][p] = oneExec[f][p] = nullptr;
+      gMaxN[f][p] = oneMaxN[f][p] = 0;
+    }
 }
 
 Engine::HostSnapshot Engine::snapshot() const {
@@ -656,17 +661,18 @@ smd_status Engine::step_one() {
     oneSeen[p] = true;
     return enqueue_step(nullptr);
   }
-  if (oneExec[p] && Nub > oneMaxN[p]) refresh_bound(true);
-  if (oneExec[p] && Nub > oneMaxN[p]) drop_graph(p);
-  if (!oneExec[p]) {
+  const int f = graph_form(Nub);
+  if (oneExec[f][p] && Nub > oneMaxN[f][p]) refresh_bound(true);
+  if (oneExec[f][p] && Nub > oneMaxN[f][p]) drop_graph(p);
+  if (!oneExec[f][p]) {
     // headroom where the bound only follows stale counts
     const uint32_t maxN = (uint32_t)std::min<uint64_t>(Nub + Nub / 2, cap);
-    st = capture(1, maxN, &oneExec[p], &oneAfter[p]);
+    st = capture(1, maxN, &oneExec[f][p], &oneAfter[f][p]);
     if (st != SMD_OK) return st;
-    oneMaxN[p] = maxN;
+    oneMaxN[f][p] = maxN;
   }
-  HIPCHK(hipGraphLaunch(oneExec[p], stream));
-  restore(oneAfter[p]);
+  HIPCHK(hipGraphLaunch(oneExec[f][p], stream));
+  restore(oneAfter[f][p]);
   std::fill(slotPending.begin(), slotPending.end(), (uint8_t)0);
   ++stepsDone;
   Nub = std::min<uint64_t>(step_bound(Nub), (uint64_t)cap);
@@ -680,7 +686,11 @@ smd_status Engine::step_one() {
 // one graph is kept per parity.
 smd_status Engine::step_graph(int pairs) {
   for (int k = 0; k < pairs; ++k) {
-    refresh_bound(false);
+    // before a run of steps is queued, one look at how the first ones sorted
+    const bool look = k > 0 && !sortSeen && graph_form(Nub) != (int)SortForm::kDigits;
+    sortSeen = sortSeen || look;
+    refresh_bound(look);
+    watch_sort();
     uint64_t need = step_bound(step_bound(Nub));  // output of the second step
     if (need > cap) {
       refresh_bound(true);
@@ -692,24 +702,25 @@ smd_status Engine::step_graph(int pairs) {
     }
     uint64_t bound = step_bound(Nub);  // input bound of the second step
     const int p = cur;
-    if (gexec[p] && bound > gMaxN[p]) {
+    const int f = graph_form(bound);
+    if (gexec[f][p] && bound > gMaxN[f][p]) {
       // a stale count alone must not force a new capture: read the exact one
       refresh_bound(true);
       bound = step_bound(Nub);
     }
     uint64_t want = bound;
-    if (gexec[p] && bound > gMaxN[p]) {
+    if (gexec[f][p] && bound > gMaxN[f][p]) {
       // outgrown: grids with headroom, so that a growing system re-captures rarely
-      want = std::max<uint64_t>(bound, (uint64_t)gMaxN[p] + gMaxN[p] / 2);
+      want = std::max<uint64_t>(bound, (uint64_t)gMaxN[f][p] + gMaxN[f][p] / 2);
       drop_graph(p);
     }
-    if (!gexec[p]) {
+    if (!gexec[f][p]) {
       const uint32_t maxN = (uint32_t)std::min<uint64_t>(want, cap);
-      smd_status st = capture(2, maxN, &gexec[p], nullptr);
+      smd_status st = capture(2, maxN, &gexec[f][p], nullptr);
       if (st != SMD_OK) return st;
-      gMaxN[p] = maxN;
+      gMaxN[f][p] = maxN;
     }
-    HIPCHK(hipGraphLaunch(gexec[p], stream));
+    HIPCHK(hipGraphLaunch(gexec[f][p], stream));
     // two steps: every ping-pong selection is back where it was
     std::fill(slotPending.begin(), slotPending.end(), (uint8_t)0);
     stepsDone += 2;
@@ -796,8 +807,47 @@ smd_status Engine::plan_cell_sort() {
   return SMD_OK;
 }
 
+// Estimates, us, fitted to single systems of 20k to 48M particles (grids of 2^6
+// to 2^24 cells, uniform, in slabs and in blocks) and ensembles of 8 to 512:
+// the counting form with its overfull slices against the digit passes and the
+// cell table kernel, which reads 4096 cells' keys per workgroup.  Step, us,
+// counted / by digits (knob 0): 100k on 2^12 cells 185 / 118, 1M on 2^14 482 /
+// 274, 1M in 1/32 of the height 450 / 190, 48k so 129 / 75, 4M in a block of
+// 1/64 606 / 394, 8 systems of 100k in slabs 381 / 139; where no slice is
+// overfull, 100k 44 / 69, 1M 74 / 98.  The tenth keeps ties as they are.
+bool Engine::digits_faster(uint32_t most, uint32_t rounds) const {
+  const double m = (double)knownN / (1 << 20), spans = std::max(1.0, deadKey / 4096.0);
+  const bool bins = sort_form(1) == SortForm::kCellsByBin;
+  const double counted = (bins ? 20.0 + 22.0 * m : 15.0 + 11.0 * m) + 0.5 * most + rounds * (1.2 / 1024.0);
+  const double passes = seg_sorted() ? 2.0 : sort_passes(keyBits, radixBits);
+  const double digits = passes * (14.0 + 8.0 * m) + 8.0 + (double)knownN / spans / 2000.0;
+  return counted > 1.1 * digits;
+}
+
+void Engine::restart_sort_watch() {
+  digitsUntil = 0;
+  digitsHold = kDigitsHold;
+  sortFrom = stepsDone;
+  sortSeen = false;
+}
+
+void Engine::watch_sort() {
+  if (digitsUntil && stepsDone >= digitsUntil) {  // look again
+    digitsUntil = 0;
+    sortFrom = stepsDone;
+    sortSeen = false;
+  }
+  if (digitsUntil || !hostSort) return;
+  const unsigned long long v = __atomic_load_n(hostSort, __ATOMIC_ACQUIRE);
+  if (!v || (int32_t)((uint32_t)(v >> 32) - (uint32_t)sortFrom) <= 0) return;
+  if (!digits_faster((uint32_t)(v >> 16) & 0xFFFFu, ((uint32_t)v & 0xFFFFu) << 6)) return;
+  if (stepsDone - sortFrom > 4 * kDigitsHold) digitsHold = kDigitsHold;  // it went well for a while
+  digitsUntil = stepsDone + digitsHold;
+  digitsHold = std::min<uint64_t>(2 * digitsHold, 1024 * kDigitsHold);
+}
+
 Engine::SortForm Engine::sort_form(uint32_t maxN) const {
-  if (!segSort || sb.algo != 1 || radixBits != 8 || maxN == 0) return SortForm::kDigits;
+  if (digitsUntil || !segSort || sb.algo != 1 || radixBits != 8 || maxN == 0) return SortForm::kDigits;
   // a system that has grown well past what the slices were laid out for
   // takes the bins
   if (cellGroups && (knownN <= cellGroupsN || !cellBinBits)) return SortForm::kCellsByReplica;
@@ -849,6 +899,7 @@ hipError_t Engine::sort_keys(uint32_t maxN, bool tilesLaid, StageTimer* timer, b
   a.dst = sb.gatherDst;
   a.packIndex = sb.packIndex;
   a.status = sb.status;
+  a.work = dCounters + 5;
   uint32_t wg = cellGroups;
   const bool part = form == SortForm::kCellsByBin;
   if (part) {
@@ -997,8 +1048,8 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
   fa.tileDeadNext = dTileDead[cur ^ 1];
   fa.tileBirth = anySplit ? dTileBirth : nullptr;
   fa.tileBirthPre = dTileBirthPre;
-  fa.candCount = anyBim ? dCounters + 3 : nullptr;
-  fa.candActing = dCounters + 4;
+  fa.pairCounts = anyBim ? dCounters + 3 : nullptr;
+  fa.hostSort = dHostSort;
   fa.particleSteps = dParticleSteps;
   fa.stepCount = dStepCount;
   fa.countRing = dCountRing;
@@ -1327,6 +1378,7 @@ smd_status Engine::set_particles(const float* pos4, const int* types, uint32_t n
   Nub = n;
   knownN = n;
   lastSeen = stepsDone;  // counts published before this call are stale
+  restart_sort_watch();
   return SMD_OK;
 }
 

@@ -1538,15 +1538,17 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
     born = a.tileBirth && tile < t1 && part == 0u ? a.tileBirth[tile] : 0u;
   };
   load_counts();
-  uint32_t stepPrev = 0, status = 0, pairs = 0, acting = 0;
+  uint32_t stepPrev = 0, status = 0, pairs = 0, acting = 0, sortMost = 0, sortRounds = 0;
   unsigned long long psPrev = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     stepPrev = *a.stepCount;
     psPrev = *a.particleSteps;
     status = *a.status;
-    if (a.candCount) {
-      pairs = *a.candCount;
-      acting = *a.candActing;
+    if (a.pairCounts) {
+      pairs = a.pairCounts[0];
+      acting = a.pairCounts[1];
+      sortMost = a.pairCounts[2];
+      sortRounds = a.pairCounts[3];
     }
   }
   for (uint32_t q = t0 + threadIdx.x; q < t1; q += 1024u) a.tileDeadNext[q] = 0u;
@@ -1590,10 +1592,10 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
       for (int k = 0; k < 4; ++k) c[k] += tot[k];
     }
     if (threadIdx.x == 0) {
-      if (a.candCount) {
+      if (a.pairCounts) {
         // a list again once half of it would do
-        *a.candCount = pairs > kPairList && acting > kPairList / 2u ? kPairList + 1u : 0u;
-        *a.candActing = 0u;
+        a.pairCounts[0] = pairs > kPairList && acting > kPairList / 2u ? kPairList + 1u : 0u;
+        a.pairCounts[1] = 0u;
       }
       a.newOff[a.R] = c[0];
       *a.dNnext = c[0];
@@ -1603,6 +1605,16 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
       // tagged with the step number (no copy or event in the stream)
       const uint32_t st = stepPrev + 1u;
       *a.stepCount = st;
+      if (sortMost) {
+        a.pairCounts[2] = a.pairCounts[3] = 0u;
+        // removed particles' keys all fall to one workgroup of the digit
+        // form's cell table kernel, 2000 of them in a microsecond
+        const uint32_t most = sortMost - min(sortMost, c[1] / 1000u);
+        if (most)
+          __hip_atomic_store(a.hostSort,
+                             ((unsigned long long)st << 32) | min(most, 0xFFFFu) << 16 | min(sortRounds >> 6, 0xFFFFu),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
       __hip_atomic_store(&a.countRing[st & a.ringMask], ((unsigned long long)st << 32) | c[0], __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_SYSTEM);
     }

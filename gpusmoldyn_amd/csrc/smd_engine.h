@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -106,6 +107,7 @@ class Engine {
   std::vector<uint32_t> lastN;      // per replica: a recent count (which way get() takes)
   std::mutex readMutex;             // several threads may read: one at a time uses this memory
   uint32_t* dHostStatus = nullptr;  // its device address
+  unsigned long long *hostSort = nullptr, *dHostSort = nullptr;
   // order-0 creation: one stream per replica, a per-step creation buffer
   uint32_t *dZMt = nullptr, *dZPar = nullptr, *dZCount = nullptr, *dZeroBase = nullptr;
   float4* dZPos = nullptr;
@@ -152,13 +154,15 @@ class Engine {
   // hipGraph replay of two-step pairs and of single steps, one executable
   // graph per ping-pong parity (a single step flips the parity)
   bool useGraphs = true;
-  hipGraphExec_t gexec[2] = {nullptr, nullptr};
-  uint32_t gMaxN[2] = {0, 0};
-  hipGraphExec_t oneExec[2] = {nullptr, nullptr};
-  uint32_t oneMaxN[2] = {0, 0};
+  // and per form of the sort
+  static constexpr int kForms = 3;
+  hipGraphExec_t gexec[kForms][2] = {};
+  uint32_t gMaxN[kForms][2] = {};
+  hipGraphExec_t oneExec[kForms][2] = {};
+  uint32_t oneMaxN[kForms][2] = {};
   bool oneSeen[2] = {false, false};  // a single step of this parity has been launched
   // Waits for the stream, then destroys the executable graph of parity
-  // `which` (-1: both).
+  // `which` (-1: both), of every form.
   void drop_graph(int which = -1);
 
   // one replica's count is the total that the finalize kernel published
@@ -176,6 +180,21 @@ class Engine {
   enum class SortForm { kDigits, kCellsByReplica, kCellsByBin };
   SortForm sort_form(uint32_t maxN) const;
   smd_status plan_cell_sort();
+  // Counting keys per cell depends on how the particles lie: a slice that
+  // holds too many for its list works through them window by window.  Steps
+  // report such slices to the host (hostSort), which takes the digit passes
+  // for digitsHold steps where they are the faster form, then looks again.
+  void watch_sort();
+  bool digits_faster(uint32_t most, uint32_t rounds) const;
+  int graph_form(uint64_t n) const {
+    return anyBim ? (int)sort_form((uint32_t)std::min<uint64_t>(n, 0xFFFFFFFFu)) : 0;
+  }
+  void restart_sort_watch();
+  static constexpr uint64_t kDigitsHold = 1024;
+  uint64_t digitsUntil = 0;           // steps done until which the digit passes run (0: they need not)
+  uint64_t digitsHold = kDigitsHold;  // doubled each time
+  uint64_t sortFrom = 0;              // reports of steps up to here are settled
+  bool sortSeen = false;              // a report could have been read since
   // sorted keys, records and cell table of the step (debug: also the values
   // and the removed particles)
   hipError_t sort_keys(uint32_t maxN, bool tilesLaid, StageTimer* timer, bool debug);
@@ -209,7 +228,7 @@ class Engine {
   };
   HostSnapshot snapshot() const;
   void restore(const HostSnapshot& s);
-  HostSnapshot oneAfter[2] = {};  // the selection after a single-step graph
+  HostSnapshot oneAfter[kForms][2] = {};  // the selection after a single-step graph
   smd_status capture(int steps, uint32_t maxN, hipGraphExec_t* exec, HostSnapshot* after);
   smd_status step_one();
 };

@@ -154,6 +154,9 @@ struct CellSortArgs {
   float4* dst;                 // records in sorted order
   int packIndex;
   uint32_t* status;
+  // what the slices cost that did not fit their lists (SortWork): the most
+  // expensive one, in half microseconds, and the rounds of all
+  uint32_t* work;
 };
 
 // Pair candidates of a step: cand[j] = (partner, step tag) for the sorted
@@ -221,8 +224,9 @@ struct FinalizeArgs {
   uint32_t* tileDeadNext;  // the other step parity's counts: cleared here
   uint32_t* tileBirth;     // nullptr: no particle can be born
   uint32_t* tileBirthPre;
-  uint32_t* candCount;   // CandList::count and acting (nullptr: no pairs)
-  uint32_t* candActing;
+  // CandList::count and acting, then CellSortArgs::work (nullptr: no pairs)
+  uint32_t* pairCounts;
+  unsigned long long* hostSort;  // host-visible: step << 32 | most << 16 | rounds / 64 of the last step with such slices
   unsigned long long* particleSteps;  // += particles entering the step
   uint32_t* stepCount;                // steps completed (incremented here)
   unsigned long long* countRing;      // host-visible: slot (steps & ringMask) = steps << 32 | particles
