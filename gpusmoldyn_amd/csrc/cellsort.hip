@@ -66,6 +66,7 @@ struct CsLds {
 static_assert(sizeof(CsLds) <= 40 * 1024, "four workgroups per CU");
 static_assert(kRound <= kCellList && kRound < 65536u, "a round fits the list, its ranks fit 16 bits");
 static_assert(4u * kRounds * kVecRound <= kIndexMask + 1u, "the remembered rounds' indices fit an entry");
+static_assert(kCellKeys + 4u == 4u * kRounds * kVecRound, "one vector more when the first is cut");
 
 // Exclusive prefix of one value per thread over the workgroup; total gets the
 // sum.  The caller's next use of wsum must be behind another barrier.

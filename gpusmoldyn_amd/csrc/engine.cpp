@@ -750,12 +750,17 @@ SegSortArgs Engine::seg_args() const {
 // Form and workgroups of the counting cell sort.  By replica, every slice of
 // a replica's cells reads all of the replica's keys; by bins, a digit pass
 // over the keys' high bits comes first and every slice of a bin reads the
-// bin's.  Measured (us per sort, by replica against by bins): 512 replicas of
-// 2k to 64k 130 / 270, 48 of 4k to 131k 32 / 70, one of 16k 8 / 17, one of
-// 100k 35 / 20; so bins take single systems from 48k particles and ensembles
-// with a replica above 131k.  Slot engines keep the digit sort (16 jobs of 1k
-// to 262k: 121 / 71, digits 65): most of their bins are empty, and an empty
-// workgroup still costs its start (4 us per 1000).
+// bin's.  Measured, us per sort, by replica / by bins / by digits (replica by
+// replica where that applies): 512 replicas of 2k to 64k 115 / 255 / 211, with
+// one of 140k beside them 119 / 250 / 225, 16 of 140k 50 / 66 / 81, 16 of 262k
+// 108 / 115 / 145, but 9 of 262k 97 / 67 / 145, 2 of 140k 39 / 31 / 64, one
+// system of 16k 8 / 17, one of 100k 35 / 20.  So bins take single systems from
+// 48k particles, replicas above 262k (whose slices would read too many keys)
+// and those above 131k unless they are a sixteenth of the whole.  Ensembles
+// whose cells outnumber their particles so that most slices are empty keep the
+// digits (an empty workgroup costs its start, 4 to 6 us per 1000): 512 replicas
+// of 2k on 2^17 cells 154 by replica, 107 by digits; 300, 98 / 83; 256, 84 / 75;
+// of 20k 267 / 305.  So do slot engines (16 jobs of 1k to 262k: 121 / 71 / 65).
 smd_status Engine::plan_cell_sort() {
   uint64_t most = 1, total = 0;
   for (uint32_t r = 0; r < R; ++r) {
@@ -767,7 +772,7 @@ smd_status Engine::plan_cell_sort() {
   // bins of up to 16 slices: more would read their keys over too often
   cellBinBits = std::max<uint32_t>(11, bits > 8 ? bits - 8 : 0);
   if (cellBinBits > kCellSliceBits + 4 || slotsMode) cellBinBits = 0;
-  if (slotsMode || most > 131072 || (R == 1 && most > 49152)) return SMD_OK;
+  if (slotsMode || most > kCellKeys || (most > 131072 && total < 16 * most) || (R == 1 && most > 49152)) return SMD_OK;
   std::vector<uint32_t> slices(R), order(R);
   // a few systems get more slices than their lists need, to spread over the
   // CUs, up to 2M keys read
@@ -793,7 +798,9 @@ smd_status Engine::plan_cell_sort() {
       if (lists[q].size() < lists[x].size()) x = q;
     for (uint32_t k = 0; k < slices[r]; ++k) lists[R < 8 ? (x + k) % 8 : x].push_back(r << kCellGroupShift | k);
   }
-  size_t longest = 0;
+  size_t longest = 0, all = 0;
+  for (uint32_t r = 0; r < R; ++r) all += slices[r];
+  if (all > 8192 + total / 1024) return SMD_OK;
   for (const auto& l : lists) longest = std::max(longest, l.size());
   std::vector<uint32_t> tab(8 * longest, kCellNoGroup);
   for (int x = 0; x < 8; ++x)
@@ -850,7 +857,11 @@ Engine::SortForm Engine::sort_form(uint32_t maxN) const {
   if (digitsUntil || !segSort || sb.algo != 1 || radixBits != 8 || maxN == 0) return SortForm::kDigits;
   // a system that has grown well past what the slices were laid out for
   // takes the bins
-  if (cellGroups && (knownN <= cellGroupsN || !cellBinBits)) return SortForm::kCellsByReplica;
+  // (an ensemble whose bins would hold more than 8 slices stays by replica: 512
+  // grown to 14.8M particles 676 us a step, by bins 884; 256 grown to 7.7M 390 /
+  // 491)
+  const bool bins = cellBinBits && !(R > 1 && cellBinBits > 15);
+  if (cellGroups && (knownN <= cellGroupsN || !bins)) return SortForm::kCellsByReplica;
   return cellBinBits ? SortForm::kCellsByBin : SortForm::kDigits;
 }
 

@@ -123,6 +123,9 @@ constexpr int kCellSliceBits = 12;
 constexpr uint32_t kCellSlice = 1u << kCellSliceBits;
 constexpr uint32_t kCellList = 5376;
 constexpr uint32_t kCellFill = 4838;
+// Keys of a segment, at any alignment, whose rounds a slice remembers; a larger
+// one takes the ordered path.
+constexpr uint32_t kCellKeys = (1u << 18) - 4u;
 constexpr int kCellGroupShift = 12;  // workgroup table: replica << kCellGroupShift | slice
 constexpr uint32_t kCellNoGroup = 0xFFFFFFFFu;  // an entry without work
 

@@ -102,3 +102,78 @@ def test_counts_again_when_particles_have_spread(smd, gpu, single):
         e.close()
     assert np.array_equal(res[0][1], res[1][1])
     assert np.array_equal(res[0][0].view(np.uint32), res[1][0].view(np.uint32))
+
+
+# ensembles: (particles, grid bits) of each replica, and the form
+ENSEMBLES = {
+    # most slices empty
+    "sparse_512": ([(2048, 17)] * 512, "segments"),
+    "sparse_256": ([(2048, 18)] * 256, "digits"),
+    "half_sparse_200": ([(2048, 17)] * 200, "replicas"),
+    # a replica above 131072 particles beside many, and with few
+    "one_large_of_many": ([(20000, 14)] * 120 + [(140000, 17)], "replicas"),
+    "large_16": ([(262140, 17)] * 16, "replicas"),
+    "large_9": ([(200001, 17)] * 9, "bins"),
+    "too_large": ([(262141, 17)] * 17, "bins"),
+}
+
+
+@pytest.mark.parametrize("name", list(ENSEMBLES))
+def test_form_of_ensembles(smd, gpu, name):
+    shapes, form = ENSEMBLES[name]
+    made = {s: _system(smd, *s) for s in dict.fromkeys(shapes)}
+    took, got = [], []
+    for radix, knob in ((0, 1), (11, 1), (0, 0)):
+        e = smd.Engine(0, radix)
+        for s in shapes:
+            e.add_replica(*made[s])
+        e.finalize()
+        e.set_knob(smd.KNOB_SEGMENTED_SORT, knob)
+        e.step(6)
+        e.sync()
+        if (radix, knob) == (0, 1):
+            assert e.sort_form() == form
+        best = 1e9
+        for _ in range(3):
+            t = time.perf_counter()
+            e.step(10)
+            e.sync()
+            best = min(best, (time.perf_counter() - t) / 10)
+        took.append(best * 1e6)
+        got.append([e.get(r) for r in (0, len(shapes) // 2, len(shapes) - 1)])
+        e.close()
+    print(f"{name}: {took[0]:.1f} us/step ({form}), 11-bit digits {took[1]:.1f}, digits {took[2]:.1f}", flush=True)
+    for other in got[1:]:
+        for (p1, t1), (p0, t0) in zip(got[0], other):
+            assert np.array_equal(t1, t0) and np.array_equal(p1.view(np.uint32), p0.view(np.uint32))
+    assert took[0] < 1.15 * min(took[1:])
+
+
+def test_grown_ensemble_keeps_its_form(smd, gpu):
+    """An ensemble that grows to several times its first size, bins of more
+    than 8 slices: by replica throughout, as by digits bit for bit."""
+    res = []
+    for knob in (1, 0):
+        e = smd.Engine(0)
+        for r in range(64):
+            spec, pos, types = _system(smd, 2000 + 97 * r, 18)
+            spec.num_reactions = 2
+            spec.rxn[1].order = 1
+            spec.rxn[1].reactants[0], spec.rxn[1].reactants[1] = 3, -1
+            spec.rxn[1].products[0], spec.rxn[1].products[1] = 3, 3
+            spec.rxn[1].nprod = 2
+            spec.rxn[1].rate = 100.0
+            e.add_replica(spec, pos, types)
+        e.finalize()
+        e.set_knob(smd.KNOB_SEGMENTED_SORT, knob)
+        n0 = int(e.counts().sum())
+        e.step(20)
+        n = int(e.counts().sum())
+        print(f"64 replicas grown from {n0} to {n}, knob {knob}: {e.sort_form()}", flush=True)
+        assert n > 4 * n0
+        if knob:
+            assert e.sort_form() == "replicas"
+        res.append([e.get(r) for r in (0, 31, 63)])
+        e.close()
+    for (p1, t1), (p0, t0) in zip(*res):
+        assert np.array_equal(t1, t0) and np.array_equal(p1.view(np.uint32), p0.view(np.uint32))
