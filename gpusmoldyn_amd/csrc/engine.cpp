@@ -175,40 +175,47 @@ int Engine::add_replica(const smd_sim_spec& spec, const float* pos4, const int* 
 
 smd_status Engine::alloc_particle_buffers(uint32_t c) {
   cap = c;
-  extraCap = (anySplit || anyZero || slotsMode) ? cap : 0;
+  // A step only starts where its outcome fits the capacity if every particle
+  // splits and all that can be created or admitted is (step_bound): half the
+  // capacity enters at most, and as much is gained.
+  const bool gains = anySplit || slotsMode;
+  stepCap = gains ? cap / 2 + 1 : cap;
+  extraCap = (gains ? cap / 2 + 1 : 0) + zeroTotal;
   for (int k = 0; k < 2; ++k) HIPCHK(dalloc(&dPT[k], (size_t)cap + extraCap));
   if (wApart) {
     smd_status st = alloc_apart();
     if (st != SMD_OK) return st;
   }
-  HIPCHK(dalloc(&dAddedPos, cap));
-  HIPCHK(dalloc(&dBirthType, cap));
-  HIPCHK(dalloc(&dSortedPT, cap));
-  HIPCHK(dalloc(&dCand, cap));
-  HIPCHK(hipMemsetAsync(dCand, 0, (size_t)cap * sizeof(uint2), stream));  // tag 0: no step's
+  if (gains) {
+    HIPCHK(dalloc(&dAddedPos, stepCap));
+    HIPCHK(dalloc(&dBirthType, stepCap));
+    HIPCHK(hipMemsetAsync(dBirthType, 0, (size_t)stepCap * sizeof(int), stream));
+  }
+  HIPCHK(dalloc(&dSortedPT, stepCap));
+  HIPCHK(dalloc(&dCand, stepCap));
+  HIPCHK(hipMemsetAsync(dCand, 0, (size_t)stepCap * sizeof(uint2), stream));  // tag 0: no step's
   HIPCHK(dalloc(&dCandList, pair_list_size()));
   // the cell sort reads keys as whole vectors of four
-  HIPCHK(dalloc(&sb.keys, (size_t)cap + 4));
-  HIPCHK(dalloc(&sb.vals, cap));
-  HIPCHK(dalloc(&sb.keysAlt, (size_t)cap + 4));
-  HIPCHK(dalloc(&sb.valsAlt, cap));
-  HIPCHK(dalloc(&sb.counts, sort_counts_words(cap, radixBits)));
-  nTilesCap = cap / kCompactTile + 2;
+  HIPCHK(dalloc(&sb.keys, (size_t)stepCap + 4));
+  HIPCHK(dalloc(&sb.vals, stepCap));
+  HIPCHK(dalloc(&sb.keysAlt, (size_t)stepCap + 4));
+  HIPCHK(dalloc(&sb.valsAlt, stepCap));
+  HIPCHK(dalloc(&sb.counts, sort_counts_words(stepCap, radixBits)));
+  nTilesCap = stepCap / kCompactTile + 2;
   const size_t words = (size_t)nTilesCap * (kCompactTile / 32);
   HIPCHK(dalloc(&dDeadBits, words));
-  HIPCHK(dalloc(&dHoles, cap));
+  HIPCHK(dalloc(&dHoles, stepCap));
   HIPCHK(dalloc(&dTileBirth, nTilesCap));
   HIPCHK(dalloc(&dTileBirthPre, nTilesCap));
   finBlockTiles = finalize_block_tiles(nTilesCap);
   HIPCHK(dalloc(&dBlockSum, (size_t)nTilesCap / finBlockTiles + 1));
-  if (segHigh) HIPCHK(dalloc(&dSegScratch, seg_sort_words(cap, (int)R, std::max(segLow, segHigh))));
+  if (segHigh) HIPCHK(dalloc(&dSegScratch, seg_sort_words(stepCap, (int)R, std::max(segLow, segHigh))));
   HIPCHK(hipMemsetAsync(dDeadBits, 0, words * sizeof(uint32_t), stream));
   for (int k = 0; k < 2; ++k) {
     HIPCHK(dalloc(&dTileDead[k], nTilesCap));
     HIPCHK(hipMemsetAsync(dTileDead[k], 0, nTilesCap * sizeof(uint32_t), stream));
   }
   HIPCHK(hipMemsetAsync(dTileBirth, 0, nTilesCap * sizeof(uint32_t), stream));
-  HIPCHK(hipMemsetAsync(dBirthType, 0, (size_t)cap * sizeof(int), stream));
   return SMD_OK;
 }
 
@@ -578,7 +585,7 @@ smd_status Engine::ensure_capacity() {
 }
 
 smd_status Engine::enqueue_step(StageTimer* timer) {
-  const uint32_t maxN = (uint32_t)std::min<uint64_t>(Nub, cap);
+  const uint32_t maxN = (uint32_t)std::min<uint64_t>(Nub, stepCap);
   smd_status st = enqueue_kernels(maxN, timer);
   if (st != SMD_OK) return st;
   ++stepsDone;
@@ -666,7 +673,7 @@ smd_status Engine::step_one() {
   if (oneExec[f][p] && Nub > oneMaxN[f][p]) drop_graph(p);
   if (!oneExec[f][p]) {
     // headroom where the bound only follows stale counts
-    const uint32_t maxN = (uint32_t)std::min<uint64_t>(Nub + Nub / 2, cap);
+    const uint32_t maxN = (uint32_t)std::min<uint64_t>(Nub + Nub / 2, stepCap);
     st = capture(1, maxN, &oneExec[f][p], &oneAfter[f][p]);
     if (st != SMD_OK) return st;
     oneMaxN[f][p] = maxN;
@@ -715,7 +722,7 @@ smd_status Engine::step_graph(int pairs) {
       drop_graph(p);
     }
     if (!gexec[f][p]) {
-      const uint32_t maxN = (uint32_t)std::min<uint64_t>(want, cap);
+      const uint32_t maxN = (uint32_t)std::min<uint64_t>(want, stepCap);
       smd_status st = capture(2, maxN, &gexec[f][p], nullptr);
       if (st != SMD_OK) return st;
       gMaxN[f][p] = maxN;
@@ -1545,6 +1552,7 @@ smd_status Engine::debug_stage(int stage, float* pos4, int* types, uint32_t* key
   }
   HIPCHK(hipSetDevice(device));
   smd_status st = sync();
+  if (st == SMD_OK) st = ensure_capacity();
   if (st != SMD_OK) return st;
   uint32_t n = 0;
   HIPCHK(hipMemcpy(&n, dN, sizeof(uint32_t), hipMemcpyDeviceToHost));

@@ -80,6 +80,7 @@ class Engine {
   float* dW[2] = {nullptr, nullptr};
   bool wApart = false;
   uint32_t extraCap = 0;
+  uint32_t stepCap = 0;  // particles that a step can start with
   float4* dAddedPos = nullptr;
   int* dBirthType = nullptr;
   float4* dSortedPT = nullptr;

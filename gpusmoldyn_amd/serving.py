@@ -23,10 +23,11 @@ import numpy as np
 from . import BC_REFLECT, Engine, SmdError
 from .configs import SEED, grid_bits_for, make_spec, streams_for
 
-# Device bytes held per particle of capacity: positions and types double
-# buffered, birth staging, sorted copy, candidates, keys and values double
-# buffered.
-BYTES_PER_PARTICLE = 2 * 16 + 2 * 4 + 16 + 4 + 16 + 4 + 4 * 4
+# Device bytes held per particle of capacity: records double buffered, with
+# room behind them for half as many gained; for the half of the capacity that
+# can enter a step, birth staging, sorted copy, candidates, keys and values
+# double buffered and the list of holes.
+BYTES_PER_PARTICLE = 3 * 16 + (16 + 4 + 16 + 8 + 4 * 4 + 4) // 2
 
 
 @dataclass
