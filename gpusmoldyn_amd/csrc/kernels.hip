@@ -567,17 +567,14 @@ __global__ __launch_bounds__(256) void k_sort_down(const uint32_t* __restrict__ 
   // consecutive digits from t * DPT (one block scan whatever the radix).
   if constexpr (TILED) {
     static_assert(RADIX == 256, "one digit per thread");
-    constexpr uint32_t kAtOnce = kTiledSums;
-    uint32_t all = 0, lower = 0;
-    for (uint32_t q0 = 0; q0 < nTiles; q0 += kAtOnce) {
-      uint32_t c[kAtOnce];
+    // nTiles <= kTiledSums (launch_sort_bins): the counts of all tiles at once
+    uint32_t c[kTiledSums], all = 0, lower = 0;
 #pragma unroll
-      for (uint32_t q = 0; q < kAtOnce; ++q) c[q] = q0 + q < nTiles && n ? counts[(size_t)(q0 + q) * RADIX + t] : 0u;
+    for (uint32_t q = 0; q < kTiledSums; ++q) c[q] = q < nTiles && n ? counts[(size_t)q * RADIX + t] : 0u;
 #pragma unroll
-      for (uint32_t q = 0; q < kAtOnce; ++q) {
-        all += c[q];
-        lower += q0 + q < tile ? c[q] : 0u;
-      }
+    for (uint32_t q = 0; q < kTiledSums; ++q) {
+      all += c[q];
+      lower += q < tile ? c[q] : 0u;
     }
     if (tile == 0u) totals[t] = all;
     s_base[t] = block_exscan256(all, wsum, &tot) + lower;
