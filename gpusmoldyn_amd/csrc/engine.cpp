@@ -693,8 +693,9 @@ smd_status Engine::step_one() {
 // one graph is kept per parity.
 smd_status Engine::step_graph(int pairs) {
   for (int k = 0; k < pairs; ++k) {
-    // before a run of steps is queued, one look at how the first ones sorted
-    const bool look = k > 0 && !sortSeen && graph_form(Nub) != (int)SortForm::kDigits;
+    // before a long run of steps is queued, one look at how the first ones
+    // sorted (a wait of some 20 us; short runs are looked at by the next call)
+    const bool look = k > 0 && !sortSeen && pairs - k >= 16 && graph_form(Nub) != (int)SortForm::kDigits;
     sortSeen = sortSeen || look;
     refresh_bound(look);
     watch_sort();
