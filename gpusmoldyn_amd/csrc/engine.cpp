@@ -918,7 +918,7 @@ hipError_t Engine::sort_keys(uint32_t maxN, bool tilesLaid, StageTimer* timer, b
   a.dst = sb.gatherDst;
   a.packIndex = sb.packIndex;
   a.status = sb.status;
-  a.work = dCounters + 5;
+  a.work = dCounters + 6;
   uint32_t wg = cellGroups;
   const bool part = form == SortForm::kCellsByBin;
   if (part) {
@@ -981,7 +981,7 @@ CandArgs Engine::cand_args() const {
   a.sortedPT = dSortedPT;
   a.first = dFirst;
   a.dLive = dLive;
-  a.cand = CandList{dCand, dCandList, dCounters + 3, dCounters + 4, dStepCount};
+  a.cand = CandList{dCand, dCandList, dCounters + 4, dCounters + 5, dStepCount};
   return a;
 }
 
@@ -993,7 +993,7 @@ ResolveArgs Engine::resolve_args() const {
   a.mtPar = dMtPar;
   a.Stot = Stot;
   a.first = dFirst;
-  a.cand = CandList{dCand, dCandList, dCounters + 3, dCounters + 4, dStepCount};
+  a.cand = CandList{dCand, dCandList, dCounters + 4, dCounters + 5, dStepCount};
   a.sortedPT = dSortedPT;
   a.vals = sb.vals;
   a.packed = sb.packIndex;
@@ -1067,7 +1067,7 @@ smd_status Engine::enqueue_kernels(uint32_t maxN, StageTimer* timer) {
   fa.tileDeadNext = dTileDead[cur ^ 1];
   fa.tileBirth = anySplit ? dTileBirth : nullptr;
   fa.tileBirthPre = dTileBirthPre;
-  fa.pairCounts = anyBim ? dCounters + 3 : nullptr;
+  fa.pairCounts = anyBim ? (uint4*)(dCounters + 4) : nullptr;  // 16-byte aligned
   fa.hostSort = dHostSort;
   fa.particleSteps = dParticleSteps;
   fa.stepCount = dStepCount;

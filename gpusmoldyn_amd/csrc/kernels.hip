@@ -1535,18 +1535,14 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
     born = a.tileBirth && tile < t1 && part == 0u ? a.tileBirth[tile] : 0u;
   };
   load_counts();
-  uint32_t stepPrev = 0, status = 0, pairs = 0, acting = 0, sortMost = 0, sortRounds = 0;
+  uint32_t stepPrev = 0, status = 0;
+  uint4 pc = make_uint4(0u, 0u, 0u, 0u);  // pairs, acting, sort's most and rounds
   unsigned long long psPrev = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     stepPrev = *a.stepCount;
     psPrev = *a.particleSteps;
     status = *a.status;
-    if (a.pairCounts) {
-      pairs = a.pairCounts[0];
-      acting = a.pairCounts[1];
-      sortMost = a.pairCounts[2];
-      sortRounds = a.pairCounts[3];
-    }
+    if (a.pairCounts) pc = *a.pairCounts;
   }
   for (uint32_t q = t0 + threadIdx.x; q < t1; q += 1024u) a.tileDeadNext[q] = 0u;
   if (blockIdx.x > 0 && t0 >= (n + kCompactTile - 1u) / kCompactTile) return;  // no particles here
@@ -1591,8 +1587,7 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
     if (threadIdx.x == 0) {
       if (a.pairCounts) {
         // a list again once half of it would do
-        a.pairCounts[0] = pairs > kPairList && acting > kPairList / 2u ? kPairList + 1u : 0u;
-        a.pairCounts[1] = 0u;
+        *a.pairCounts = make_uint4(pc.x > kPairList && pc.y > kPairList / 2u ? kPairList + 1u : 0u, 0u, 0u, 0u);
       }
       a.newOff[a.R] = c[0];
       *a.dNnext = c[0];
@@ -1602,14 +1597,13 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
       // tagged with the step number (no copy or event in the stream)
       const uint32_t st = stepPrev + 1u;
       *a.stepCount = st;
-      if (sortMost) {
-        a.pairCounts[2] = a.pairCounts[3] = 0u;
+      if (pc.z) {
         // removed particles' keys all fall to one workgroup of the digit
         // form's cell table kernel, 2000 of them in a microsecond
-        const uint32_t most = sortMost - min(sortMost, c[1] / 1000u);
+        const uint32_t most = pc.z - min(pc.z, c[1] / 1000u);
         if (most)
           __hip_atomic_store(a.hostSort,
-                             ((unsigned long long)st << 32) | min(most, 0xFFFFu) << 16 | min(sortRounds >> 6, 0xFFFFu),
+                             ((unsigned long long)st << 32) | min(most, 0xFFFFu) << 16 | min(pc.w >> 6, 0xFFFFu),
                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       }
       __hip_atomic_store(&a.countRing[st & a.ringMask], ((unsigned long long)st << 32) | c[0], __ATOMIC_RELAXED,

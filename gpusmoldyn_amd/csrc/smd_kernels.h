@@ -228,7 +228,7 @@ struct FinalizeArgs {
   uint32_t* tileBirth;     // nullptr: no particle can be born
   uint32_t* tileBirthPre;
   // CandList::count and acting, then CellSortArgs::work (nullptr: no pairs)
-  uint32_t* pairCounts;
+  uint4* pairCounts;
   unsigned long long* hostSort;  // host-visible: step << 32 | most << 16 | rounds / 64 of the last step with such slices
   unsigned long long* particleSteps;  // += particles entering the step
   uint32_t* stepCount;                // steps completed (incremented here)
