@@ -1613,7 +1613,10 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeArgs a) {
   uint32_t c[2] = {0u, 0u};  // deaths and births so far, of this workgroup
   bool placed = false;       // c[0] counts the earlier workgroups' deaths too
   for (uint32_t tb = t0; tb < t1; tb = MANY ? tb + kFinTiles : t1, tile += kFinTiles) {
-    if (MANY && tb != t0) load_counts();
+    if (MANY && tb != t0) {
+      if (tb >= (n + kCompactTile - 1u) / kCompactTile) break;
+      load_counts();
+    }
     if (!__syncthreads_or((dead | born) != 0u)) continue;
     uint2 x = make_uint2(0u, 0u);
     if (dead) {
