@@ -76,7 +76,8 @@ def stage_bytes(name, n, S, nb, passes, packed=True, form="digits"):
     if name == "first" and form in ("digits", "segments"):
         return 4 * (nb + 1) + 4 * n
     if name == "candidates":
-        return 24 * n
+        # key 4, record 16 and the cell table in; a candidate only where there is a partner
+        return 20 * n + 4 * (nb + 1)
     # pairs, bookkeeping and the particles gained: a few records
     return 0
 
