@@ -21,7 +21,10 @@
 // before / this kernel: one system of 16k particles (2^18 cells) 41 / 8,
 // 256 replicas of 2k 39 / 8, 512 replicas of 2k to 64k 225 / 125, 48 of 4k to
 // 131k 64 / 27; with the digit pass over the high bits in front, 100k 45 / 20,
-// 1M 58 / 37, 4M clustered 138 / 131.
+// 1M 58 / 37, 4M clustered 138 / 131.  A slice with more particles than its
+// list holds, or a cell of more than a few, takes the ordered path, 5 to 10 us
+// for each of its windows; what that came to is reported to the host
+// (CellSortArgs::work), which turns to the digit passes where they are faster.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

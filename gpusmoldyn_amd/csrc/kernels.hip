@@ -4,7 +4,7 @@
 //   k_producer    diffuse + unimolecular reactions + boundaries + hash   (one thread per RNG stream)
 //   k_cell_sort   (cellsort.hip) records sorted by bucket and the lower bound of every bucket;
 //                 for one large system behind one k_sort_* pass over the keys' high bits
-//   k_sort_*      for slot engines and other digit widths: stable LSD radix sort of (bucket key,
+//   k_sort_*      for slot engines, other digit widths and where particles crowd: stable LSD radix sort of (bucket key,
 //                 particle index); the last digit pass also copies each particle's record into
 //                 sorted order, and k_first finds the lower bound of every bucket
 //   k_candidates  neighbour-cell search for each particle's nearest reactive partner

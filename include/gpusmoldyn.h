@@ -189,9 +189,9 @@ typedef enum smd_knob {
   SMD_KNOB_PRODUCER_BLOCK = 0,
   SMD_KNOB_PAIR_BLOCK = 1,
   /* 1 (default): keys are sorted by counting them per cell where that applies
-   * (8-bit digits, not in slot engines), otherwise an engine of several
-   * replicas sorts each replica's keys on its local cells (two digit passes
-   * where the global keys need three); 0: one digit sort over all keys */
+   * (8-bit digits, not in slot engines) and is faster, otherwise an engine of
+   * several replicas sorts each replica's keys on its local cells (two digit
+   * passes where the global keys need three); 0: one digit sort over all keys */
   SMD_KNOB_SEGMENTED_SORT = 2
 } smd_knob;
 smd_status smd_engine_set_knob(smd_engine* e, int knob, int value);
